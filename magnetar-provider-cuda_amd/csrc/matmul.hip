@@ -5,35 +5,20 @@
 // [n, k]), f32 accumulation, the addend added to the finished sum.
 //
 // Two kernel families, chosen by shape:
-//  - MFMA tiles. A workgroup owns a BM x BN tile of C and walks k in BK
-//    slices, double-buffered in LDS. Each slice keeps its operand's global
-//    orientation, unpadded: rows along k (B stored [k, n], A stored [k, m])
-//    as they are, rows along m or n (A stored [m, k], B stored [n, k]) with
-//    their 16-byte chunks XOR-swizzled. Interior slices of f32 operands go
-//    straight from global memory to LDS (buffer_load_dwordx4 with the lds bit: no
-//    registers, no LDS write instructions) while the MFMAs run on the other
-//    buffer; edge and partial slices, and compact bf16 B, go through
-//    registers (zero-filled, widened) and one 16-byte LDS write per chunk.
-//    Each wave owns WM x WN of the tile as (WM/32) x (WN/32)
-//    v_mfma_f32_32x32x2_f32 accumulators. A slice's k is summed in the order
-//    8g + 4h + e (group g, lane half h, step e), so a swizzled row gives a
-//    half's four k values of a group in one 16-byte read, and a k-major row
-//    is read as 32 consecutive words per half-wave; every fill path and
-//    transpose uses this order and gives the same bits. Four
-//    configurations, picked by a time model: 256 x 256 tiles of 8 waves
-//    (one per CU) for large products; 128 x 128 of 4 waves (two per CU) or
-//    of 8 waves (one per CU, in steps of two slices when every workgroup
-//    fits on the CUs at once); 64 x 64 of 8 waves in two k groups, in steps
-//    of four slices, for products of about one such tile per CU. With one
-//    slice per barrier every wave issues a part of the next slice's direct
-//    loads at each of its k groups; the stepped kernels spread the older
-//    waves' loads over the step (64 x 64) or issue them in one burst
-//    (128 x 128). Tiles are ordered so that
-//    consecutive tiles share a block row of A and each of the 8 XCDs (own
-//    L2) gets a contiguous band of tiles. When the tiles cannot fill the
-//    device, k is split: over up to 8 workgroups per tile (split-k), or in
-//    equal runs of (tile, k slice) units per workgroup (stream-K) when the
-//    tiles divide the device badly; partial tiles go to a workspace and a
+//  - MFMA tiles. A workgroup owns a BM x BN tile of C and sums it as bf16
+//    plane products (split_tile.hpp): each operand is read into registers
+//    two or three stages ahead of its use, split there into three bf16 planes
+//    and written to LDS once for all the waves that read it. Every operand
+//    orientation, alignment and weight format gives the same bits. Ragged
+//    edges repeat the last row or column, so edge tiles run the same loop.
+//    Four configurations, picked by a time model: 256 x 256 tiles of 8 waves
+//    (one per CU) for large products; 128 x 128 of 4 waves (two per CU) or of
+//    8 waves (one per CU); 64 x 64 of 8 waves in two k groups. Tiles are
+//    ordered so that consecutive tiles share a block row of A and each of the
+//    8 XCDs (own L2) gets a contiguous band of tiles. When the tiles cannot
+//    fill the device, k is split: over up to 8 workgroups per tile (split-k),
+//    or in equal runs of (tile, k slice) units per workgroup (stream-K) when
+//    the tiles divide the device badly; partial tiles go to a workspace and a
 //    second launch adds them in k order (deterministic) with the addend.
 //  - m <= kGemvMaxRows (decode), or up to 32 rows of a small product with
 //    k > 1024 in row blocks of 8: the work is reading B once (HBM-bound), so
@@ -54,6 +39,7 @@
 #include "internal.hpp"
 #include "decode_merge.hpp"
 #include "reduce.hpp"
+#include "split_tile.hpp"
 
 namespace {
 
@@ -102,184 +88,33 @@ mhip_status workspace(mhip_ctx* ctx, size_t bytes, float** out) {
 // MFMA tiles
 // ---------------------------------------------------------------------------
 
-// KG: the waves form KG groups that each cover the whole tile over every
-// KG-th part of each slice's k (summed in LDS at the end), so a small tile
-// still gives each SIMD two waves.
-template <int BM, int BN, int BK, int WM, int WN, bool A_T, bool B_T, int KG = 1, int STEP = 0>
-struct TileCfg {
-    static constexpr int kWavesN = BN / WN;
-    static constexpr int kTileWaves = (BM / WM) * kWavesN;
-    static constexpr int kWaves = kTileWaves * KG;
-    static constexpr int kThreads = 64 * kWaves;
-    static constexpr int kMI = WM / 32;
-    static constexpr int kNI = WN / 32;
-    // LDS slices keep the operand's global orientation, unpadded: A as
-    // [BK][BM] when stored [k, m] (A_T), else [BM][BK]; B as [BK][BN], or
-    // [BN][BK] when stored [n, k] (B_T). Rows along m or n (BK floats each)
-    // have their 16-byte chunks XOR-swizzled; rows along k are plain.
-    static constexpr int kLdsA = BM * BK;
-    static constexpr int kLdsB = BK * BN;
-    // Tiles of at most 64 x 64 give a wave only 8 MFMAs per slice, too few
-    // to cover a barrier and the first LDS reads of each slice: they move in
-    // steps of kGroup slices (one barrier per step), double-buffered, so
-    // kStages = 2 * kGroup slice buffers per operand. STEP > 0 sets kGroup
-    // (launch_mfma picks 2 for 8-wave 128 x 128 tiles in a single wave of
-    // workgroups).
-    static constexpr int kGroup = STEP > 0 ? STEP : (BM * BN <= 64 * 64 ? 4 : 1);
-    static constexpr int kStages = 2 * kGroup;
-    static constexpr int kLdsFloats = kStages * (kLdsA + kLdsB);
-    // Global slices as (rows x cols) with cols contiguous in memory.
-    static constexpr int kARows = A_T ? BK : BM, kACols = A_T ? BM : BK;
-    static constexpr int kBRows = B_T ? BN : BK, kBCols = B_T ? BK : BN;
-    static constexpr int kAChunks = kARows * kACols / 4 / kThreads;
-    static constexpr int kBChunks = kBRows * kBCols / 4 / kThreads;
-    static_assert(kARows * kACols % (4 * kThreads) == 0, "A slice must split evenly");
-    static_assert(kBRows * kBCols % (4 * kThreads) == 0, "B slice must split evenly");
-    static_assert(BK == 32, "swizzled rows hold 8 chunks");
-    static_assert(KG == 1 || KG == 2 || KG == 4, "k groups split a slice's 4 groups of 8");
-    static_assert(KG == 1 || kTileWaves * kMI * kNI * 16 * 64 <= kLdsFloats,
-                  "the k groups' sums are staged in the slice buffers");
-};
-
-typedef __attribute__((address_space(3))) void lds_void_t;
-typedef __attribute__((address_space(1))) void global_void_t;
-
-// XOR pattern of the 16-byte chunks of row r of an m- or n-major slice (8
-// chunks per row). Distinct over any 8 consecutive rows, and (r & 1, pattern)
-// distinct over 16, so 16-byte reads of one chunk position down 16 rows hit
-// distinct banks.
-__device__ __forceinline__ int chunk_swizzle(int r) { return (r & 7) ^ ((r >> 3) & 1); }
-
-// Float offset in an LDS slice of the 16-byte chunk whose global position is
-// (row r, column c) of a slice with COLS columns; SWZ for m- or n-major rows.
-template <int COLS, bool SWZ>
-__device__ __forceinline__ int chunk_offset(int r, int c) {
-    if constexpr (SWZ)
-        return r * COLS + (((c >> 2) ^ chunk_swizzle(r)) << 2);
-    else
-        return r * COLS + c;
-}
-
 using mhip::elem;
 using mhip::load4;
 using mhip::load4_nt;
 
-// Loads this thread's chunks of a (ROWS x COLS) slice whose columns are
-// contiguous in memory (leading dimension ld), rows from r0 and columns from
-// c0, zero-filling outside (rows_total, cols_total).
-template <int ROWS, int COLS, int CHUNKS, int THREADS, bool VEC, class T>
-__device__ __forceinline__ void load_slice(float4 (&regs)[CHUNKS], const T* __restrict__ g,
-                                           uint64_t ld, uint64_t r0, uint64_t c0,
-                                           uint64_t rows_total, uint64_t cols_total) {
-    constexpr int kChunksPerRow = COLS / 4;
-#pragma unroll
-    for (int i = 0; i < CHUNKS; ++i) {
-        const int chunk = threadIdx.x + i * THREADS;
-        const int r = chunk / kChunksPerRow;
-        const int c = (chunk % kChunksPerRow) * 4;
-        const uint64_t gr = r0 + r, gc = c0 + c;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (gr < rows_total) {
-            const T* p = g + gr * ld + gc;
-            if (VEC && gc + 3 < cols_total) {
-                v = load4(p);
-            } else {
-                if (gc + 0 < cols_total) v.x = elem(p + 0);
-                if (gc + 1 < cols_total) v.y = elem(p + 1);
-                if (gc + 2 < cols_total) v.z = elem(p + 2);
-                if (gc + 3 < cols_total) v.w = elem(p + 3);
-            }
-        }
-        regs[i] = v;
-    }
-}
+// One tile configuration (mhip::SplitTile's parameters but the operands').
+template <int BM_, int BN_, int WM_, int WN_, int KG_, int BK_, int BUFS_>
+struct TileShape {
+    static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, KG = KG_, BK = BK_, BUFS = BUFS_;
+    static constexpr int kWaves = (BM / WM) * (BN / WN) * KG;
+    // Workgroups per CU a configuration is planned for: one of 8 waves
+    // already gives each SIMD two.
+    static constexpr uint64_t kPerCu = kWaves >= 8 ? 1 : 2;
+    template <bool A_T, bool B_T, class BT>
+    using Tile = mhip::SplitTile<BM, BN, WM, WN, KG, BK, A_T, B_T, BT, BUFS>;
+};
 
-// The same slice when it lies wholly inside the matrix (rows r0 .. r0 + ROWS
-// and columns c0 .. c0 + COLS in range, 16-byte aligned rows): plain
-// dwordx4 loads with no bounds checks, issued back to back.
-template <int ROWS, int COLS, int CHUNKS, int THREADS, class T>
-__device__ __forceinline__ void load_slice_interior(float4 (&regs)[CHUNKS], const T* __restrict__ g,
-                                                    uint64_t ld, uint64_t r0, uint64_t c0) {
-    constexpr int kChunksPerRow = COLS / 4;
-#pragma unroll
-    for (int i = 0; i < CHUNKS; ++i) {
-        const int chunk = threadIdx.x + i * THREADS;
-        const int r = chunk / kChunksPerRow;
-        const int c = (chunk % kChunksPerRow) * 4;
-        regs[i] = load4(g + (r0 + r) * ld + c0 + c);
-    }
-}
-
-// Stores the chunks into an LDS slice (one 16-byte write each, at the
-// chunk's possibly swizzled position).
-template <int ROWS, int COLS, int CHUNKS, int THREADS, bool SWZ>
-__device__ __forceinline__ void store_slice(const float4 (&regs)[CHUNKS], float* lds) {
-    constexpr int kChunksPerRow = COLS / 4;
-#pragma unroll
-    for (int i = 0; i < CHUNKS; ++i) {
-        const int chunk = threadIdx.x + i * THREADS;
-        const int r = chunk / kChunksPerRow;
-        const int c = (chunk % kChunksPerRow) * 4;
-        *reinterpret_cast<float4*>(lds + chunk_offset<COLS, SWZ>(r, c)) = regs[i];
-    }
-}
-
-// The same slice copied straight from global memory into LDS (interior
-// slices of f32 operands, 16-byte aligned rows): one buffer_load_dwordx4 with
-// the lds bit fills 64 consecutive 16-byte slots, lane i slot i, so each lane
-// fetches the chunk that belongs in its slot. No registers, no LDS write
-// instructions; completion is tracked by vmcnt (wait before the barrier).
-// Buffer loads, not global_load_lds: the compiler counts a pending global
-// (FLAT) load into LDS as a possible LDS access, and then waits for every
-// LDS read at once (lgkmcnt(0)) before each MFMA group, so no operand read
-// could run ahead of the MFMAs (4096^3 985 -> 961-968 us, 2048^3 141 ->
-// 134 us). The buffer is the slice itself, from its first element, so the
-// lane offsets are 32-bit: launch_mfma takes this path only for leading
-// dimensions up to kDmaMaxLd.
-// Word 3 of a raw (unformatted, unswizzled) buffer descriptor on gfx950.
-constexpr int kRawBufferWord3 = 0x00020000;
-// Longest leading dimension (floats) whose 256-row slice stays under 2^31
-// bytes, the reach of a buffer's 32-bit lane offsets.
-constexpr uint64_t kDmaMaxLd = 1ull << 21;
-
-template <int ROWS, int COLS, int WAVES, bool SWZ>
-__device__ __forceinline__ void dma_slice(const float* __restrict__ g, uint64_t ld, uint64_t r0,
-                                          uint64_t c0, float* lds, int wave, int lane, int part = 0,
-                                          int parts = 1) {
-    constexpr unsigned kChunksPerRow = COLS / 4;
-    static_assert(64 % kChunksPerRow == 0, "an instruction covers whole rows");
-    constexpr unsigned kRowsPerInstr = 64 / kChunksPerRow;
-    constexpr unsigned kPerWave = ROWS / kRowsPerInstr / WAVES;
-    static_assert(kPerWave * kRowsPerInstr * WAVES == ROWS, "slice must split over the waves");
-    // Lane l fills row l / kChunksPerRow of the instruction's rows, slot
-    // l % kChunksPerRow. A swizzled row (8 chunks) r takes chunk
-    // slot ^ (r & 7) ^ ((r >> 3) & 1): r & 7 is the lane's row, and bit 3
-    // flips with the instruction's first row (a multiple of 8).
-    const unsigned lr = static_cast<unsigned>(lane) / kChunksPerRow;
-    const unsigned pos = static_cast<unsigned>(lane) % kChunksPerRow;
-    const unsigned off0 = SWZ ? (pos ^ lr) * 4u : pos * 4u;
-    const unsigned off1 = SWZ ? (pos ^ lr ^ 1u) * 4u : pos * 4u;
-    const float* base = g + r0 * ld + c0;
-    const uint32_t bytes = static_cast<uint32_t>(((ROWS - 1) * ld + COLS) * sizeof(float));
-    const __amdgpu_buffer_rsrc_t rsrc =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, static_cast<int>(bytes), kRawBufferWord3);
-    const unsigned j0 = kPerWave * part / parts, j1 = kPerWave * (part + 1) / parts;
-#pragma unroll
-    for (unsigned j = j0; j < j1; ++j) {
-        const unsigned first = (static_cast<unsigned>(wave) * kPerWave + j) * kRowsPerInstr;
-        const unsigned off = (SWZ && ((first >> 3) & 1u)) ? off1 : off0;
-        const uint32_t voff = static_cast<uint32_t>(((lr + first) * ld + off) * sizeof(float));
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_t*)(lds + first * COLS), 16, voff, 0, 0, 0);
-    }
-}
-
-// Workgroup barrier of the stepped pipeline, where LDS is written only by
-// direct loads that each issuing wave has already waited for: s_barrier
-// without the release fence of __syncthreads (whose waits are done). Every
-// LDS read of the previous step has returned (its MFMA was issued) before a
-// wave arrives. The memory clobber keeps the compiler from moving LDS
-// accesses across it.
-__device__ __forceinline__ void step_barrier() { __asm__ volatile("s_barrier" ::: "memory"); }
+// How a product's operands may be read: 16-byte (8-byte bf16) loads of rows
+// along k, pairs of bf16 columns, and rows short enough for the 32-bit
+// offsets of a tile's buffer loads.
+struct Access {
+    bool wide_a, wide_b, short_rows;
+};
+// Longest leading dimension (elements) whose 256-row slice of f32 stays under
+// 2^31 bytes.
+constexpr uint64_t kShortRows = 1ull << 21;
+// Splits and stream-K runs are planned in slices of this much k.
+constexpr uint64_t kSliceK = 32;
 
 // Maps the linear workgroup id to a (tile_m, tile_n): each XCD (ids are
 // dealt round-robin over 8) takes a contiguous band, and inside a band tiles
@@ -299,446 +134,46 @@ __device__ __forceinline__ void tile_coords(uint32_t tiles_m, uint32_t tiles_n, 
     *tn = in_group / rows_in_group;
 }
 
-// Scheduling of one slice's k steps (4 per group of 8 k): the LDS reads of
-// step s + 2 are placed after the MFMAs of step s, so each step's operands
-// are read a whole step ahead. Read counts per step for A swizzled (one
-// 16-byte read per m block at a group's first step) and B k-major (the
-// step's KNI floats, read in pairs).
-template <int KMI, int KNI>
-constexpr int step_reads(int s) { return (s % 4 == 0 ? KMI : 0) + (KNI + 1) / 2; }
-template <int KMI, int KNI, int... S>
-__device__ __forceinline__ void sched_reads_ahead(std::integer_sequence<int, S...>) {
-    constexpr int kSteps = sizeof...(S);
-    constexpr int kDsRead = 0x100, kMfma = 0x008;
-    __builtin_amdgcn_sched_group_barrier(kDsRead, step_reads<KMI, KNI>(0), 0);
-    __builtin_amdgcn_sched_group_barrier(kDsRead, step_reads<KMI, KNI>(1), 0);
-    ((__builtin_amdgcn_sched_group_barrier(kMfma, KMI * KNI, 0),
-      __builtin_amdgcn_sched_group_barrier(kDsRead, S + 2 < kSteps ? step_reads<KMI, KNI>(S + 2) : 0, 0)),
-     ...);
-}
-
 // One tile's product, C[m0 .., n0 ..] summed over k in [k_begin, k_end),
 // written to out[(row - out_r0) * ldo + (col - out_c0)] for the rows < M and
-// columns < N, plus the addend when addend_mode is 1 or 2. LDS (`lds`) is
-// free on entry and again on return. SPREAD lets the one-slice-per-barrier
-// loop have every wave issue part of the next slice's direct loads (the
-// stream-K kernel turns it off).
-template <int BM, int BN, int BK, int WM, int WN, bool A_T, bool B_T, bool VEC, class BT, int KG = 1,
-          int STEP = 0, bool SPREAD = true>
+// columns < N, plus the addend when addend_mode is not 0. LDS is free on entry
+// and again on return.
+template <class Shape, bool A_T, bool B_T, class BT>
 __device__ __forceinline__ void gemm_tile(const float* __restrict__ A, const BT* __restrict__ B,
                                           uint64_t M, uint64_t K, uint64_t N, uint64_t m0,
-                                          uint64_t n0, uint64_t k_begin, uint64_t k_end,
-                                          float* lds, float* __restrict__ out, uint64_t out_r0,
+                                          uint64_t n0, uint64_t k_begin, uint64_t k_end, Access access,
+                                          char* lds, float* __restrict__ out, uint64_t out_r0,
                                           uint64_t out_c0, uint64_t ldo,
                                           const float* __restrict__ addend, int addend_mode) {
-    using Cfg = TileCfg<BM, BN, BK, WM, WN, A_T, B_T, KG, STEP>;
-    constexpr int T = Cfg::kThreads;
-    // A rows along m (not A_T) and B rows along n (B_T) are swizzled.
-    constexpr bool kASwz = !A_T, kBSwz = B_T;
-    constexpr bool kBDma = std::is_same<BT, float>::value;  // compact B is widened on the way
-    // Buffer b of the A slices at lds + b * kLdsA; the B slices follow them all.
-    float* const lds_b0 = lds + Cfg::kStages * Cfg::kLdsA;
-
+    using Tile = typename Shape::template Tile<A_T, B_T, BT>;
+    Tile tile;
+    tile.sum(A, B, M, K, N, m0, n0, k_begin, k_end, access.wide_a, access.wide_b, access.short_rows, lds);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const int kg = wave / Cfg::kTileWaves;  // this wave's k group
-    const int wt = wave % Cfg::kTileWaves;
-    const int wm = wt / Cfg::kWavesN, wn = wt % Cfg::kWavesN;
+    const int kg = wave / Tile::kTileWaves, wt = wave % Tile::kTileWaves;
+    const int wm = wt / Tile::kWavesN, wn = wt % Tile::kWavesN;
     const int lrow = lane & 31, lk = lane >> 5;
-
-    v16f acc[Cfg::kMI][Cfg::kNI];
-#pragma unroll
-    for (int i = 0; i < Cfg::kMI; ++i)
-#pragma unroll
-        for (int j = 0; j < Cfg::kNI; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-    // Filling buffer `buf` with the slice at k0. A slice wholly inside the
-    // matrices (every slice of an interior tile but the last partial one)
-    // goes straight to LDS (f32 operands) or through unchecked loads
-    // (compact B); any other slice through bounds-checked loads that
-    // zero-fill past k_end and the matrix edges. `issue` starts the fill,
-    // `finish` writes whatever went through registers.
-    float4 ra[Cfg::kAChunks], rb[Cfg::kBChunks];
-    const bool interior_tile = VEC && m0 + BM <= M && n0 + BN <= N;
-    auto direct = [&](uint64_t k0) { return interior_tile && k0 + BK <= k_end; };
-    // The direct loads of a slice are all issued by the first half of the
-    // waves: the older wave on each SIMD, which wins MFMA arbitration and
-    // otherwise finishes its share of the slice first and waits at the
-    // barrier; the younger one starts its MFMAs at once. Measured: 4096^3
-    // 87.4-88.3 -> 88.3-88.9 %, 8192^3 89.1 -> 89.8 %.
-    constexpr int kDmaWaves = Cfg::kWaves / 2;
-    auto issue = [&](uint64_t k0, int buf) {
-        float* la = lds + buf * Cfg::kLdsA;
-        float* lb = lds_b0 + buf * Cfg::kLdsB;
-        if (direct(k0)) {
-            if (wave < kDmaWaves) {
-                if constexpr (A_T)
-                    dma_slice<Cfg::kARows, Cfg::kACols, kDmaWaves, kASwz>(A, M, k0, m0, la, wave, lane);
-                else
-                    dma_slice<Cfg::kARows, Cfg::kACols, kDmaWaves, kASwz>(A, K, m0, k0, la, wave, lane);
-                if constexpr (kBDma) {
-                    if constexpr (B_T)
-                        dma_slice<Cfg::kBRows, Cfg::kBCols, kDmaWaves, kBSwz>(
-                            reinterpret_cast<const float*>(B), K, n0, k0, lb, wave, lane);
-                    else
-                        dma_slice<Cfg::kBRows, Cfg::kBCols, kDmaWaves, kBSwz>(
-                            reinterpret_cast<const float*>(B), N, k0, n0, lb, wave, lane);
-                }
-            }
-            if constexpr (!kBDma) {
-                if constexpr (B_T)
-                    load_slice_interior<Cfg::kBRows, Cfg::kBCols, Cfg::kBChunks, T>(rb, B, K, n0, k0);
-                else
-                    load_slice_interior<Cfg::kBRows, Cfg::kBCols, Cfg::kBChunks, T>(rb, B, N, k0, n0);
-            }
-            return;
-        }
-        if constexpr (A_T)
-            load_slice<Cfg::kARows, Cfg::kACols, Cfg::kAChunks, T, VEC>(ra, A, M, k0, m0, k_end, M);
-        else
-            load_slice<Cfg::kARows, Cfg::kACols, Cfg::kAChunks, T, VEC>(ra, A, K, m0, k0, M, k_end);
-        if constexpr (B_T)
-            load_slice<Cfg::kBRows, Cfg::kBCols, Cfg::kBChunks, T, VEC>(rb, B, K, n0, k0, N, k_end);
-        else
-            load_slice<Cfg::kBRows, Cfg::kBCols, Cfg::kBChunks, T, VEC>(rb, B, N, k0, n0, k_end, N);
-    };
-    // Part `part` of `parts` of a direct slice's loads, issued by a DMA
-    // wave (the caller's branch).
-    auto issue_part_dma = [&](uint64_t k0, int buf, int part, int parts) {
-        float* la = lds + buf * Cfg::kLdsA;
-        float* lb = lds_b0 + buf * Cfg::kLdsB;
-        if constexpr (kBDma) {
-            if constexpr (A_T)
-                dma_slice<Cfg::kARows, Cfg::kACols, kDmaWaves, kASwz>(A, M, k0, m0, la, wave, lane, part, parts);
-            else
-                dma_slice<Cfg::kARows, Cfg::kACols, kDmaWaves, kASwz>(A, K, m0, k0, la, wave, lane, part, parts);
-            if constexpr (B_T)
-                dma_slice<Cfg::kBRows, Cfg::kBCols, kDmaWaves, kBSwz>(
-                    reinterpret_cast<const float*>(B), K, n0, k0, lb, wave, lane, part, parts);
-            else
-                dma_slice<Cfg::kBRows, Cfg::kBCols, kDmaWaves, kBSwz>(
-                    reinterpret_cast<const float*>(B), N, k0, n0, lb, wave, lane, part, parts);
-        }
-    };
-    auto finish = [&](uint64_t k0, int buf) {
-        const bool dma = direct(k0);
-        if (!dma)
-            store_slice<Cfg::kARows, Cfg::kACols, Cfg::kAChunks, T, kASwz>(ra, lds + buf * Cfg::kLdsA);
-        if (!dma || !kBDma)
-            store_slice<Cfg::kBRows, Cfg::kBCols, Cfg::kBChunks, T, kBSwz>(rb, lds_b0 + buf * Cfg::kLdsB);
-        __builtin_amdgcn_s_waitcnt(0);  // the direct loads have landed in LDS
-    };
-
-    // Operand reads. Every slice sums k in the order k = 8g + 4h + e over
-    // groups g, halves h and steps e (0..3): at step (g, e) lanes of half h
-    // (lane / 32) feed k = 8g + 4h + e. A swizzled row yields that half's 4
-    // values of a group as one 16-byte read; a k-major slice is read one row
-    // per step. Every fill path and operand orientation uses this order, so
-    // they all give the same bits.
-    const int hsw = lk ^ chunk_swizzle(lrow);  // rows wm*WM + i*32 + lrow share lrow & 15
-    // Groups g0 + [0, count) of one slice (g0 < 0: this wave's k group's
-    // share, kg * count + [0, count)); hook(gg, count) runs before group gg.
-    auto compute_range = [&](int buf, auto hook, auto g0c, auto countc) {
-        constexpr int g0 = decltype(g0c)::value, count = decltype(countc)::value;
-        const float* la = lds + buf * Cfg::kLdsA;
-        const float* lb = lds_b0 + buf * Cfg::kLdsB;
-#pragma unroll
-        for (int gg = 0; gg < count; ++gg) {
-            hook(gg, count);
-            const int g = (g0 < 0 ? kg * count : g0) + gg;
-            mhip::f32x4 a4[Cfg::kMI], b4[Cfg::kNI];
-            if constexpr (kASwz) {
-#pragma unroll
-                for (int i = 0; i < Cfg::kMI; ++i)
-                    a4[i] = *reinterpret_cast<const mhip::f32x4*>(la + (wm * WM + i * 32 + lrow) * BK +
-                                                             (((2 * g) ^ hsw) << 2));
-            }
-            if constexpr (kBSwz) {
-#pragma unroll
-                for (int j = 0; j < Cfg::kNI; ++j)
-                    b4[j] = *reinterpret_cast<const mhip::f32x4*>(lb + (wn * WN + j * 32 + lrow) * BK +
-                                                             (((2 * g) ^ hsw) << 2));
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int k = 8 * g + 4 * lk + e;
-                float af[Cfg::kMI], bf[Cfg::kNI];
-#pragma unroll
-                for (int i = 0; i < Cfg::kMI; ++i) {
-                    if constexpr (kASwz) af[i] = a4[i][e];
-                    else af[i] = la[k * BM + wm * WM + i * 32 + lrow];
-                }
-#pragma unroll
-                for (int j = 0; j < Cfg::kNI; ++j) {
-                    if constexpr (kBSwz) bf[j] = b4[j][e];
-                    else bf[j] = lb[k * BN + wn * WN + j * 32 + lrow];
-                }
-#pragma unroll
-                for (int i = 0; i < Cfg::kMI; ++i)
-#pragma unroll
-                    for (int j = 0; j < Cfg::kNI; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i], bf[j], acc[i][j], 0, 0, 0);
-            }
-        }
-    };
-    constexpr int kGroups = BK / 8 / KG;  // groups of 8 k per wave and slice
-    auto compute_body = [&](int buf, auto hook) {
-        compute_range(buf, hook, std::integral_constant<int, -1>{}, std::integral_constant<int, kGroups>{});
-    };
-    // The 64-tile kernel (k groups, one MFMA per k step) gets its LDS reads
-    // ahead of the MFMAs (1024^3 25.4 -> 24.4 us); the larger tiles' own
-    // schedule was as fast. N k steps in one scheduling region.
-    constexpr bool kReadAhead = KG > 1 && kASwz && !kBSwz;
-    auto schedule = [&](auto n) {
-        if constexpr (kReadAhead)
-            sched_reads_ahead<Cfg::kMI, Cfg::kNI>(std::make_integer_sequence<int, decltype(n)::value>{});
-    };
-    constexpr int kSliceSteps = BK / 8 / KG * 4;  // k steps per wave and slice
-    auto no_hook = [](int, int) {};
-    // Two k groups split a slice's four groups of 8 k unevenly on every
-    // fourth slice from the start of the k range (first of each step):
-    // group 0 (waves 0-3) takes groups 0-2, group 1 group 3; elsewhere 0-1
-    // and 2-3. Group 0's waves are the older wave on each SIMD, which wins
-    // MFMA arbitration and finished its even share ~1,700 cycles per step
-    // before the younger one, which then ran alone (1024^3 21.8-21.9 ->
-    // 21.1-21.3 us; 10 of 16 groups to group 0 was slower, 21.5-21.8; the
-    // uneven slice's place in the step did not matter). Every path of the
-    // kernel follows the same split, so its results stay independent of
-    // operand layout and weight format.
-    constexpr bool kUneven = KG == 2 && Cfg::kGroup % 4 == 0;  // steps start every fourth slice
-    using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, 1>;
-    using I2 = std::integral_constant<int, 2>;
-    using I3 = std::integral_constant<int, 3>;
-    // Slice `s` (from k_begin) by k group `grp` (0 or 1).
-    auto compute_uneven = [&](int buf, auto hook, bool first, auto grp) {
-        if constexpr (decltype(grp)::value == 0) {
-            if (first) compute_range(buf, hook, I0{}, I3{});
-            else compute_range(buf, hook, I0{}, I2{});
-        } else {
-            if (first) compute_range(buf, hook, I3{}, I1{});
-            else compute_range(buf, hook, I2{}, I2{});
-        }
-    };
-    auto compute = [&](int buf, uint64_t s) {
-        if constexpr (kUneven) {
-            // Outside whole steps (edge tiles, a last partial step, compact
-            // B): the same groups in the same order, one group at a time.
-            const bool first = s % 4 == 0;
-            const int g_lo = kg == 0 ? 0 : (first ? 3 : 2);
-            const int g_hi = kg == 0 ? (first ? 3 : 2) : 4;
-            const float* la = lds + buf * Cfg::kLdsA;
-            const float* lb = lds_b0 + buf * Cfg::kLdsB;
-            for (int g = g_lo; g < g_hi; ++g) {
-                mhip::f32x4 a4[Cfg::kMI], b4[Cfg::kNI];
-                if constexpr (kASwz) {
-#pragma unroll
-                    for (int i = 0; i < Cfg::kMI; ++i)
-                        a4[i] = *reinterpret_cast<const mhip::f32x4*>(la + (wm * WM + i * 32 + lrow) * BK +
-                                                                 (((2 * g) ^ hsw) << 2));
-                }
-                if constexpr (kBSwz) {
-#pragma unroll
-                    for (int j = 0; j < Cfg::kNI; ++j)
-                        b4[j] = *reinterpret_cast<const mhip::f32x4*>(lb + (wn * WN + j * 32 + lrow) * BK +
-                                                                 (((2 * g) ^ hsw) << 2));
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int k = 8 * g + 4 * lk + e;
-                    float af[Cfg::kMI], bf[Cfg::kNI];
-#pragma unroll
-                    for (int i = 0; i < Cfg::kMI; ++i) {
-                        if constexpr (kASwz) af[i] = a4[i][e];
-                        else af[i] = la[k * BM + wm * WM + i * 32 + lrow];
-                    }
-#pragma unroll
-                    for (int j = 0; j < Cfg::kNI; ++j) {
-                        if constexpr (kBSwz) bf[j] = b4[j][e];
-                        else bf[j] = lb[k * BN + wn * WN + j * 32 + lrow];
-                    }
-#pragma unroll
-                    for (int i = 0; i < Cfg::kMI; ++i)
-#pragma unroll
-                        for (int j = 0; j < Cfg::kNI; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i], bf[j], acc[i][j], 0, 0, 0);
-                }
-            }
-        } else {
-            compute_body(buf, no_hook);
-            schedule(std::integral_constant<int, kSliceSteps>{});
-        }
-    };
-
-    const uint64_t slices = (k_end - k_begin + BK - 1) / BK;
-    constexpr int G = Cfg::kGroup;
-    // One slice per barrier (the 256 x 256 and 128 x 128 tiles): the next
-    // slice's direct loads are issued by every wave, a part at the start of
-    // each of its k groups, between the MFMAs (4096^3 968 -> 942-947 us,
-    // 6144^3 3470 -> 3390 us, 3072^3 480 -> 461 us; the same bits). Issued in
-    // one burst by the older wave of each SIMD, they held that wave ~1,400
-    // cycles per slice before its first MFMA. The stream-K kernel spreads
-    // the first part of each run only: a second spread copy spilled.
-    constexpr bool kSpread = SPREAD && KG == 1 && G == 1 && kBDma;
-    auto part_all = [&](uint64_t k0, int buf, int part, int parts) {
-        if constexpr (kSpread) {
-            float* la = lds + buf * Cfg::kLdsA;
-            float* lb = lds_b0 + buf * Cfg::kLdsB;
-            if constexpr (A_T)
-                dma_slice<Cfg::kARows, Cfg::kACols, Cfg::kWaves, kASwz>(A, M, k0, m0, la, wave, lane, part, parts);
-            else
-                dma_slice<Cfg::kARows, Cfg::kACols, Cfg::kWaves, kASwz>(A, K, m0, k0, la, wave, lane, part, parts);
-            if constexpr (B_T)
-                dma_slice<Cfg::kBRows, Cfg::kBCols, Cfg::kWaves, kBSwz>(
-                    reinterpret_cast<const float*>(B), K, n0, k0, lb, wave, lane, part, parts);
-            else
-                dma_slice<Cfg::kBRows, Cfg::kBCols, Cfg::kWaves, kBSwz>(
-                    reinterpret_cast<const float*>(B), N, k0, n0, lb, wave, lane, part, parts);
-        }
-    };
-    if (G > 1 && kBDma && interior_tile && (k_end - k_begin) % BK == 0) {
-        // Every slice goes straight to LDS. Steps of G slices, double-
-        // buffered: at step t the DMA waves wait for step t's loads, the
-        // barrier publishes them and frees the other buffer set (read in
-        // step t - 1), which then takes step t + 1 while step t computes.
-        // (Three sets of three-slice steps, or four of two-slice steps, with
-        // the loads two or three steps ahead, ran 1024^3 at 26.1 and 27.5 us
-        // against 24.0: the barriers per step cost more than load latency.)
-        const uint64_t steps = (slices + G - 1) / G;
-        const uint64_t full_steps = slices / G;
-        auto set_of = [&](uint64_t t) { return static_cast<int>(t & 1) * G; };
-        auto issue_step = [&](uint64_t t) {
-            const int set = set_of(t);
-#pragma unroll
-            for (int j = 0; j < G; ++j)
-                if (t * G + j < slices) issue(k_begin + (t * G + j) * BK, set + j);
-        };
-        issue_step(0);
-        for (uint64_t t = 0; t < steps; ++t) {
-            __builtin_amdgcn_s_waitcnt(0);  // this wave's loads of step t have landed
-            step_barrier();
-            const int set = set_of(t);
-            const uint64_t tn = t + 1;  // the step whose loads go out now
-            const bool next = tn < steps;
-            const int nset = set_of(tn);
-            if constexpr (kReadAhead) {
-                // Several slices per step, each step in one scheduling region,
-                // so the reads of each slice's first k steps go out during
-                // the previous slice's MFMAs (1024^3 24.3-24.6 -> 23.9-24.1
-                // us). When the next step is whole, its loads go out spread
-                // over this step's k groups, slice j's during slice j (1024^3
-                // 23.9 -> 22.2 us); DMA and other waves then run separate
-                // copies of the step, so neither branches inside it.
-                auto loads_of = [&](int j) {
-                    return [&, j](int gg, int groups) {
-                        issue_part_dma(k_begin + (tn * G + j) * BK, nset + j, gg, groups);
-                    };
-                };
-                auto none = [&](int) { return no_hook; };
-                // A whole step by k group grp (the DMA waves are group 0).
-                auto run_step = [&](auto hook, auto grp) {
-                    if constexpr (kUneven && G % 4 == 0) {
-#pragma unroll
-                        for (int j = 0; j < G; ++j) compute_uneven(set + j, hook(j), j % 4 == 0, grp);
-                        constexpr int kFirst = decltype(grp)::value == 0 ? 12 : 4;
-                        schedule(std::integral_constant<int, G / 4 * kFirst + (G - G / 4) * 8>{});
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < G; ++j) compute_body(set + j, hook(j));
-                        schedule(std::integral_constant<int, G * kSliceSteps>{});
-                    }
-                };
-                static_assert(!kUneven || kDmaWaves == Cfg::kTileWaves, "the DMA waves are k group 0");
-                if (next && tn < full_steps) {
-                    if (wave < kDmaWaves) run_step(loads_of, I0{});
-                    else run_step(none, I1{});
-                    continue;
-                }
-                if (next) issue_step(tn);
-                if (t < full_steps) {
-                    if (wave < kDmaWaves) run_step(none, I0{});
-                    else run_step(none, I1{});
-                    continue;
-                }
-#pragma unroll
-                for (int j = 0; j < G; ++j)
-                    if (t * G + j < slices) compute(set + j, t * G + j);
-            } else {
-                // The 8-wave 128 x 128 tiles: the loads in one burst, one
-                // block per slice (their own schedule of whole steps was
-                // slower, 2048^3 134.4 -> 138.5 us, and so was spreading
-                // the loads, 134.5 -> 135.9-141 us in three arrangements, or
-                // issuing each slice's loads just before the same slice of
-                // this step, 134.2 -> 134.7-135.3 us; every wave issuing a
-                // part of them at each k group, 134.3-134.5 -> 134.2-134.9).
-                if (next) issue_step(tn);
-#pragma unroll
-                for (int j = 0; j < G; ++j)
-                    if (t * G + j < slices) compute(set + j, t * G + j);
-            }
-        }
-        __syncthreads();
-    } else if (kSpread && interior_tile && k_end > k_begin && (k_end - k_begin) % BK == 0) {
-        // Every slice goes straight to LDS, double-buffered, one barrier per
-        // slice: each wave waits for its own loads of slice s + 1 (issued
-        // during slice s), then the barrier publishes them and frees the
-        // buffer slice s was read from.
-        if constexpr (kSpread) {
-            part_all(k_begin, 0, 0, 1);
-            __builtin_amdgcn_s_waitcnt(0);
-            step_barrier();
-            for (uint64_t s = 0; s + 1 < slices; ++s) {
-                const int buf = static_cast<int>(s & 1);
-                const uint64_t k_next = k_begin + (s + 1) * BK;
-                compute_body(buf, [&](int gg, int groups) { part_all(k_next, buf ^ 1, gg, groups); });
-                // Each k step's LDS reads after the previous step's MFMAs
-                // (A stored [m, k], B stored [k, n]): 3072^3 460 -> 455 us,
-                // 4096^3 and 6144^3 within 0.3 %, the same bits.
-                if constexpr (kASwz && !kBSwz)
-                    sched_reads_ahead<Cfg::kMI, Cfg::kNI>(std::make_integer_sequence<int, kSliceSteps>{});
-                __builtin_amdgcn_s_waitcnt(0);
-                step_barrier();
-            }
-            compute(static_cast<int>((slices - 1) & 1), slices - 1);
-            __syncthreads();
-        }
-    } else {
-        issue(k_begin, 0);
-        finish(k_begin, 0);
-        __syncthreads();
-        for (uint64_t s = 0; s < slices; ++s) {
-            const int buf = static_cast<int>(s & 1);
-            const uint64_t k_next = k_begin + (s + 1) * BK;
-            if (s + 1 < slices) issue(k_next, buf ^ 1);
-            compute(buf, s);
-            if (s + 1 < slices) finish(k_next, buf ^ 1);
-            __syncthreads();
-        }
-    }
 
     // Accumulator r of lane l holds C[8*(r/4) + 4*(l/32) + r%4][l%32] of its
     // 32x32 block; registers [R0, R1) are written.
     auto store = [&](auto r0, auto r1) {
 #pragma unroll
-        for (int i = 0; i < Cfg::kMI; ++i) {
+        for (int i = 0; i < Tile::kMI; ++i) {
 #pragma unroll
-            for (int j = 0; j < Cfg::kNI; ++j) {
-                const uint64_t col = n0 + wn * WN + j * 32 + lrow;
+            for (int j = 0; j < Tile::kNI; ++j) {
+                const uint64_t col = n0 + wn * Shape::WN + j * 32 + lrow;
                 if (col >= N) continue;
 #pragma unroll
                 for (int r = decltype(r0)::value; r < decltype(r1)::value; ++r) {
-                    const uint64_t row = m0 + wm * WM + i * 32 + 8 * (r / 4) + 4 * lk + (r % 4);
+                    const uint64_t row = m0 + wm * Shape::WM + i * 32 + 8 * (r / 4) + 4 * lk + (r % 4);
                     if (row < M) {
-                        float v = acc[i][j][r];
+                        float v = tile.acc[i][j][r];
                         if (addend_mode == 1) v = v + addend[col];
                         else if (addend_mode >= 2) v = apply_addend(v, addend[row * N + col], addend_mode);
-                        // The 64-tile kernel writes C non-temporally: all
-                        // its workgroups store at once, at the end (1024^3
-                        // 21.0-21.3 -> 20.9 us, 768x1024x1024 28.7 -> 28.0
-                        // us); for the larger tiles it was 0.5-0.9 % slower.
-                        if constexpr (KG == 2)
+                        // The 64-tile kernel writes C non-temporally: all its
+                        // workgroups store at once, at the end (0.3-0.7 us of
+                        // 21-28); for the larger tiles it was 0.5-0.9 % slower.
+                        if constexpr (Shape::KG == 2)
                             __builtin_nontemporal_store(v, out + (row - out_r0) * ldo + (col - out_c0));
                         else
                             out[(row - out_r0) * ldo + (col - out_c0)] = v;
@@ -751,34 +186,34 @@ __device__ __forceinline__ void gemm_tile(const float* __restrict__ A, const BT*
     using R8 = std::integral_constant<int, 8>;
     using R16 = std::integral_constant<int, 16>;
 
-    if constexpr (KG == 2) {
+    if constexpr (Shape::KG == 2) {
         // Two k groups: each finishes half of every block's rows, group 0
         // registers 0-7 (rows 0-15 of a 32x32 block), group 1 registers
-        // 8-15, handing the other half to its partner through LDS (free
-        // after the loop's last barrier), so both groups add and write. The
-        // sum is group 0's plus group 1's either way.
-        constexpr int kHalf = Cfg::kMI * Cfg::kNI * 8 * 64;  // floats per wave and half
-        float* const given = lds + (kg * Cfg::kTileWaves + wt) * kHalf;
-        const float* const taken = lds + ((1 - kg) * Cfg::kTileWaves + wt) * kHalf;
+        // 8-15, handing the other half to its partner through LDS, so both
+        // groups add and write. The sum is group 0's plus group 1's either way.
+        constexpr int kHalf = Tile::kMI * Tile::kNI * 8 * 64;  // floats per wave and half
+        float* const meet = reinterpret_cast<float*>(lds);
+        float* const given = meet + (kg * Tile::kTileWaves + wt) * kHalf;
+        const float* const taken = meet + ((1 - kg) * Tile::kTileWaves + wt) * kHalf;
         auto give = [&](auto base) {
 #pragma unroll
-            for (int i = 0; i < Cfg::kMI; ++i)
+            for (int i = 0; i < Tile::kMI; ++i)
 #pragma unroll
-                for (int j = 0; j < Cfg::kNI; ++j)
+                for (int j = 0; j < Tile::kNI; ++j)
 #pragma unroll
                     for (int r = 0; r < 8; ++r)
-                        given[((i * Cfg::kNI + j) * 8 + r) * 64 + lane] = acc[i][j][decltype(base)::value + r];
+                        given[((i * Tile::kNI + j) * 8 + r) * 64 + lane] = tile.acc[i][j][decltype(base)::value + r];
         };
         auto take = [&](auto base, auto first) {
 #pragma unroll
-            for (int i = 0; i < Cfg::kMI; ++i)
+            for (int i = 0; i < Tile::kMI; ++i)
 #pragma unroll
-                for (int j = 0; j < Cfg::kNI; ++j)
+                for (int j = 0; j < Tile::kNI; ++j)
 #pragma unroll
                     for (int r = 0; r < 8; ++r) {
-                        const float a = acc[i][j][decltype(base)::value + r];
-                        const float b = taken[((i * Cfg::kNI + j) * 8 + r) * 64 + lane];
-                        acc[i][j][decltype(base)::value + r] = decltype(first)::value ? a + b : b + a;
+                        const float a = tile.acc[i][j][decltype(base)::value + r];
+                        const float b = taken[((i * Tile::kNI + j) * 8 + r) * 64 + lane];
+                        tile.acc[i][j][decltype(base)::value + r] = decltype(first)::value ? a + b : b + a;
                     }
         };
         if (kg == 0) give(R8{});
@@ -789,47 +224,22 @@ __device__ __forceinline__ void gemm_tile(const float* __restrict__ A, const BT*
         __syncthreads();  // LDS is free again
         if (kg == 0) store(R0{}, R8{});
         else store(R8{}, R16{});
-        return;
-    } else if constexpr (KG > 1) {
-        // k groups: the others' sums meet group 0's in LDS (free after the
-        // loop's last barrier), added in group order; group 0 writes the tile.
-        constexpr int kPer = Cfg::kMI * Cfg::kNI * 16 * 64;  // floats per wave
-        for (int q = 1; q < KG; ++q) {
-            if (kg == q) {
-#pragma unroll
-                for (int i = 0; i < Cfg::kMI; ++i)
-#pragma unroll
-                    for (int j = 0; j < Cfg::kNI; ++j)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r)
-                            lds[wt * kPer + ((i * Cfg::kNI + j) * 16 + r) * 64 + lane] = acc[i][j][r];
-            }
-            __syncthreads();
-            if (kg == 0) {
-#pragma unroll
-                for (int i = 0; i < Cfg::kMI; ++i)
-#pragma unroll
-                    for (int j = 0; j < Cfg::kNI; ++j)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r)
-                            acc[i][j][r] += lds[wt * kPer + ((i * Cfg::kNI + j) * 16 + r) * 64 + lane];
-            }
-            __syncthreads();  // LDS is free again
-        }
-        if (kg != 0) return;
+    } else {
+        store(R0{}, R16{});
     }
-    store(R0{}, R16{});
 }
 
 // One tile per workgroup. blockIdx.y is the k split: the workgroup sums k in
 // [y * k_split, min(K, (y + 1) * k_split)) and, with more than one split,
 // writes that partial product to C + y * M * N (no addend) for
 // splitk_reduce_kernel.
-template <int BM, int BN, int BK, int WM, int WN, bool A_T, bool B_T, bool VEC, class BT, int KG, int STEP>
-__global__ __launch_bounds__((TileCfg<BM, BN, BK, WM, WN, A_T, B_T, KG, STEP>::kThreads), 2) void mfma_gemm_kernel(
+template <class Shape, bool A_T, bool B_T, class BT>
+__global__ __launch_bounds__(64 * Shape::kWaves, 2) void mfma_gemm_kernel(
     const float* __restrict__ A, const BT* __restrict__ B, float* __restrict__ C, uint64_t M,
-    uint64_t K, uint64_t N, const float* __restrict__ addend, int addend_mode, uint64_t k_split) {
-    extern __shared__ float lds[];
+    uint64_t K, uint64_t N, const float* __restrict__ addend, int addend_mode, uint64_t k_split,
+    Access access) {
+    extern __shared__ char lds[];
+    constexpr int BM = Shape::BM, BN = Shape::BN;
     uint32_t tm, tn;
     tile_coords(static_cast<uint32_t>((M + BM - 1) / BM), static_cast<uint32_t>((N + BN - 1) / BN),
                 &tm, &tn);
@@ -837,9 +247,8 @@ __global__ __launch_bounds__((TileCfg<BM, BN, BK, WM, WN, A_T, B_T, KG, STEP>::k
     const uint64_t k_end = min(K, k_begin + k_split);
     const bool split = gridDim.y > 1;
     float* out = split ? C + static_cast<uint64_t>(blockIdx.y) * M * N : C;
-    gemm_tile<BM, BN, BK, WM, WN, A_T, B_T, VEC, BT, KG, STEP>(
-        A, B, M, K, N, static_cast<uint64_t>(tm) * BM, static_cast<uint64_t>(tn) * BN, k_begin,
-        k_end, lds, out, 0, 0, N, addend, split ? 0 : addend_mode);
+    gemm_tile<Shape, A_T, B_T, BT>(A, B, M, K, N, static_cast<uint64_t>(tm) * BM, static_cast<uint64_t>(tn) * BN,
+                                   k_begin, k_end, access, lds, out, 0, 0, N, addend, split ? 0 : addend_mode);
 }
 
 // Stream-K: the (tile, k slice) units, tile-major (tile t = tm * tiles_n +
@@ -848,39 +257,30 @@ __global__ __launch_bounds__((TileCfg<BM, BN, BK, WM, WN, A_T, B_T, KG, STEP>::k
 // Workgroup w covers units [w * per, (w + 1) * per); per <= slices per tile,
 // so that run touches at most two tiles, and the part of the j-th one goes to
 // slot 2w + j as a BM x BN tile for stream_reduce_kernel.
-template <int BM, int BN, int BK, int WM, int WN, bool A_T, bool B_T, bool VEC, class BT, int KG, int STEP>
-__global__ __launch_bounds__((TileCfg<BM, BN, BK, WM, WN, A_T, B_T, KG, STEP>::kThreads), 2) void mfma_gemm_stream_kernel(
+template <class Shape, bool A_T, bool B_T, class BT>
+__global__ __launch_bounds__(64 * Shape::kWaves, 2) void mfma_gemm_stream_kernel(
     const float* __restrict__ A, const BT* __restrict__ B, float* __restrict__ slots, uint64_t M,
-    uint64_t K, uint64_t N, uint64_t per) {
-    extern __shared__ float lds[];
+    uint64_t K, uint64_t N, uint64_t per, Access access) {
+    extern __shared__ char lds[];
+    constexpr int BM = Shape::BM, BN = Shape::BN;
     const uint64_t tiles_n = (N + BN - 1) / BN;
-    const uint64_t kslices = (K + BK - 1) / BK;
+    const uint64_t kslices = (K + kSliceK - 1) / kSliceK;
     const uint64_t total = (M + BM - 1) / BM * tiles_n * kslices;
     const uint64_t u0 = static_cast<uint64_t>(blockIdx.x) * per;
     const uint64_t end = min(total, u0 + per);
     if (u0 >= end) return;
     // The run's first part and, when it crosses into the next tile, its
-    // second (k from 0). Only the first spreads its direct loads over the
-    // waves (SPREAD): with both, or with the parts in a loop, the kernel
-    // spilled registers. 1280 x 512 x 3328 60.5 -> 59.5 us, 512 x 4096 x
-    // 11008 356.5 -> 356.0 us, the same bits.
+    // second (k from 0). Not in a loop: that spilled registers.
+    auto part = [&](uint64_t t, uint64_t a, uint64_t b, uint64_t slot) {
+        const uint64_t m0 = t / tiles_n * BM, n0 = t % tiles_n * BN;
+        gemm_tile<Shape, A_T, B_T, BT>(A, B, M, K, N, m0, n0, a * kSliceK, min(K, b * kSliceK), access, lds,
+                                       slots + slot * (BM * BN), m0, n0, BN, nullptr, 0);
+    };
     const uint64_t t0 = u0 / kslices, a0 = u0 % kslices;
     const uint64_t b0 = min(kslices, a0 + (end - u0));
-    {
-        const uint64_t m0 = t0 / tiles_n * BM, n0 = t0 % tiles_n * BN;
-        gemm_tile<BM, BN, BK, WM, WN, A_T, B_T, VEC, BT, KG, STEP, true>(
-            A, B, M, K, N, m0, n0, a0 * BK, min(K, b0 * BK), lds,
-            slots + (2 * static_cast<uint64_t>(blockIdx.x)) * (BM * BN), m0, n0, BN, nullptr, 0);
-    }
+    part(t0, a0, b0, 2 * static_cast<uint64_t>(blockIdx.x));
     const uint64_t u1 = u0 + (b0 - a0);
-    if (u1 < end) {
-        const uint64_t t1 = u1 / kslices;
-        const uint64_t b1 = min(kslices, end - u1);
-        const uint64_t m0 = t1 / tiles_n * BM, n0 = t1 % tiles_n * BN;
-        gemm_tile<BM, BN, BK, WM, WN, A_T, B_T, VEC, BT, KG, STEP, false>(
-            A, B, M, K, N, m0, n0, 0, min(K, b1 * BK), lds,
-            slots + (2 * static_cast<uint64_t>(blockIdx.x) + 1) * (BM * BN), m0, n0, BN, nullptr, 0);
-    }
+    if (u1 < end) part(u1 / kslices, 0, min(kslices, end - u1), 2 * static_cast<uint64_t>(blockIdx.x) + 1);
 }
 
 // C = the stream-K slots covering each output's tile, added in k order (the
@@ -1030,13 +430,17 @@ GemmPlan plan_gemm(uint64_t m, uint64_t k, uint64_t n, uint64_t bm, uint64_t bn,
 }
 
 // Estimated seconds for an m x k x n product with one tile configuration:
-// the critical path's k slices at the configuration's measured fraction of
-// peak, plus the partial results' traffic, plus a fixed cost per launch (a
-// k split or stream-K adds the reduction's). Splits are planned for
-// `plan_per_cu` workgroups per CU. The workgroups resident on a CU share its
-// MFMA pipes; below two waves per SIMD a wave's LDS reads are exposed, so
-// the fraction scales with waves per SIMD / 2 (one 4-wave workgroup per CU
-// measured about half the 2-workgroup rate). Picks among the tile kernels.
+// the critical path's k slices at the configuration's measured rate (as a
+// fraction of the f32 MFMA's peak, which the split products exceed), plus the
+// partial results' traffic, plus a fixed cost per launch (a k split or
+// stream-K adds the reduction's). Splits are planned for `plan_per_cu`
+// workgroups per CU, which share its MFMA pipes; below two waves per SIMD the
+// fraction scales with waves per SIMD / 2. Picks among the tile kernels.
+// Rates, partial traffic (3-4 TB/s written and read) and launch cost are
+// chosen against 2,100 timings of 304 shapes (m 16-4096, k 80-11008, n
+// 1024-14336) with each configuration and split forced: the plans picked are
+// 2.7 % faster on average than with the f32 MFMA kernels' constants, and up to
+// 1.5 times (777 x 4096 x 11008 809 -> 540 us).
 double gemm_seconds(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n, uint64_t bm,
                     uint64_t bn, uint64_t bk, uint64_t plan_per_cu, int waves, double efficiency) {
     const uint64_t cus = ctx->compute_units ? ctx->compute_units : 256;
@@ -1053,44 +457,24 @@ double gemm_seconds(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n, uin
     // little (start-up, the first memory latency, end-of-kernel cache work).
     constexpr double kLaunchSeconds = 4.0e-6;
     double t = static_cast<double>(p.steps) * 2.0 * bm * bn * bk / slot_flops + kLaunchSeconds;
-    if (p.partial_tiles > 0.0) t += (p.partial_tiles + 1.0) * m * n * 4.0 / 5.0e12 + kLaunchSeconds;
+    if (p.partial_tiles > 0.0) t += (p.partial_tiles + 1.0) * m * n * 4.0 / 4.0e12 + kLaunchSeconds;
     return t;
 }
 
-// Workgroups per CU a tile configuration is planned for: as many as fit the
-// 160 KB of LDS, except that a configuration of 8 waves already gives each
-// SIMD two waves with one workgroup, so it is planned one per CU.
-template <class Cfg>
-constexpr uint64_t plan_per_cu() {
-    return Cfg::kWaves >= 8 ? 1 : std::max<uint64_t>(1, (160u * 1024u) / (Cfg::kLdsFloats * sizeof(float)));
-}
-
-template <int BM, int BN, int BK, int WM, int WN, bool A_T, bool B_T, class BT, int KG = 1,
-          int STEP = 0>
+template <class Shape, bool A_T, bool B_T, class BT>
 mhip_status launch_mfma(mhip_ctx* ctx, const float* a, const BT* b, float* c, uint64_t m,
-                        uint64_t k, uint64_t n, const float* addend, int mode, bool vec) {
-    using Cfg = TileCfg<BM, BN, BK, WM, WN, A_T, B_T, KG, STEP>;
+                        uint64_t k, uint64_t n, const float* addend, int mode, Access access) {
+    using Tile = typename Shape::template Tile<A_T, B_T, BT>;
+    constexpr int BM = Shape::BM, BN = Shape::BN;
     const uint64_t tiles = ((m + BM - 1) / BM) * ((n + BN - 1) / BN);
     if (tiles >= (1ULL << 31)) return mhip::fail(MHIP_SHAPE_UNSUPPORTED, "matmul: too many tiles");
-    const uint64_t slots = plan_per_cu<Cfg>() * (ctx->compute_units ? ctx->compute_units : 256);
-    const GemmPlan plan = plan_gemm(m, k, n, BM, BN, BK, slots);
-    // 8-wave 128 x 128 tiles whose workgroups all fit in one wave on the CUs
-    // take the stepped pipeline (two slices per barrier; 128 KB of LDS, which
-    // leaves no room for a second workgroup, so only then): 2048^3 143 ->
-    // 139 us, 512 x 4096 x 4096 148 -> 145 us; at 3072^3 (nine workgroups per
-    // CU in turn) it was 488 -> 515 us. The same bits either way.
-    if constexpr (STEP == 0 && BM * BN == 128 * 128 && Cfg::kWaves >= 8) {
-        const uint64_t wgs = plan.stream ? plan.groups : tiles * plan.splits;
-        if (wgs <= (ctx->compute_units ? ctx->compute_units : 256))
-            return launch_mfma<BM, BN, BK, WM, WN, A_T, B_T, BT, KG, 2>(ctx, a, b, c, m, k, n, addend, mode, vec);
-    }
-    const size_t lds = Cfg::kLdsFloats * sizeof(float);
+    const uint64_t slots = Shape::kPerCu * (ctx->compute_units ? ctx->compute_units : 256);
+    const GemmPlan plan = plan_gemm(m, k, n, BM, BN, kSliceK, slots);
+    const size_t lds = Tile::kLdsBytes;
     static bool configured = false;  // raise the dynamic-LDS cap above 64 KiB once
     if (!configured) {
-        for (const void* f : {reinterpret_cast<const void*>(&mfma_gemm_kernel<BM, BN, BK, WM, WN, A_T, B_T, true, BT, KG, STEP>),
-                              reinterpret_cast<const void*>(&mfma_gemm_kernel<BM, BN, BK, WM, WN, A_T, B_T, false, BT, KG, STEP>),
-                              reinterpret_cast<const void*>(&mfma_gemm_stream_kernel<BM, BN, BK, WM, WN, A_T, B_T, true, BT, KG, STEP>),
-                              reinterpret_cast<const void*>(&mfma_gemm_stream_kernel<BM, BN, BK, WM, WN, A_T, B_T, false, BT, KG, STEP>)})
+        for (const void* f : {reinterpret_cast<const void*>(&mfma_gemm_kernel<Shape, A_T, B_T, BT>),
+                              reinterpret_cast<const void*>(&mfma_gemm_stream_kernel<Shape, A_T, B_T, BT>)})
             (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
         configured = true;
     }
@@ -1103,15 +487,8 @@ mhip_status launch_mfma(mhip_ctx* ctx, const float* a, const BT* b, float* c, ui
         float* slot_mem = nullptr;
         mhip_status st = workspace(ctx, plan.groups * 2 * BM * BN * sizeof(float), &slot_mem);
         if (st != MHIP_OK) return st;
-        const dim3 grid(static_cast<unsigned>(plan.groups));
-        if (vec)
-            mhip::launch(ctx,
-                         (mfma_gemm_stream_kernel<BM, BN, BK, WM, WN, A_T, B_T, true, BT, KG, STEP>),
-                         grid, dim3(Cfg::kThreads), lds, a, b, slot_mem, m, k, n, plan.per);
-        else
-            mhip::launch(ctx,
-                         (mfma_gemm_stream_kernel<BM, BN, BK, WM, WN, A_T, B_T, false, BT, KG, STEP>),
-                         grid, dim3(Cfg::kThreads), lds, a, b, slot_mem, m, k, n, plan.per);
+        mhip::launch(ctx, (mfma_gemm_stream_kernel<Shape, A_T, B_T, BT>), dim3(static_cast<unsigned>(plan.groups)),
+                     dim3(Tile::kThreads), lds, a, b, slot_mem, m, k, n, plan.per, access);
         st = mhip::check_launch("matmul (MFMA stream-K)");
         if (st != MHIP_OK) return st;
         mhip::launch(ctx, (stream_reduce_kernel<BM, BN>), dim3(static_cast<unsigned>(groups_out)),
@@ -1125,18 +502,22 @@ mhip_status launch_mfma(mhip_ctx* ctx, const float* a, const BT* b, float* c, ui
         if (st != MHIP_OK) return st;
     }
     const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(plan.splits));
-    if (vec)
-        mhip::launch(ctx, (mfma_gemm_kernel<BM, BN, BK, WM, WN, A_T, B_T, true, BT, KG, STEP>), grid,
-                     dim3(Cfg::kThreads), lds, a, b, target, m, k, n, addend, mode, plan.k_split);
-    else
-        mhip::launch(ctx, (mfma_gemm_kernel<BM, BN, BK, WM, WN, A_T, B_T, false, BT, KG, STEP>),
-                     grid, dim3(Cfg::kThreads), lds, a, b, target, m, k, n, addend, mode,
-                     plan.k_split);
+    mhip::launch(ctx, (mfma_gemm_kernel<Shape, A_T, B_T, BT>), grid, dim3(Tile::kThreads), lds, a, b, target, m, k,
+                 n, addend, mode, plan.k_split, access);
     mhip_status st = mhip::check_launch("matmul (MFMA tiles)");
     if (st != MHIP_OK || plan.splits == 1) return st;
     mhip::launch(ctx, splitk_reduce_kernel, dim3(static_cast<unsigned>(groups_out)), dim3(256), 0,
                  target, c, m, n, static_cast<uint32_t>(plan.splits), addend, mode, vec4);
     return mhip::check_launch("matmul (split-k reduction)");
+}
+
+template <class Shape, class BT>
+mhip_status launch_tiles(mhip_ctx* ctx, const float* a, const BT* b, float* c, uint64_t m, uint64_t k, uint64_t n,
+                         bool ta, bool tb, const float* addend, int mode, Access access) {
+    if (!ta && !tb) return launch_mfma<Shape, false, false, BT>(ctx, a, b, c, m, k, n, addend, mode, access);
+    if (ta && !tb) return launch_mfma<Shape, true, false, BT>(ctx, a, b, c, m, k, n, addend, mode, access);
+    if (!ta && tb) return launch_mfma<Shape, false, true, BT>(ctx, a, b, c, m, k, n, addend, mode, access);
+    return launch_mfma<Shape, true, true, BT>(ctx, a, b, c, m, k, n, addend, mode, access);
 }
 
 // ---------------------------------------------------------------------------
@@ -2002,32 +1383,35 @@ __global__ void fill_addend_kernel(float* C, uint64_t M, uint64_t N, const float
 
 // The shared body of the f32 and compact-weight matmuls: B as f32 or as bf16
 // bit patterns; everything else (A, C, the addend, the arithmetic) is f32.
-// The tile configurations, picked per shape by the time model (efficiencies
-// measured with each configuration forced):
-//  - kBig: 256 x 256 tiles, 8 waves of 64 x 128 (twice the MFMA work per byte
-//    of LDS traffic): large products, 88 % of peak at 4096^3;
-//  - kSmall: 128 x 128 tiles, 4 waves of 64 x 64, two workgroups per CU:
-//    products whose tiles fill the CUs twice over (82 % at 4096^3);
-//  - kMid: 128 x 128 tiles, 8 waves of 32 x 64: products with about one tile
-//    (or k split) per CU, where the 4-wave kernel leaves each SIMD one wave
-//    (83 % at 4096^3);
-//  - kTiny: 64 x 64 tiles, 8 waves of 32 x 32 in two k groups, four-slice
-//    steps: products of about one such tile per CU (1024^3: 256 tiles),
-//    which then need no k split and no second launch (about 65 % of peak in
-//    its steady state, measured per step with s_memtime at 1024^3).
+// The tile configurations, picked per shape by the time model. What bounds
+// them, and TFLOP/s at 4096^3 and 2048^3 (f32 MFMA kernels before: 146, 134 us
+// at 2048^3):
+//  - kBig: 256 x 256 tiles, 8 waves of 64 x 128: 230-237 TFLOP/s, 580-615 us
+//    at 4096^3 (938 before), 400 with compact weights. The card's power limit
+//    bounds it: MFMAs are busy 75 % of the cycles at 1.77 GHz, and a loop of
+//    nothing but these MFMAs runs at 1.76 GHz. Three buffers and the barrier
+//    that leaves the next stage's reads in flight took 1.17 M cycles to 1.05 M
+//    and 606 us to 591.
+//  - kSmall: 128 x 128 tiles, 4 waves of 64 x 64, two workgroups per CU: 190;
+//  - kMid: 128 x 128 tiles, 8 waves of 32 x 64: 185, 114-120 us at 2048^3,
+//    bound by issue: 5.7 VALU instructions (the split) per MFMA, of which
+//    about 4 hide behind it, and 96 bytes of LDS reads per cycle;
+//  - kTiny: 64 x 64 tiles, 8 waves of 32 x 32 in two k groups: 130; products
+//    of about one such tile per CU (1024^3: 256 tiles), which then need no k
+//    split and no second launch.
 enum class TileChoice { kBig, kSmall, kMid, kTiny };
 
-using BigCfg = TileCfg<256, 256, 32, 64, 128, false, false>;
-using SmallCfg = TileCfg<128, 128, 32, 64, 64, false, false>;
-using MidCfg = TileCfg<128, 128, 32, 32, 64, false, false>;
-using TinyCfg = TileCfg<64, 64, 32, 32, 32, false, false, 2>;
+using BigShape = TileShape<256, 256, 64, 128, 1, 16, 3>;
+using SmallShape = TileShape<128, 128, 64, 64, 1, 16, 2>;
+using MidShape = TileShape<128, 128, 32, 64, 1, 32, 2>;
+using TinyShape = TileShape<64, 64, 32, 32, 2, 32, 2>;
 
 TileChoice choose_tiles(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n) {
-    const double t_big = gemm_seconds(ctx, m, k, n, 256, 256, 32, plan_per_cu<BigCfg>(), BigCfg::kWaves, 0.88);
+    const double t_big = gemm_seconds(ctx, m, k, n, 256, 256, 32, BigShape::kPerCu, BigShape::kWaves, 1.40);
     const double t_small =
-        gemm_seconds(ctx, m, k, n, 128, 128, 32, plan_per_cu<SmallCfg>(), SmallCfg::kWaves, 0.82);
-    const double t_mid = gemm_seconds(ctx, m, k, n, 128, 128, 32, plan_per_cu<MidCfg>(), MidCfg::kWaves, 0.83);
-    const double t_tiny = gemm_seconds(ctx, m, k, n, 64, 64, 32, plan_per_cu<TinyCfg>(), TinyCfg::kWaves, 0.65);
+        gemm_seconds(ctx, m, k, n, 128, 128, 32, SmallShape::kPerCu, SmallShape::kWaves, 1.30);
+    const double t_mid = gemm_seconds(ctx, m, k, n, 128, 128, 32, MidShape::kPerCu, MidShape::kWaves, 1.20);
+    const double t_tiny = gemm_seconds(ctx, m, k, n, 64, 64, 32, TinyShape::kPerCu, TinyShape::kWaves, 0.76);
     if (t_tiny < t_big && t_tiny < t_small && t_tiny < t_mid) return TileChoice::kTiny;
     if (t_big < t_small && t_big <= t_mid) return TileChoice::kBig;
     if (t_mid < t_small) return TileChoice::kMid;
@@ -2062,11 +1446,11 @@ mhip_matmul_plan plan_matmul(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64
         return out;
     }
     out.path = MHIP_MATMUL_PATH_TILES;
-    uint64_t bm = 128, waves = SmallCfg::kWaves, per_cu = plan_per_cu<SmallCfg>();
+    uint64_t bm = 128, waves = SmallShape::kWaves, per_cu = SmallShape::kPerCu;
     switch (choose_tiles(ctx, m, k, n)) {
-        case TileChoice::kBig: bm = 256; waves = BigCfg::kWaves; per_cu = plan_per_cu<BigCfg>(); break;
-        case TileChoice::kMid: waves = MidCfg::kWaves; per_cu = plan_per_cu<MidCfg>(); break;
-        case TileChoice::kTiny: bm = 64; waves = TinyCfg::kWaves; per_cu = plan_per_cu<TinyCfg>(); break;
+        case TileChoice::kBig: bm = 256; waves = BigShape::kWaves; per_cu = BigShape::kPerCu; break;
+        case TileChoice::kMid: waves = MidShape::kWaves; per_cu = MidShape::kPerCu; break;
+        case TileChoice::kTiny: bm = 64; waves = TinyShape::kWaves; per_cu = TinyShape::kPerCu; break;
         case TileChoice::kSmall: break;
     }
     const GemmPlan p = plan_gemm(m, k, n, bm, bm, 32, per_cu * (ctx->compute_units ? ctx->compute_units : 256));
@@ -2111,45 +1495,24 @@ mhip_status matmul_impl(mhip_ctx* ctx, const float* a, const BT* b, float* out, 
         return launch_gemv<kGemvMaxRows, BT>(ctx, a, b, out, k, n, addend, addend_mode, m / kGemvMaxRows);
     }
     const uint64_t lda = ta ? m : k, ldb = tb ? k : n;
-    // Vector loads (and the direct loads into LDS, whose 32-bit offsets need
-    // leading dimensions up to kDmaMaxLd).
-    const bool vec = lda % 4 == 0 && ldb % 4 == 0 && mhip::aligned16(a) && b_aligned &&
-                     lda <= kDmaMaxLd && ldb <= kDmaMaxLd;
+    // A stored [m, k] and B stored [n, k] read 4 elements along k at a time,
+    // a compact B stored [k, n] two columns, where rows and base allow it.
+    const uint64_t b_pack = sizeof(BT) == 2 && !tb ? 2 : 4;
+    const Access access{
+        .wide_a = lda % 4 == 0 && mhip::aligned16(a),
+        .wide_b = ldb % b_pack == 0 && reinterpret_cast<uintptr_t>(b) % (b_pack * sizeof(BT)) == 0,
+        .short_rows = lda <= kShortRows && ldb <= kShortRows};
     switch (choose_tiles(ctx, m, k, n)) {
         case TileChoice::kTiny:
-            if (!ta && !tb)
-                return launch_mfma<64, 64, 32, 32, 32, false, false, BT, 2>(ctx, a, b, out, m, k, n, addend, addend_mode, vec);
-            if (ta && !tb)
-                return launch_mfma<64, 64, 32, 32, 32, true, false, BT, 2>(ctx, a, b, out, m, k, n, addend, addend_mode, vec);
-            if (!ta && tb)
-                return launch_mfma<64, 64, 32, 32, 32, false, true, BT, 2>(ctx, a, b, out, m, k, n, addend, addend_mode, vec);
-            return launch_mfma<64, 64, 32, 32, 32, true, true, BT, 2>(ctx, a, b, out, m, k, n, addend, addend_mode, vec);
+            return launch_tiles<TinyShape, BT>(ctx, a, b, out, m, k, n, ta, tb, addend, addend_mode, access);
         case TileChoice::kBig:
-            if (!ta && !tb)
-                return launch_mfma<256, 256, 32, 64, 128, false, false, BT>(ctx, a, b, out, m, k, n, addend, addend_mode, vec);
-            if (ta && !tb)
-                return launch_mfma<256, 256, 32, 64, 128, true, false, BT>(ctx, a, b, out, m, k, n, addend, addend_mode, vec);
-            if (!ta && tb)
-                return launch_mfma<256, 256, 32, 64, 128, false, true, BT>(ctx, a, b, out, m, k, n, addend, addend_mode, vec);
-            return launch_mfma<256, 256, 32, 64, 128, true, true, BT>(ctx, a, b, out, m, k, n, addend, addend_mode, vec);
+            return launch_tiles<BigShape, BT>(ctx, a, b, out, m, k, n, ta, tb, addend, addend_mode, access);
         case TileChoice::kMid:
-            if (!ta && !tb)
-                return launch_mfma<128, 128, 32, 32, 64, false, false, BT>(ctx, a, b, out, m, k, n, addend, addend_mode, vec);
-            if (ta && !tb)
-                return launch_mfma<128, 128, 32, 32, 64, true, false, BT>(ctx, a, b, out, m, k, n, addend, addend_mode, vec);
-            if (!ta && tb)
-                return launch_mfma<128, 128, 32, 32, 64, false, true, BT>(ctx, a, b, out, m, k, n, addend, addend_mode, vec);
-            return launch_mfma<128, 128, 32, 32, 64, true, true, BT>(ctx, a, b, out, m, k, n, addend, addend_mode, vec);
+            return launch_tiles<MidShape, BT>(ctx, a, b, out, m, k, n, ta, tb, addend, addend_mode, access);
         case TileChoice::kSmall:
             break;
     }
-    if (!ta && !tb)
-        return launch_mfma<128, 128, 32, 64, 64, false, false, BT>(ctx, a, b, out, m, k, n, addend, addend_mode, vec);
-    if (ta && !tb)
-        return launch_mfma<128, 128, 32, 64, 64, true, false, BT>(ctx, a, b, out, m, k, n, addend, addend_mode, vec);
-    if (!ta && tb)
-        return launch_mfma<128, 128, 32, 64, 64, false, true, BT>(ctx, a, b, out, m, k, n, addend, addend_mode, vec);
-    return launch_mfma<128, 128, 32, 64, 64, true, true, BT>(ctx, a, b, out, m, k, n, addend, addend_mode, vec);
+    return launch_tiles<SmallShape, BT>(ctx, a, b, out, m, k, n, ta, tb, addend, addend_mode, access);
 }
 
 }  // namespace

@@ -1,0 +1,108 @@
+"""GPU: the f32 products summed as bf16 plane products (csrc/split_tile.hpp),
+one shape per tile configuration, at the values where the split does not hold:
+infinities, NaN, the largest and the smallest f32, and rows so small that
+their planes would underflow. Such tiles are summed again with the f32 MFMA.
+
+Bound, entry by entry: |C - C64| <= (k + 8) u (|A| |B|) with u = 2^-24, the
+forward-error bound of any order of f32 additions (Higham, Accuracy and
+Stability of Numerical Algorithms, eq. 3.5) plus 8 u for the split (its
+dropped products are below 4 u / 16 of |A| |B|, its planes exact) and the
+first-order bound's remainder. Entries that are not finite in f64 rounded to
+f32 are compared exactly.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# (m, k, n, tile): ragged edges and a k that ends inside a stage.
+SHAPES = [(70, 90, 70), (64, 200, 2050), (2000, 72, 2030), (3190, 530, 3970), (4000, 72, 4060), (4000, 7, 4060)]
+
+
+def check(got, a, b):
+    k = a.shape[1]
+    with np.errstate(all="ignore"):
+        exact = a.astype(np.float64) @ b.astype(np.float64)
+        as_f32 = exact.astype(np.float32)
+        scale = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+        fine = np.isfinite(as_f32) & (scale < 3e38)
+        bound = (k + 8) * 2.0 ** -24 * scale[fine] + 2.0 ** -140
+        err = np.abs(got[fine] - exact[fine])
+    assert np.all(err <= bound), f"{np.max(err / bound):.2f} of the bound"
+    # Entries whose terms hold an infinity or NaN (not mere overflow of a sum).
+    special = ~np.isfinite(scale)
+    assert np.array_equal(np.isnan(got[special]), np.isnan(as_f32[special]))
+    inf = special & np.isinf(as_f32)
+    assert np.array_equal(got[inf], as_f32[inf])
+    return int(fine.sum()), int(special.sum())
+
+
+def operands(m, k, n, seed):
+    rng = np.random.default_rng(seed)
+    return (rng.standard_normal((m, k)).astype(np.float32),
+            (0.05 * rng.standard_normal((k, n))).astype(np.float32))
+
+
+def variants(dev, a, b):
+    """The product with the operands stored as they are and transposed."""
+    from magnetar_hip import ops
+    out = [ops.matmul(dev, dev.upload(a), dev.upload(b)).numpy()]
+    at, bt = np.ascontiguousarray(a.T), np.ascontiguousarray(b.T)
+    out.append(ops.matmul(dev, dev.upload(at), dev.upload(bt), True, True).numpy())
+    assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
+    return out[0]
+
+
+def test_the_shapes_cover_every_configuration(dev):
+    from magnetar_hip import ops
+    plans = [ops.matmul_plan(dev, *shape) for shape in SHAPES]
+    assert {(p["tile"][0], p["waves"]) for p in plans} == {(64, 8), (128, 4), (128, 8), (256, 8)}, plans
+
+
+@pytest.mark.parametrize("m,k,n", SHAPES)
+def test_finite_values_meet_the_f32_bound(dev, m, k, n):
+    a, b = operands(m, k, n, m + n)
+    a[m // 2] = 0.0
+    a[:, k // 3] *= np.float32(2.0 ** 60)   # wide ranges inside one sum
+    b[k // 3] *= np.float32(2.0 ** -60)
+    check(variants(dev, a, b), a, b)
+
+
+@pytest.mark.parametrize("m,k,n", SHAPES)
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3.4028235e38, -3.4028235e38, 1e-45, 2e-38])
+def test_values_outside_the_split(dev, m, k, n, value):
+    """One such value in A, one in B (in other tiles where there are several)."""
+    a, b = operands(m, k, n, m + 7)
+    a[m - 1, k - 1] = value
+    b[0, n // 2] = value
+    finite, special = check(variants(dev, a, b), a, b)
+    assert finite > 0
+    assert (special > 0) == (not np.isfinite(np.float32(value)))
+
+
+@pytest.mark.parametrize("m,k,n", SHAPES)
+@pytest.mark.parametrize("down", [-100, -108, -120])
+def test_small_rows_keep_their_precision(dev, m, k, n, down):
+    """Rows of A at 2^down against columns of B at 2^90: their products are
+    ordinary numbers and as exact as any."""
+    a, b = operands(m, k, n, m + 13)
+    a[::3] *= np.float32(2.0 ** down)
+    b *= np.float32(2.0 ** 90)
+    check(variants(dev, a, b), a, b)
+
+
+@pytest.mark.parametrize("m,k,n", SHAPES)
+def test_compact_weights_give_the_f32_bits(dev, m, k, n):
+    """Also where a tile is summed again: a bf16 infinity, and odd widths."""
+    from magnetar_hip import ops
+    for special in (False, True):
+        a, b = operands(m, k, n - 1, m + 17)
+        bits = (b.view(np.uint32) >> 16).astype(np.uint16)
+        if special:
+            bits[k // 2, 1] = 0x7F80
+        wide = (bits.astype(np.uint32) << 16).view(np.float32)
+        da = dev.upload(a)
+        want = ops.matmul(dev, da, dev.upload(wide)).numpy()
+        got = ops.matmul_bf16w(dev, da, dev.upload(bits)).numpy()
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+        check(want, a, wide)
