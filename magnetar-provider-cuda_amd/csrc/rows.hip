@@ -7,8 +7,9 @@
 // and one LDS exchange between waves, then written once. Many RMSNorm rows of
 // 2052-4096 floats take a 1024-thread workgroup per two rows instead, the
 // second row's loads ahead of the first row's reduction, with the same bits.
-// Rows that are longer, not a multiple of 4 or not 16-byte aligned take a
-// looped kernel that re-reads the row from cache.
+// RMSNorm rows that are longer, not a multiple of 4 or not 16-byte aligned take
+// a looped kernel that re-reads the row from cache; such softmax rows a
+// workgroup of up to 1024 threads that holds up to 65536 floats.
 //
 // The reference uses one 256-thread block and a shared-memory tree for
 // RMSNorm (src/kernels.cu:1098-1138) and one thread per row for softmax
@@ -25,7 +26,6 @@ namespace {
 constexpr int kThreads = 256;
 
 using mhip::group_reduce;
-using mhip::MaxOp;
 using mhip::SumOp;
 using mhip::wave_reduce;
 
@@ -153,14 +153,14 @@ constexpr float kLog2e = 1.4426950408889634f;
 // Softmax partial state over a set of entries: their maximum m (NaN-ignoring,
 // as fmaxf) and s = the sum of exp(x - m) over them. Two states merge into
 // the state of their union by rescaling each sum to the larger maximum; no
-// finite maximum leaves s = 0 (the row then fails). A NaN entry makes s NaN,
+// finite maximum leaves s = 0 or NaN (the row then fails). A NaN entry makes s NaN,
 // which every merge keeps, so the whole row comes out NaN as in the
 // reference's sum.
 __device__ __forceinline__ void merge_state(float& m, float& s, float m2, float s2) {
     const float mm = fmaxf(m, m2);
-    if (mm == -INFINITY) {
+    if (mm == -INFINITY) {  // two zeros, or a NaN
         m = mm;
-        s = 0.0f;
+        s = s + s2;
         return;
     }
     s = s * exp2f((m - mm) * kLog2e) + s2 * exp2f((m2 - mm) * kLog2e);
@@ -188,6 +188,18 @@ __device__ __forceinline__ void group_merge(float& m, float& s, float2* scratch)
 #pragma unroll
         for (int w = 1; w < 4; ++w) merge_state(m, s, scratch[w].x, scratch[w].y);
     }
+}
+
+// The same over all T threads of a workgroup.
+template <int T>
+__device__ __forceinline__ void block_merge(float& m, float& s, float2* scratch) {
+    group_merge<64>(m, s, scratch);
+    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x / 64] = make_float2(m, s);
+    __syncthreads();
+    m = scratch[0].x;
+    s = scratch[0].y;
+#pragma unroll
+    for (int w = 1; w < T / 64; ++w) merge_state(m, s, scratch[w].x, scratch[w].y);
 }
 
 // One pass over the row in registers: each thread takes the maximum m_t of
@@ -267,23 +279,112 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_loop_kernel(
         y[c] = w ? x[c] * inv * w[c] : x[c] * inv;
 }
 
-__global__ __launch_bounds__(kThreads) void softmax_loop_kernel(const float* in, float* out,
-                                                                uint64_t cols, uint32_t* flags) {
-    __shared__ float scratch[4];
+// Rows that softmax_vec_kernel does not take -- longer than 16384, or no whole
+// 16-byte vectors -- on one workgroup of T threads each: E vectors of V floats
+// per thread, all loaded before any is used, then as softmax_vec_kernel. A
+// loop that read the row three times with one load in flight per thread took
+// 59-93 us for one row of 32000 (a vocabulary), 526 for 4096 of them and 90 for
+// 8192 rows of 4095; this takes 9, 201 and 43.
+template <int T, int V, int E>
+__global__ __launch_bounds__(T) void softmax_wide_kernel(const float* in, float* out, uint64_t cols,
+                                                         uint32_t* flags) {
+    __shared__ float2 scratch[T / 64];
     const uint64_t row = blockIdx.x;
     const float* x = in + row * cols;
-    float m = -INFINITY;
-    for (uint64_t c = threadIdx.x; c < cols; c += kThreads) m = fmaxf(m, x[c]);
-    m = group_reduce<256>(m, MaxOp{}, scratch);
-    if (!isfinite(m)) {
+    float v[E][V];
+    float mt = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const uint64_t c = (threadIdx.x + static_cast<uint64_t>(e) * T) * V;
+#pragma unroll
+        for (int i = 0; i < V; ++i) v[e][i] = -INFINITY;
+        if (c < cols) {
+            if constexpr (V == 4) {
+                const float4 t = *reinterpret_cast<const float4*>(x + c);
+                v[e][0] = t.x; v[e][1] = t.y; v[e][2] = t.z; v[e][3] = t.w;
+            } else {
+                v[e][0] = x[c];
+            }
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+#pragma unroll
+        for (int i = 0; i < V; ++i) mt = fmaxf(mt, v[e][i]);
+    const float base = mt == -INFINITY ? 0.0f : mt;
+    float st = 0.0f;
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            v[e][i] = expf(v[e][i] - base);
+            st += v[e][i];
+        }
+    float M = mt, S = st;
+    block_merge<T>(M, S, scratch);
+    if (!isfinite(M)) {
         if (threadIdx.x == 0) atomicOr(flags, MHIP_FLAG_SOFTMAX_NON_FINITE);
         return;
     }
-    float s = 0.0f;
-    for (uint64_t c = threadIdx.x; c < cols; c += kThreads) s += expf(x[c] - m);
-    s = block_reduce_sum(s, scratch);
+    const float scale = expf(mt - M) * (1.0f / S);
     float* y = out + row * cols;
-    for (uint64_t c = threadIdx.x; c < cols; c += kThreads) y[c] = expf(x[c] - m) / s;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const uint64_t c = (threadIdx.x + static_cast<uint64_t>(e) * T) * V;
+        if (c >= cols) continue;
+        if constexpr (V == 4)
+            *reinterpret_cast<float4*>(y + c) =
+                make_float4(v[e][0] * scale, v[e][1] * scale, v[e][2] * scale, v[e][3] * scale);
+        else
+            y[c] = v[e][0] * scale;
+    }
+}
+
+// Rows too long for a workgroup's registers: the row's state in one pass,
+// eight loads in flight per thread, then the outputs from a second (one row of
+// 128000: 225 -> 44 us).
+__global__ __launch_bounds__(1024) void softmax_loop_kernel(const float* in, float* out, uint64_t cols,
+                                                            uint32_t* flags) {
+    constexpr int T = 1024, kU = 8;
+    __shared__ float2 scratch[T / 64];
+    const uint64_t row = blockIdx.x;
+    const float* x = in + row * cols;
+    float M = -INFINITY, S = 0.0f;
+    for (uint64_t c0 = threadIdx.x; c0 < cols; c0 += kU * T) {
+        float v[kU];
+        float m = -INFINITY, s = 0.0f;
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const uint64_t c = c0 + static_cast<uint64_t>(u) * T;
+            v[u] = c < cols ? x[c] : -INFINITY;
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u) m = fmaxf(m, v[u]);
+        const float base = m == -INFINITY ? 0.0f : m;
+#pragma unroll
+        for (int u = 0; u < kU; ++u) s += expf(v[u] - base);
+        merge_state(M, S, m, s);
+    }
+    block_merge<T>(M, S, scratch);
+    if (!isfinite(M)) {
+        if (threadIdx.x == 0) atomicOr(flags, MHIP_FLAG_SOFTMAX_NON_FINITE);
+        return;
+    }
+    const float inv = 1.0f / S;
+    float* y = out + row * cols;
+    for (uint64_t c0 = threadIdx.x; c0 < cols; c0 += kU * T) {
+        float v[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const uint64_t c = c0 + static_cast<uint64_t>(u) * T;
+            v[u] = c < cols ? x[c] : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const uint64_t c = c0 + static_cast<uint64_t>(u) * T;
+            if (c < cols) y[c] = expf(v[u] - M) * inv;
+        }
+    }
 }
 
 enum class RowKind { Rms, Softmax };
@@ -385,9 +486,19 @@ mhip_status mhip_softmax_rows_f32(mhip_ctx* ctx, const float* in, float* out, ui
     if (!in || !out) return mhip::fail(MHIP_SHAPE_UNSUPPORTED, "softmax: null buffer");
     if (rows >= (1ULL << 31)) return mhip::fail(MHIP_SHAPE_UNSUPPORTED, "softmax: too many rows");
     const bool vec = cols % 4 == 0 && mhip::aligned16(in) && mhip::aligned16(out);
-    if (!(vec && dispatch_vec<RowKind::Softmax>(ctx, rows, in, nullptr, out, cols, 0, 0.0f)))
-        mhip::launch(ctx, softmax_loop_kernel, dim3(static_cast<unsigned>(rows)), dim3(kThreads), 0,
-                     in, out, cols, ctx->flags);
+    if (vec && dispatch_vec<RowKind::Softmax>(ctx, rows, in, nullptr, out, cols, 0, 0.0f))
+        return mhip::check_launch("softmax");
+    const dim3 grid(static_cast<unsigned>(rows));
+    // The fewest registers per thread that hold the row; unaligned rows of more
+    // than 32 floats a thread would spill.
+    auto wide = [&](auto kernel, int threads) { mhip::launch(ctx, kernel, grid, dim3(threads), 0, in, out, cols, ctx->flags); };
+    if (vec && cols <= 1024 * 4 * 8) wide(softmax_wide_kernel<1024, 4, 8>, 1024);
+    else if (vec && cols <= 1024 * 4 * 16) wide(softmax_wide_kernel<1024, 4, 16>, 1024);
+    else if (cols <= 256 * 4) wide(softmax_wide_kernel<256, 1, 4>, 256);
+    else if (cols <= 256 * 16) wide(softmax_wide_kernel<256, 1, 16>, 256);
+    else if (cols <= 1024 * 16) wide(softmax_wide_kernel<1024, 1, 16>, 1024);
+    else if (cols <= 1024 * 32) wide(softmax_wide_kernel<1024, 1, 32>, 1024);
+    else wide(softmax_loop_kernel, 1024);
     return mhip::check_launch("softmax");
 }
 
