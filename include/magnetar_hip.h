@@ -199,7 +199,10 @@ enum {
     MHIP_MATMUL_PATH_GEMV = 0,
     MHIP_MATMUL_PATH_GEMV_ROW_BLOCKS = 1,
     MHIP_MATMUL_PATH_TILES = 2,
-    MHIP_MATMUL_PATH_SMALL_TILES = 3
+    MHIP_MATMUL_PATH_SMALL_TILES = 3,
+    MHIP_MATMUL_PATH_GEMV_RAGGED = 4, /* rows of b that are no whole vectors */
+    MHIP_MATMUL_PATH_ROW_DOTS = 5,    /* up to 8 rows, b stored [n, k] */
+    MHIP_MATMUL_PATH_ROW_PANEL = 6    /* 9-32 rows, b stored [k, n] */
 };
 typedef struct {
     uint32_t path;

@@ -1,0 +1,374 @@
+// Products of a few rows whose time is the reading of B once.
+//
+//  - ragged_gemv_kernel: up to 8 rows, B stored [k, n] with rows that are not
+//    whole 16-byte vectors.
+//  - panel_kernel: 9-32 rows, B stored [k, n]. Every wave streams its own 32
+//    columns (64 of a compact B) of a k slice straight into the MFMA's operand
+//    layout, 64 k ahead, splits them in registers and multiplies them with A's
+//    planes, which the workgroup keeps in LDS; nothing waits between the waves
+//    but the change of A's chunk.
+//  - dot_kernel: up to 8 rows, B stored [n, k] (a tied output head). Lanes run
+//    along k, a wave takes several rows of B at a time.
+#pragma once
+
+#include "split_tile.hpp"
+
+namespace mhip {
+
+// ---------------------------------------------------------------------------
+// 9-32 rows, B [k, n]
+// ---------------------------------------------------------------------------
+
+constexpr int kPanelRows = 32;
+constexpr int kPanelWaves = 8;
+constexpr int kPanelK = 256;    // k of A in LDS at a time (48 KB of planes)
+constexpr int kPanelDepth = 4;  // steps of 16 k that a wave reads ahead
+// Column blocks of 32 a wave takes: two of a compact B, read in pairs of
+// columns. The f32 tests and sums again 256 columns at a time.
+template <class BT>
+constexpr int kPanelBlocks = sizeof(BT) == 2 ? 2 : 1;
+template <class BT>
+constexpr int kPanelCols = kPanelWaves * 32 * kPanelBlocks<BT>;
+
+// A k slice's sums of 32 rows by kPanelCols columns: blockIdx.x the columns,
+// blockIdx.y the slice [y * k_slice, ...), k_slice a multiple of 16. Writes C
+// itself (one slice, with the addend) or the slice's partial product at
+// C + y * M * N. n is even and B 4-byte aligned.
+//
+// What bounds it: the bytes in flight, so the waves a CU holds (two workgroups
+// at 128 registers). The 64 x 64 tiles that these products took before keep 8
+// KB of B in flight per workgroup; here each of 16 waves per CU keeps 8 KB.
+// 24 x 4096 x 11008: f32 MFMA tiles 149 us, split tiles 74, this 48-51.
+template <class BT, class Addend>
+__global__ __launch_bounds__(64 * kPanelWaves, 4) void panel_kernel(
+    const float* __restrict__ A, const BT* __restrict__ B, float* __restrict__ C, uint64_t M, uint64_t K,
+    uint64_t N, uint64_t k_slice, Addend epilogue) {
+    constexpr bool kBf16 = sizeof(BT) == 2;
+    constexpr int kBlocks = kPanelBlocks<BT>;
+    constexpr int kPlanes = kBf16 ? 1 : 3;
+    constexpr int kChunkBytes = kPanelRows * 16, kPlaneBytes = kPanelK / 8 * kChunkBytes;
+    constexpr int kStream = 2;  // non-temporal
+    __shared__ __attribute__((aligned(16))) char lds[3 * kPlaneBytes];
+    __shared__ int redo[2];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int l32 = lane & 31, h = lane >> 5;
+    const uint32_t n = static_cast<uint32_t>(N);  // the launch checks n < 2^24
+    const uint32_t col0 = (blockIdx.x * kPanelWaves + wave) * 32 * kBlocks;
+    const uint64_t k_begin = static_cast<uint64_t>(blockIdx.y) * k_slice;
+    const uint64_t k_end = min(K, k_begin + k_slice);
+    const uint32_t steps = static_cast<uint32_t>((k_end - k_begin + 15) / 16);
+    // Columns past the edge repeat the last one (the last pair).
+    const uint32_t col = min(col0 + l32 * kBlocks, n - kBlocks);
+
+    // Step t of B: word i is k 16 t + 8 h + i, by buffer loads whose range ends
+    // with the matrix (k past its end reads as zero; a slice that ends before
+    // it is whole steps). Steps past the slice repeat its last.
+    const uint32_t voff = (8 * h * n + col) * static_cast<uint32_t>(sizeof(BT));
+    auto load = [&](uint32_t t, uint32_t (&r)[8]) {
+        const uint64_t k0 = k_begin + min(t, steps - 1) * 16;
+        const uint64_t left = (K - k0) * N * sizeof(BT);
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<BT*>(B + k0 * N), 0, static_cast<int>(static_cast<uint32_t>(min<uint64_t>(left, 0xFFFFFFFFu))),
+            0x00020000);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t soff = i * n * static_cast<uint32_t>(sizeof(BT));
+            r[i] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, voff, soff, kStream);
+        }
+    };
+
+    f32x16 acc[kBlocks];
+    auto clear = [&]() {
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[b][r] = 0.0f;
+    };
+    clear();
+    if (threadIdx.x < 2) redo[threadIdx.x] = 0;  // (the chunks' barriers follow)
+    uint32_t tiny = 0xFFFFFFFFu;
+    uint32_t raw[kPanelDepth][8];
+#pragma unroll
+    for (int d = 0; d < kPanelDepth; ++d) load(d, raw[d]);
+    constexpr uint32_t kChunkSteps = kPanelK / 16;
+    for (uint32_t c0 = 0; c0 < steps; c0 += kChunkSteps) {
+        // A's chunk: 8 threads to a row and 32 k, zeros past the slice.
+        __syncthreads();
+        uint32_t tiny_a = 0xFFFFFFFFu;
+#pragma unroll
+        for (int q = 0; q < kPanelRows * kPanelK / 4 / (64 * kPanelWaves); ++q) {
+            const int f = threadIdx.x + q * 64 * kPanelWaves;
+            const int row = f / 8 % kPanelRows, kk = f % 8 * 4 + f / (8 * kPanelRows) * 32;
+            const uint64_t k = k_begin + c0 * 16 + kk;
+            const float* p = A + min<uint64_t>(row, M - 1) * K;
+            float x[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[i] = k + i < k_end ? p[k + i] : 0.0f;
+            uint32_t lo[3], hi[3];
+            split_pair(x[0], x[1], lo);
+            split_pair(x[2], x[3], hi);
+            tiny_a = split_min(split_min(tiny_a, x[0], x[1]), x[2], x[3]);
+            char* at = lds + kk / 8 * kChunkBytes + row * 16 + kk % 8 * 2;
+#pragma unroll
+            for (int p3 = 0; p3 < 3; ++p3) *reinterpret_cast<u32x2*>(at + p3 * kPlaneBytes) = u32x2{lo[p3], hi[p3]};
+        }
+        if (tiny_a < kSplitTiny) redo[0] = redo[kBlocks - 1] = 1;
+        __syncthreads();
+        const uint32_t c_end = min(steps, c0 + kChunkSteps);
+        for (uint32_t t0 = c0; t0 < c_end; t0 += kPanelDepth) {
+#pragma unroll
+            for (int d = 0; d < kPanelDepth; ++d) {
+                const uint32_t t = t0 + d;
+                if (t >= c_end) break;
+                uint32_t(&r)[8] = raw[d];
+                u32x4 b[kBlocks][kPlanes];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if constexpr (kBf16) {
+                        b[0][0][i] = __builtin_amdgcn_perm(r[2 * i + 1], r[2 * i], 0x05040100u);
+                        b[kBlocks - 1][0][i] = __builtin_amdgcn_perm(r[2 * i + 1], r[2 * i], 0x07060302u);
+#pragma unroll
+                        for (int e = 0; e < 2; ++e)
+                            tiny = split_min(tiny, bf16_lo(r[2 * i + e]), bf16_hi(r[2 * i + e]));
+                    } else {
+                        uint32_t p[3];
+                        const float x0 = __uint_as_float(r[2 * i]), x1 = __uint_as_float(r[2 * i + 1]);
+                        split_pair(x0, x1, p);
+                        tiny = split_min(tiny, x0, x1);
+#pragma unroll
+                        for (int q = 0; q < 3; ++q) b[0][q][i] = p[q];
+                    }
+                }
+                load(t + kPanelDepth, r);
+                bf16x8 a[3];
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+                    a[q] = *reinterpret_cast<const bf16x8*>(lds + q * kPlaneBytes +
+                                                            (2 * static_cast<int>(t - c0) + h) * kChunkBytes + l32 * 16);
+                auto mul = [&](int p, int q) {
+#pragma unroll
+                    for (int j = 0; j < kBlocks; ++j)
+                        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[p], __builtin_bit_cast(bf16x8, b[j][q]),
+                                                                         acc[j], 0, 0, 0);
+                };
+                // The order of SplitTile::stage.
+                if constexpr (!kBf16) mul(0, 2);
+                mul(2, 0);
+                if constexpr (!kBf16) {
+                    mul(1, 1);
+                    mul(0, 1);
+                }
+                mul(1, 0);
+                mul(0, 0);
+            }
+        }
+    }
+
+    // Values outside the split (split_tile.hpp): the waves of 256 columns (the
+    // same whatever B's format) sum again with the f32 MFMA, straight from memory.
+    float probe = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kBlocks; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(acc[j][r], 0.0f, probe);
+    const int part = wave / (kPanelWaves / kBlocks);
+    if (tiny < kSplitTiny || probe != 0.0f) redo[part] = 1;
+    __syncthreads();
+    if (redo[part]) {
+        clear();
+        const float* arow = A + min<uint64_t>(l32, M - 1) * K;
+        for (uint64_t k = k_begin; k < k_end; k += 2) {
+            const uint64_t kh = min(k + h, k_end - 1);
+            const bool on = k + h < k_end;
+            const float x = on ? arow[kh] : 0.0f;
+#pragma unroll
+            for (int j = 0; j < kBlocks; ++j)
+                acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, on ? elem(B + kh * N + col + j) : 0.0f,
+                                                              acc[j], 0, 0, 0);
+        }
+    }
+
+    const bool split = gridDim.y > 1;
+    float* out = split ? C + static_cast<uint64_t>(blockIdx.y) * M * N : C;
+#pragma unroll
+    for (int j = 0; j < kBlocks; ++j) {
+        const uint32_t c = col0 + l32 * kBlocks + j;
+        if (c >= n) continue;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const uint32_t row = 8 * (r / 4) + 4 * h + r % 4;
+            if (row < M) out[row * N + c] = split ? acc[j][r] : epilogue(acc[j][r], row, c);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Up to 8 rows, B [k, n] of any width and alignment
+// ---------------------------------------------------------------------------
+
+// The decode GEMV's split (256 columns and a k slice per workgroup, the
+// slice's rows dealt to 4 waves that meet in LDS) for rows of B that 16-byte
+// loads cannot read: lane l takes columns l, 64 + l, 128 + l, 192 + l of the
+// 256, whole 256-byte runs per load. Such products ran on the 64 x 64 tiles
+// before: 1 x 4096 x 32001 291 us, 8 rows 302; now 93 and 101 us (5.2-5.6 TB/s).
+// The wave number is a scalar, so that A's elements are scalar loads: as vector
+// loads, one per row and k, they bounded 8 rows at 182 us.
+template <int ROWS, class BT, class Addend>
+__global__ __launch_bounds__(256) void ragged_gemv_kernel(const float* __restrict__ A, const BT* __restrict__ B,
+                                                          float* __restrict__ C, uint64_t K, uint64_t N,
+                                                          uint64_t k_per_slice, Addend epilogue) {
+    __shared__ float red[4][ROWS][4][64];
+    const int lane = threadIdx.x & 63;
+    // (A scalar: A's elements are then scalar loads.)
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const uint64_t col0 = static_cast<uint64_t>(blockIdx.x) * 256 + lane;
+    const uint64_t k_begin = static_cast<uint64_t>(blockIdx.y) * k_per_slice;
+    const uint64_t k_end = min(K, k_begin + k_per_slice);
+    uint64_t col[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) col[j] = min(col0 + 64 * j, N - 1);
+    float acc[ROWS][4];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[r][j] = 0.0f;
+    auto add = [&](const BT (&b)[4], uint64_t k) {
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            const float a = A[r * K + k];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[r][j] = __builtin_fmaf(a, elem(&b[j]), acc[r][j]);
+        }
+    };
+    constexpr int kU = 8;  // rows of B in flight: 128 bytes per lane
+    uint64_t k = k_begin + wave;
+    for (; k + 4 * (kU - 1) < k_end; k += 4 * kU) {
+        BT b[kU][4];
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) b[u][j] = __builtin_nontemporal_load(B + (k + 4 * u) * N + col[j]);
+#pragma unroll
+        for (int u = 0; u < kU; ++u) add(b[u], k + 4 * u);
+    }
+    for (; k < k_end; k += 4) {
+        BT b[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) b[j] = B[k * N + col[j]];
+        add(b, k);
+    }
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) red[wave][r][j][lane] = acc[r][j];
+    __syncthreads();
+    // Wave j adds column block j over the waves, in order.
+    const uint64_t c = col0 + 64 * wave;
+    if (c >= N) return;
+    const bool split = gridDim.y > 1;
+    float* out = split ? C + static_cast<uint64_t>(blockIdx.y) * ROWS * N : C;
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+        float v = red[0][r][wave][lane];
+#pragma unroll
+        for (int w = 1; w < 4; ++w) v += red[w][r][wave][lane];
+        out[r * N + c] = split ? v : epilogue(v, r, c);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Up to 8 rows, B [n, k]
+// ---------------------------------------------------------------------------
+
+// C[r, n] = sum_k A[r, k] B[n, k] for ROWS rows of A: a wave takes COLS rows
+// of B, lane l the k of [512 i + 8 l, + 8), its sums met by a butterfly. k is
+// a multiple of 8 and the rows are 16-byte aligned. The f32 and the compact B
+// sum in the same order.
+//
+// What bounds it: HBM for few rows, A's reads from L1 towards 8 (a wave reads
+// all of A for COLS rows of B). One row on the 64 x 64 tiles, 63 of 64 rows of
+// MFMA work for padding, read a 32000 x 4096 head in 370 us (f32 MFMA) and 188
+// (split); here 1 row 104 us (5.0 TB/s), 4 rows 115, 8 rows 173.
+template <int ROWS, int COLS, class BT, class Addend>
+__global__ __launch_bounds__(256) void dot_kernel(const float* __restrict__ A, const BT* __restrict__ B,
+                                                  float* __restrict__ C, uint64_t K, uint64_t N,
+                                                  Addend epilogue) {
+    constexpr bool kBf16 = sizeof(BT) == 2;
+    constexpr int kVecs = kBf16 ? 1 : 2;  // 16-byte loads per 8 elements
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const uint64_t n0 = (static_cast<uint64_t>(blockIdx.x) * 4 + wave) * COLS;
+    if (n0 >= N) return;
+    const BT* rows[COLS];
+#pragma unroll
+    for (int c = 0; c < COLS; ++c) rows[c] = B + min(n0 + c, N - 1) * K;
+    float acc[ROWS][COLS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+        for (int c = 0; c < COLS; ++c) acc[r][c] = 0.0f;
+    auto load = [&](uint64_t k, uint4 (&v)[COLS][kVecs]) {
+#pragma unroll
+        for (int c = 0; c < COLS; ++c)
+#pragma unroll
+            for (int q = 0; q < kVecs; ++q) {
+                v[c][q] = make_uint4(0, 0, 0, 0);
+                if (k < K) v[c][q] = load_nt(reinterpret_cast<const uint4*>(rows[c] + k) + q);
+            }
+    };
+    uint4 next[COLS][kVecs];
+    load(8 * lane, next);
+    for (uint64_t k0 = 0; k0 < K; k0 += 512) {
+        const uint64_t k = k0 + 8 * lane;
+        uint4 cur[COLS][kVecs];
+#pragma unroll
+        for (int c = 0; c < COLS; ++c)
+#pragma unroll
+            for (int q = 0; q < kVecs; ++q) cur[c][q] = next[c][q];
+        if (k0 + 512 < K) load(k + 512, next);
+        float x[ROWS][8];
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (k < K) v = *reinterpret_cast<const float4*>(A + r * K + k + 4 * q);
+                x[r][4 * q] = v.x; x[r][4 * q + 1] = v.y; x[r][4 * q + 2] = v.z; x[r][4 * q + 3] = v.w;
+            }
+#pragma unroll
+        for (int c = 0; c < COLS; ++c) {
+            float b[8];
+            if constexpr (kBf16) {
+                const uint32_t w[4] = {cur[c][0].x, cur[c][0].y, cur[c][0].z, cur[c][0].w};
+#pragma unroll
+                for (int e = 0; e < 8; ++e) b[e] = e & 1 ? bf16_hi(w[e / 2]) : bf16_lo(w[e / 2]);
+            } else {
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    b[4 * q] = __uint_as_float(cur[c][q].x); b[4 * q + 1] = __uint_as_float(cur[c][q].y);
+                    b[4 * q + 2] = __uint_as_float(cur[c][q].z); b[4 * q + 3] = __uint_as_float(cur[c][q].w);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) acc[r][c] = __builtin_fmaf(x[r][e], b[e], acc[r][c]);
+        }
+    }
+    float mine = 0.0f;  // lane r * COLS + c: output (r, n0 + c)
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+        for (int c = 0; c < COLS; ++c) {
+            float v = acc[r][c];
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+            if (lane == r * COLS + c) mine = v;
+        }
+    const int r = lane / COLS;
+    const uint64_t c = n0 + lane % COLS;
+    if (lane < ROWS * COLS && c < N) C[r * N + c] = epilogue(mine, r, c);
+}
+
+}  // namespace mhip

@@ -4,7 +4,7 @@
 // src/kernels.cu:1262-1306): optional transposes (A stored [k, m], B stored
 // [n, k]), f32 accumulation, the addend added to the finished sum.
 //
-// Two kernel families, chosen by shape:
+// Kernel families, chosen by shape:
 //  - MFMA tiles. A workgroup owns a BM x BN tile of C and sums it as bf16
 //    plane products (split_tile.hpp): each operand is read into registers
 //    two or three stages ahead of its use, split there into three bf16 planes
@@ -20,6 +20,9 @@
 //    or in equal runs of (tile, k slice) units per workgroup (stream-K) when
 //    the tiles divide the device badly; partial tiles go to a workspace and a
 //    second launch adds them in k order (deterministic) with the addend.
+//  - Few rows over a large B (few_rows.hpp): 9-32 rows stream B past A's
+//    planes; up to 8 rows take B [n, k], or rows that are no whole vectors, as
+//    it lies.
 //  - m <= kGemvMaxRows (decode), or up to 32 rows of a small product with
 //    k > 1024 in row blocks of 8: the work is reading B once (HBM-bound), so
 //    each wave streams 256 columns of B (512 for compact bf16 weights on up
@@ -39,6 +42,7 @@
 #include "internal.hpp"
 #include "decode_merge.hpp"
 #include "reduce.hpp"
+#include "few_rows.hpp"
 #include "split_tile.hpp"
 
 namespace {
@@ -338,37 +342,64 @@ __global__ __launch_bounds__(256) void stream_reduce_kernel(const float* __restr
 }
 
 // C = sum over splits s = 0, 1, ... of partial[s] (+ addend), added in split
-// order: deterministic. Four floats per thread; `vec`: as one dwordx4.
+// order: deterministic. Four consecutive outputs of one row per thread.
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ partial,
                                                             float* __restrict__ C, uint64_t M,
                                                             uint64_t N, uint32_t splits,
                                                             const float* __restrict__ addend,
-                                                            int addend_mode, int vec) {
+                                                            int addend_mode) {
     const uint64_t total = M * N;
     const uint64_t i = (static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
     if (i >= total) return;
-    if (vec && i + 3 < total) {
-        float4 v = mhip::load_nt(reinterpret_cast<const float4*>(partial + i));
-        for (uint32_t s = 1; s < splits; ++s) {
-            const float4 p = mhip::load_nt(reinterpret_cast<const float4*>(partial + s * total + i));
-            v.x += p.x; v.y += p.y; v.z += p.z; v.w += p.w;
-        }
-        if (addend_mode == 1) {
-            const float4 b = *reinterpret_cast<const float4*>(addend + i % N);
-            v.x = v.x + b.x; v.y = v.y + b.y; v.z = v.z + b.z; v.w = v.w + b.w;
-        } else if (addend_mode >= 2) {
-            v = apply_addend(v, *reinterpret_cast<const float4*>(addend + i), addend_mode);
-        }
-        *reinterpret_cast<float4*>(C + i) = v;
-        return;
+    float4 v = mhip::load_nt(reinterpret_cast<const float4*>(partial + i));
+    for (uint32_t s = 1; s < splits; ++s) {
+        const float4 p = mhip::load_nt(reinterpret_cast<const float4*>(partial + s * total + i));
+        v.x += p.x; v.y += p.y; v.z += p.z; v.w += p.w;
     }
-    for (uint64_t e = i; e < i + 4 && e < total; ++e) {
-        float v = partial[e];
-        for (uint32_t s = 1; s < splits; ++s) v += partial[s * total + e];
-        if (addend_mode == 1) v = v + addend[e % N];
-        else if (addend_mode >= 2) v = apply_addend(v, addend[e], addend_mode);
-        C[e] = v;
+    if (addend_mode == 1) {
+        const float4 b = *reinterpret_cast<const float4*>(addend + i % N);
+        v.x = v.x + b.x; v.y = v.y + b.y; v.z = v.z + b.z; v.w = v.w + b.w;
+    } else if (addend_mode >= 2) {
+        v = apply_addend(v, *reinterpret_cast<const float4*>(addend + i), addend_mode);
     }
+    *reinterpret_cast<float4*>(C + i) = v;
+}
+
+// The same, one element per thread (rows that are not whole vectors), eight
+// splits' loads in flight.
+__global__ __launch_bounds__(256) void splitk_reduce_scalar_kernel(const float* __restrict__ partial,
+                                                                   float* __restrict__ C, uint64_t M, uint64_t N,
+                                                                   uint32_t splits, const float* __restrict__ addend,
+                                                                   int addend_mode) {
+    const uint64_t total = M * N;
+    const uint64_t e = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (e >= total) return;
+    float v = partial[e];
+    uint32_t s = 1;
+    for (; s + 7 < splits; s += 8) {
+        float p[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) p[u] = partial[(s + u) * total + e];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v += p[u];
+    }
+    for (; s < splits; ++s) v += partial[s * total + e];
+    if (addend_mode == 1) v = v + addend[e % N];
+    else if (addend_mode >= 2) v = apply_addend(v, addend[e], addend_mode);
+    C[e] = v;
+}
+
+// Adds a product's partial results (splits of m x n at `partial`) into c.
+mhip_status launch_splitk_reduce(mhip_ctx* ctx, const float* partial, float* c, uint64_t m, uint64_t n,
+                                 uint64_t splits, const float* addend, int mode, const char* what) {
+    // dwordx4: whole rows of 4 and 16-byte aligned output and addend.
+    if (n % 4 == 0 && mhip::aligned16(c) && (mode == 0 || mhip::aligned16(addend)))
+        mhip::launch(ctx, splitk_reduce_kernel, dim3(static_cast<unsigned>((m * n + 1023) / 1024)), dim3(256), 0,
+                     partial, c, m, n, static_cast<uint32_t>(splits), addend, mode);
+    else
+        mhip::launch(ctx, splitk_reduce_scalar_kernel, dim3(static_cast<unsigned>((m * n + 255) / 256)), dim3(256), 0,
+                     partial, c, m, n, static_cast<uint32_t>(splits), addend, mode);
+    return mhip::check_launch(what);
 }
 
 // How many k splits fill the device best: minimises the number of rounds of
@@ -506,9 +537,7 @@ mhip_status launch_mfma(mhip_ctx* ctx, const float* a, const BT* b, float* c, ui
                  n, addend, mode, plan.k_split, access);
     mhip_status st = mhip::check_launch("matmul (MFMA tiles)");
     if (st != MHIP_OK || plan.splits == 1) return st;
-    mhip::launch(ctx, splitk_reduce_kernel, dim3(static_cast<unsigned>(groups_out)), dim3(256), 0,
-                 target, c, m, n, static_cast<uint32_t>(plan.splits), addend, mode, vec4);
-    return mhip::check_launch("matmul (split-k reduction)");
+    return launch_splitk_reduce(ctx, target, c, m, n, plan.splits, addend, mode, "matmul (split-k reduction)");
 }
 
 template <class Shape, class BT>
@@ -600,7 +629,9 @@ __device__ __forceinline__ void gemv_partial_body(
     constexpr int H = CPL / 4;  // float4 groups per lane
     using L = GemvLoad<BT, CPL>;
     __shared__ float4 red[4][ROWS][H][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    // (A scalar: the stored rows' elements are then scalar loads.)
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const uint64_t col = static_cast<uint64_t>(cg) * (64 * CPL) + lane * CPL;
     const bool live = col < N;  // N % CPL == 0: a live lane's columns are all in range
     const uint64_t k_begin = static_cast<uint64_t>(slice) * k_per_slice;
@@ -625,10 +656,12 @@ __device__ __forceinline__ void gemv_partial_body(
         }
     };
     // B rows in flight per lane: 256 bytes for compact weights read 8
-    // columns at a time and for blocks of 8 rows (measured: bf16
-    // 1x4096x11008 22.1 -> 18.3 us, the C1 block 80 -> 61 us), 128 bytes
-    // otherwise (256 was no faster for the f32 decode GEMVs).
-    constexpr int kU = (CPL == 8 || ROWS >= 8 ? 256 : 128) / sizeof(typename L::Raw);
+    // columns at a time and for blocks of 8 rows of a small matrix (measured:
+    // bf16 1x4096x11008 22.1 -> 18.3 us, the C1 block 80 -> 61 us), 128 bytes
+    // otherwise (256 was no faster for the f32 decode GEMVs, and for 8 rows of
+    // a large one its registers cost the waves that hide the latency: with A's
+    // elements as scalar loads, 8x4096x32000 184 -> 92 us, compact 158 -> 82).
+    constexpr int kU = (CPL == 8 || (ROWS >= 8 && !STREAM) ? 256 : 128) / sizeof(typename L::Raw);
     uint64_t kk = k_begin + wave;
     typename L::Raw first[kU];
     const bool first_batch = live && kk + 4 * (kU - 1) < k_end;
@@ -1370,6 +1403,116 @@ mhip_status launch_small_set(mhip_ctx* ctx, const float* a, uint64_t rows, uint6
     return mhip::check_launch("GEMV set (small MFMA tiles)");
 }
 
+// The epilogue of one finished sum at (row, col) (apply_addend).
+struct AddendEpilogue {
+    const float* addend;
+    uint64_t n;
+    int mode;
+    __device__ __forceinline__ float operator()(float v, uint64_t row, uint64_t col) const {
+        if (mode == 1) return v + addend[col];
+        if (mode >= 2) return apply_addend(v, addend[row * n + col], mode);
+        return v;
+    }
+};
+
+// The k slices of a product on panel_kernel: as many as two workgroups per CU
+// (one round of them) allow, at least 128 k each. (The same for compact
+// weights, whose sums are then the f32 weights' bits.)
+void panel_slicing(const mhip_ctx* ctx, uint64_t k, uint64_t n, uint64_t* slices, uint64_t* k_slice) {
+    const uint64_t groups = (n + mhip::kPanelCols<float> - 1) / mhip::kPanelCols<float>;
+    const uint64_t room = (ctx->compute_units ? ctx->compute_units : 256) * 2 / groups;
+    const uint64_t s = std::max<uint64_t>(1, std::min(room, k / 128));
+    *k_slice = ((k + s - 1) / s + 15) / 16 * 16;
+    *slices = (k + *k_slice - 1) / *k_slice;
+}
+
+template <class BT>
+mhip_status launch_panel(mhip_ctx* ctx, const float* a, const BT* b, float* c, uint64_t m, uint64_t k, uint64_t n,
+                         const float* addend, int mode) {
+    constexpr uint64_t kCols = mhip::kPanelCols<BT>;
+    uint64_t slices, k_slice;
+    panel_slicing(ctx, k, n, &slices, &k_slice);
+    float* target = c;
+    if (slices > 1) {
+        mhip_status st = workspace(ctx, slices * m * n * sizeof(float), &target);
+        if (st != MHIP_OK) return st;
+    }
+    mhip::launch(ctx, (mhip::panel_kernel<BT, AddendEpilogue>),
+                 dim3(static_cast<unsigned>((n + kCols - 1) / kCols), static_cast<unsigned>(slices)),
+                 dim3(64 * mhip::kPanelWaves), 0, a, b, target, m, k, n, k_slice,
+                 AddendEpilogue{addend, n, mode});
+    mhip_status st = mhip::check_launch("matmul (row panel)");
+    if (st != MHIP_OK || slices == 1) return st;
+    return launch_splitk_reduce(ctx, target, c, m, n, slices, addend, mode, "matmul (row panel reduction)");
+}
+
+template <class BT, int ROWS>
+mhip_status launch_ragged_gemv(mhip_ctx* ctx, const float* a, const BT* b, float* c, uint64_t k, uint64_t n,
+                               const float* addend, int mode) {
+    uint64_t slices, k_per_slice;
+    gemv_slicing(ctx, k, n, &slices, &k_per_slice);
+    float* target = c;
+    if (slices > 1) {
+        mhip_status st = workspace(ctx, slices * ROWS * n * sizeof(float), &target);
+        if (st != MHIP_OK) return st;
+    }
+    mhip::launch(ctx, (mhip::ragged_gemv_kernel<ROWS, BT, AddendEpilogue>),
+                 dim3(static_cast<unsigned>((n + 255) / 256), static_cast<unsigned>(slices)), dim3(256), 0, a, b,
+                 target, k, n, k_per_slice, AddendEpilogue{addend, n, mode});
+    mhip_status st = mhip::check_launch("matmul (decode partial sums, ragged rows)");
+    if (st != MHIP_OK || slices == 1) return st;
+    return launch_splitk_reduce(ctx, target, c, ROWS, n, slices, addend, mode, "matmul (decode reduction)");
+}
+
+template <class BT>
+mhip_status dispatch_ragged_gemv(mhip_ctx* ctx, const float* a, const BT* b, float* c, uint64_t m, uint64_t k,
+                                 uint64_t n, const float* addend, int mode) {
+    switch (m) {
+        case 1: return launch_ragged_gemv<BT, 1>(ctx, a, b, c, k, n, addend, mode);
+        case 2: return launch_ragged_gemv<BT, 2>(ctx, a, b, c, k, n, addend, mode);
+        case 3: return launch_ragged_gemv<BT, 3>(ctx, a, b, c, k, n, addend, mode);
+        case 4: return launch_ragged_gemv<BT, 4>(ctx, a, b, c, k, n, addend, mode);
+        case 5: return launch_ragged_gemv<BT, 5>(ctx, a, b, c, k, n, addend, mode);
+        case 6: return launch_ragged_gemv<BT, 6>(ctx, a, b, c, k, n, addend, mode);
+        case 7: return launch_ragged_gemv<BT, 7>(ctx, a, b, c, k, n, addend, mode);
+        default: return launch_ragged_gemv<BT, 8>(ctx, a, b, c, k, n, addend, mode);
+    }
+}
+
+// Rows of B per wave: 4 where that leaves every CU eight waves, fewer for
+// short outputs and for more rows of A (their registers).
+template <int ROWS, class BT>
+mhip_status launch_dot(mhip_ctx* ctx, const float* a, const BT* b, float* c, uint64_t k, uint64_t n,
+                       const float* addend, int mode) {
+    const uint64_t waves = static_cast<uint64_t>(ctx->compute_units ? ctx->compute_units : 256) * 8;
+    const AddendEpilogue epilogue{addend, n, mode};
+    auto go = [&](auto cols) {
+        constexpr int kCols = decltype(cols)::value;
+        mhip::launch(ctx, (mhip::dot_kernel<ROWS, kCols, BT, AddendEpilogue>),
+                     dim3(static_cast<unsigned>((n + 4 * kCols - 1) / (4 * kCols))), dim3(256), 0, a, b, c, k, n,
+                     epilogue);
+        return mhip::check_launch("matmul (row dots)");
+    };
+    if (ROWS <= 4 && n >= 4 * waves) return go(std::integral_constant<int, ROWS <= 4 ? 4 : 2>{});
+    if (n >= 2 * waves) return go(std::integral_constant<int, 2>{});
+    return go(std::integral_constant<int, 1>{});
+}
+
+template <class BT>
+mhip_status dispatch_dot(mhip_ctx* ctx, const float* a, const BT* b, float* c, uint64_t m, uint64_t k, uint64_t n,
+                         const float* addend, int mode) {
+    switch (m) {
+        case 1: return launch_dot<1, BT>(ctx, a, b, c, k, n, addend, mode);
+        case 2: return launch_dot<2, BT>(ctx, a, b, c, k, n, addend, mode);
+        case 3: return launch_dot<3, BT>(ctx, a, b, c, k, n, addend, mode);
+        case 4: return launch_dot<4, BT>(ctx, a, b, c, k, n, addend, mode);
+        case 5: return launch_dot<5, BT>(ctx, a, b, c, k, n, addend, mode);
+        case 6: return launch_dot<6, BT>(ctx, a, b, c, k, n, addend, mode);
+        case 7: return launch_dot<7, BT>(ctx, a, b, c, k, n, addend, mode);
+        default: return launch_dot<8, BT>(ctx, a, b, c, k, n, addend, mode);
+    }
+}
+
 // Zero-inner-dimension product: C = 0 (+ addend).
 __global__ void fill_addend_kernel(float* C, uint64_t M, uint64_t N, const float* addend,
                                    int mode) {
@@ -1418,6 +1561,24 @@ TileChoice choose_tiles(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n)
     return TileChoice::kSmall;
 }
 
+// Few-row products by shape (few_rows.hpp), after the vector GEMV: up to 8
+// rows over a B stored [k, n] whose rows (or base) are no whole vectors; up to
+// 8 rows over a B stored [n, k]; 9-32 rows over a B stored [k, n]. Against
+// the 64 x 64 tiles, f32, k 4096, us: 8 ragged rows x 32001 101 (237 on the
+// tiles), 8 row dots x 32000 173 (188); the panel 32 x 11008 53 (74), while
+// 9-32 rows over [n, k] stay on the tiles (16 x 32000 184; a panel whose lanes
+// read along k, 230).
+bool ragged_gemv_fits(uint64_t m, uint64_t n, bool ta, bool tb) {
+    return m <= kGemvMaxRows && !ta && !tb && m * n < (1ULL << 31);
+}
+bool dot_fits(uint64_t m, uint64_t k, uint64_t n, bool ta, bool tb, bool b_aligned) {
+    return m <= kGemvMaxRows && !ta && tb && k % 8 == 0 && b_aligned && n < (1ULL << 31);
+}
+// (Pairs of a compact B's columns; 32-bit offsets over 16 rows of B.)
+bool panel_fits(uint64_t m, uint64_t n, bool ta, bool tb) {
+    return m > kGemvMaxRows && m <= mhip::kPanelRows && !ta && !tb && n % 2 == 0 && n < (1ULL << 24);
+}
+
 // Which kernel path a product takes (the decode GEMV rules of matmul_impl,
 // then the tile choice); `b_aligned`: B's base allows its vector loads.
 mhip_matmul_plan plan_matmul(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n, bool ta,
@@ -1442,6 +1603,28 @@ mhip_matmul_plan plan_matmul(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64
         uint64_t slices, per;
         gemv_slicing(ctx, k, n, &slices, &per);
         out.path = MHIP_MATMUL_PATH_GEMV_ROW_BLOCKS;
+        out.splits = static_cast<uint32_t>(slices);
+        return out;
+    }
+    if (ragged_gemv_fits(m, n, ta, tb)) {
+        uint64_t slices, per;
+        gemv_slicing(ctx, k, n, &slices, &per);
+        out.path = MHIP_MATMUL_PATH_GEMV_RAGGED;
+        out.splits = static_cast<uint32_t>(slices);
+        return out;
+    }
+    if (dot_fits(m, k, n, ta, tb, b_aligned)) {
+        out.path = MHIP_MATMUL_PATH_ROW_DOTS;
+        out.splits = 1;
+        return out;
+    }
+    if (panel_fits(m, n, ta, tb)) {
+        uint64_t slices, per;
+        panel_slicing(ctx, k, n, &slices, &per);
+        out.path = MHIP_MATMUL_PATH_ROW_PANEL;
+        out.tile_m = mhip::kPanelRows;
+        out.tile_n = mhip::kPanelCols<float>;
+        out.waves = mhip::kPanelWaves;
         out.splits = static_cast<uint32_t>(slices);
         return out;
     }
@@ -1477,7 +1660,8 @@ mhip_status matmul_impl(mhip_ctx* ctx, const float* a, const BT* b, float* out, 
                      dim3(256), 0, out, m, n, addend, addend_mode);
         return mhip::check_launch("matmul (empty inner dimension)");
     }
-    const bool ta = transpose_a != 0, tb = transpose_b != 0;
+    // One row of A lies the same either way.
+    const bool ta = transpose_a != 0 && m != 1, tb = transpose_b != 0;
     // B's vector accesses (dwordx4 of f32, or 8 bytes of bf16) need rows of a
     // multiple of 4 elements and an aligned base.
     const uintptr_t b_align = sizeof(BT) == 4 ? 15u : 7u;
@@ -1494,6 +1678,12 @@ mhip_status matmul_impl(mhip_ctx* ctx, const float* a, const BT* b, float* out, 
             return launch_small_mfma<BT>(ctx, a, b, out, m, k, n, addend, addend_mode);
         return launch_gemv<kGemvMaxRows, BT>(ctx, a, b, out, k, n, addend, addend_mode, m / kGemvMaxRows);
     }
+    if (ragged_gemv_fits(m, n, ta, tb))
+        return dispatch_ragged_gemv<BT>(ctx, a, b, out, m, k, n, addend, addend_mode);
+    if (dot_fits(m, k, n, ta, tb, mhip::aligned16(b)) && mhip::aligned16(a))
+        return dispatch_dot<BT>(ctx, a, b, out, m, k, n, addend, addend_mode);
+    if (panel_fits(m, n, ta, tb) && reinterpret_cast<uintptr_t>(b) % 4 == 0)
+        return launch_panel<BT>(ctx, a, b, out, m, k, n, addend, addend_mode);
     const uint64_t lda = ta ? m : k, ldb = tb ? k : n;
     // A stored [m, k] and B stored [n, k] read 4 elements along k at a time,
     // a compact B stored [k, n] two columns, where rows and base allow it.
@@ -1522,7 +1712,7 @@ extern "C" mhip_status mhip_matmul_plan_f32(mhip_ctx* ctx, uint64_t m, uint64_t 
                                             mhip_matmul_plan* plan) {
     MHIP_REQUIRE_CTX(ctx);
     if (!plan) return mhip::fail(MHIP_SHAPE_UNSUPPORTED, "matmul plan: null output");
-    *plan = plan_matmul(ctx, m, k, n, transpose_a != 0, transpose_b != 0, true);
+    *plan = plan_matmul(ctx, m, k, n, transpose_a != 0 && m != 1, transpose_b != 0, true);
     return MHIP_OK;
 }
 

@@ -80,7 +80,8 @@ class MatmulPlan(ctypes.Structure):
                 ("waves", ctypes.c_uint32), ("splits", ctypes.c_uint32), ("stream_k", ctypes.c_uint32)]
 
 
-MATMUL_PATHS = {0: "gemv", 1: "gemv_row_blocks", 2: "tiles", 3: "small_tiles"}
+MATMUL_PATHS = {0: "gemv", 1: "gemv_row_blocks", 2: "tiles", 3: "small_tiles",
+                4: "gemv_ragged", 5: "row_dots", 6: "row_panel"}
 
 
 class AttentionParams(ctypes.Structure):
