@@ -69,7 +69,7 @@ __global__ __launch_bounds__(64 * kPanelWaves, 4) void panel_kernel(
         const uint64_t k0 = k_begin + min(t, steps - 1) * 16;
         const uint64_t left = (K - k0) * N * sizeof(BT);
         const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<BT*>(B + k0 * N), 0, static_cast<int>(static_cast<uint32_t>(min<uint64_t>(left, 0xFFFFFFFFu))),
+            const_cast<BT*>(B + k0 * N), 0, static_cast<int>(static_cast<uint32_t>(left < 0xFFFFFFFFu ? left : 0xFFFFFFFFu)),
             0x00020000);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(64 * kPanelWaves, 4) void panel_kernel(
             const int f = threadIdx.x + q * 64 * kPanelWaves;
             const int row = f / 8 % kPanelRows, kk = f % 8 * 4 + f / (8 * kPanelRows) * 32;
             const uint64_t k = k_begin + c0 * 16 + kk;
-            const float* p = A + min<uint64_t>(row, M - 1) * K;
+            const float* p = A + (row < M ? row : M - 1) * K;
             float x[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) x[i] = k + i < k_end ? p[k + i] : 0.0f;
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(64 * kPanelWaves, 4) void panel_kernel(
     __syncthreads();
     if (redo[part]) {
         clear();
-        const float* arow = A + min<uint64_t>(l32, M - 1) * K;
+        const float* arow = A + (static_cast<uint64_t>(l32) < M ? l32 : M - 1) * K;
         for (uint64_t k = k_begin; k < k_end; k += 2) {
             const uint64_t kh = min(k + h, k_end - 1);
             const bool on = k + h < k_end;
