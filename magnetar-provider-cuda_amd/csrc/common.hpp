@@ -236,6 +236,8 @@ void launch(mhip_ctx* ctx, void (*kernel)(P...), dim3 grid, dim3 block, size_t s
 // attention chunk records). Growing it waits for the stream; a buffer a live
 // graph may read is retired, not freed. Refused while capturing.
 mhip_status workspace(mhip_ctx* ctx, size_t bytes, void** out);
+// Whether that would be refused for a capture.
+bool workspace_short(const mhip_ctx* ctx, size_t bytes);
 
 // Looks up (once per device, with the context's device current) the device
 // address of the allocation-free matmul's fixed scratch array; called when a

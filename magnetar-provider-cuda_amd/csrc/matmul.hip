@@ -88,6 +88,10 @@ mhip_status workspace(mhip_ctx* ctx, size_t bytes, float** out) {
     return st;
 }
 
+// Whether a capture that would take a product of this size without partial
+// sums cannot have the bytes that its few-row kernel wants (choose_tiles).
+bool scratch_short(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n, size_t bytes);
+
 // ---------------------------------------------------------------------------
 // MFMA tiles
 // ---------------------------------------------------------------------------
@@ -460,7 +464,7 @@ GemmPlan plan_gemm(uint64_t m, uint64_t k, uint64_t n, uint64_t bm, uint64_t bn,
     return p;
 }
 
-// Estimated seconds for an m x k x n product with one tile configuration:
+// Estimated seconds for a product m rows high and n wide on plan p of one tile configuration:
 // the critical path's k slices at the configuration's measured rate (as a
 // fraction of the f32 MFMA's peak, which the split products exceed), plus the
 // partial results' traffic, plus a fixed cost per launch (a k split or
@@ -472,11 +476,10 @@ GemmPlan plan_gemm(uint64_t m, uint64_t k, uint64_t n, uint64_t bm, uint64_t bn,
 // 1024-14336) with each configuration and split forced: the plans picked are
 // 2.7 % faster on average than with the f32 MFMA kernels' constants, and up to
 // 1.5 times (777 x 4096 x 11008 809 -> 540 us).
-double gemm_seconds(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n, uint64_t bm,
-                    uint64_t bn, uint64_t bk, uint64_t plan_per_cu, int waves, double efficiency) {
+double gemm_seconds(const mhip_ctx* ctx, uint64_t m, uint64_t n, const GemmPlan& p, uint64_t bm,
+                    uint64_t bn, uint64_t plan_per_cu, int waves, double efficiency, double traffic) {
     const uint64_t cus = ctx->compute_units ? ctx->compute_units : 256;
     const uint64_t slots = plan_per_cu * cus;
-    const GemmPlan p = plan_gemm(m, k, n, bm, bn, bk, slots);
     const uint64_t wgs = p.stream ? p.groups : p.tiles * p.splits;
     const uint64_t resident =
         std::max<uint64_t>(1, std::min<uint64_t>(plan_per_cu, (std::min(wgs, slots) + cus - 1) / cus));
@@ -487,8 +490,8 @@ double gemm_seconds(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n, uin
     // A dependent launch costs about 4 us on this device even when it moves
     // little (start-up, the first memory latency, end-of-kernel cache work).
     constexpr double kLaunchSeconds = 4.0e-6;
-    double t = static_cast<double>(p.steps) * 2.0 * bm * bn * bk / slot_flops + kLaunchSeconds;
-    if (p.partial_tiles > 0.0) t += (p.partial_tiles + 1.0) * m * n * 4.0 / 4.0e12 + kLaunchSeconds;
+    double t = static_cast<double>(p.steps) * 2.0 * bm * bn * kSliceK / slot_flops + kLaunchSeconds;
+    if (p.partial_tiles > 0.0) t += (p.partial_tiles + 1.0) * m * n * 4.0 / traffic + kLaunchSeconds;
     return t;
 }
 
@@ -1432,6 +1435,10 @@ mhip_status launch_panel(mhip_ctx* ctx, const float* a, const BT* b, float* c, u
     constexpr uint64_t kCols = mhip::kPanelCols<BT>;
     uint64_t slices, k_slice;
     panel_slicing(ctx, k, n, &slices, &k_slice);
+    if (slices > 1 && scratch_short(ctx, m, k, n, slices * m * n * sizeof(float))) {
+        slices = 1;
+        k_slice = (k + 15) / 16 * 16;
+    }
     float* target = c;
     if (slices > 1) {
         mhip_status st = workspace(ctx, slices * m * n * sizeof(float), &target);
@@ -1451,6 +1458,10 @@ mhip_status launch_ragged_gemv(mhip_ctx* ctx, const float* a, const BT* b, float
                                const float* addend, int mode) {
     uint64_t slices, k_per_slice;
     gemv_slicing(ctx, k, n, &slices, &k_per_slice);
+    if (slices > 1 && scratch_short(ctx, ROWS, k, n, slices * ROWS * n * sizeof(float))) {
+        slices = 1;
+        k_per_slice = k;
+    }
     float* target = c;
     if (slices > 1) {
         mhip_status st = workspace(ctx, slices * ROWS * n * sizeof(float), &target);
@@ -1549,16 +1560,63 @@ using SmallShape = TileShape<128, 128, 64, 64, 1, 16, 2>;
 using MidShape = TileShape<128, 128, 32, 64, 1, 32, 2>;
 using TinyShape = TileShape<64, 64, 32, 32, 2, 32, 2>;
 
+// One configuration on one product: its estimated time and the bytes of its
+// partial sums.
+struct TileOption {
+    TileChoice choice;
+    double seconds;
+    uint64_t bytes;
+};
+
+// The fastest option by `efficiency` (of kBig, kSmall, kMid, kTiny), of those
+// whose partial sums take at most `limit` bytes; on equal times the one the
+// comparisons name.
+TileOption fastest_tiles(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n, const double (&efficiency)[4],
+                         double traffic, uint64_t limit) {
+    auto option = [&](auto shape, TileChoice choice) {
+        using Shape = decltype(shape);
+        const uint64_t slots = Shape::kPerCu * (ctx->compute_units ? ctx->compute_units : 256);
+        const GemmPlan p = plan_gemm(m, k, n, Shape::BM, Shape::BN, kSliceK, slots);
+        const uint64_t bytes = (p.stream       ? p.groups * 2 * Shape::BM * Shape::BN
+                                : p.splits > 1 ? p.splits * m * n
+                                               : 0) * sizeof(float);
+        double t = gemm_seconds(ctx, m, n, p, Shape::BM, Shape::BN, Shape::kPerCu, Shape::kWaves,
+                                efficiency[static_cast<int>(choice)], traffic);
+        if (bytes > limit) t = INFINITY;
+        return TileOption{choice, t, bytes};
+    };
+    const TileOption big = option(BigShape{}, TileChoice::kBig), small = option(SmallShape{}, TileChoice::kSmall),
+                     mid = option(MidShape{}, TileChoice::kMid), tiny = option(TinyShape{}, TileChoice::kTiny);
+    if (tiny.seconds < big.seconds && tiny.seconds < small.seconds && tiny.seconds < mid.seconds) return tiny;
+    if (big.seconds < small.seconds && big.seconds <= mid.seconds) return big;
+    if (mid.seconds < small.seconds) return mid;
+    return small;
+}
+
+// Which products the entry points with limited scratch take was settled by the
+// plans of the f32 MFMA kernels, whose fractions of the peak kF32 is:
+// mhip_matmul_f32_noalloc, which gives mhip_matmul_f32's bits, refuses partial
+// sums beyond its array, and a capture those beyond the context's workspace,
+// which does not grow while recording. A product whose plan was within the
+// limit then stays within it, by the fastest option that does (for the array
+// one product in 500 over m 9-16384, k and n 1-65536).
+constexpr double kSplit[4] = {1.40, 1.30, 1.20, 0.76}, kF32[4] = {0.88, 0.82, 0.83, 0.65};
+
+bool within_before(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n, uint64_t limit) {
+    return fastest_tiles(ctx, m, k, n, kF32, 5.0e12, UINT64_MAX).bytes <= limit;
+}
+
 TileChoice choose_tiles(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n) {
-    const double t_big = gemm_seconds(ctx, m, k, n, 256, 256, 32, BigShape::kPerCu, BigShape::kWaves, 1.40);
-    const double t_small =
-        gemm_seconds(ctx, m, k, n, 128, 128, 32, SmallShape::kPerCu, SmallShape::kWaves, 1.30);
-    const double t_mid = gemm_seconds(ctx, m, k, n, 128, 128, 32, MidShape::kPerCu, MidShape::kWaves, 1.20);
-    const double t_tiny = gemm_seconds(ctx, m, k, n, 64, 64, 32, TinyShape::kPerCu, TinyShape::kWaves, 0.76);
-    if (t_tiny < t_big && t_tiny < t_small && t_tiny < t_mid) return TileChoice::kTiny;
-    if (t_big < t_small && t_big <= t_mid) return TileChoice::kBig;
-    if (t_mid < t_small) return TileChoice::kMid;
-    return TileChoice::kSmall;
+    TileOption best = fastest_tiles(ctx, m, k, n, kSplit, 4.0e12, UINT64_MAX);
+    if (best.bytes > MHIP_NOALLOC_SCRATCH_BYTES && within_before(ctx, m, k, n, MHIP_NOALLOC_SCRATCH_BYTES))
+        best = fastest_tiles(ctx, m, k, n, kSplit, 4.0e12, MHIP_NOALLOC_SCRATCH_BYTES);
+    if (!ctx->fixed_scratch && mhip::workspace_short(ctx, best.bytes) && within_before(ctx, m, k, n, ctx->workspace_bytes))
+        best = fastest_tiles(ctx, m, k, n, kSplit, 4.0e12, ctx->workspace_bytes);
+    return best.choice;
+}
+
+bool scratch_short(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n, size_t bytes) {
+    return !ctx->fixed_scratch && mhip::workspace_short(ctx, bytes) && within_before(ctx, m, k, n, ctx->workspace_bytes);
 }
 
 // Few-row products by shape (few_rows.hpp), after the vector GEMV: up to 8
@@ -1666,7 +1724,11 @@ mhip_status matmul_impl(mhip_ctx* ctx, const float* a, const BT* b, float* out, 
     // multiple of 4 elements and an aligned base.
     const uintptr_t b_align = sizeof(BT) == 4 ? 15u : 7u;
     const bool b_aligned = (reinterpret_cast<uintptr_t>(b) & b_align) == 0;
-    if (m <= kGemvMaxRows && !ta && !tb && n % 4 == 0 && b_aligned)
+    // (One stored [k, 1] goes the way of ragged rows where a capture has no room.)
+    uint64_t slices = 1, per_slice = k;
+    if (transpose_a && m == 1) gemv_slicing(ctx, k, n, &slices, &per_slice);
+    const bool roomy = slices == 1 || !scratch_short(ctx, m, k, n, slices * n * sizeof(float));
+    if (m <= kGemvMaxRows && !ta && !tb && n % 4 == 0 && b_aligned && roomy)
         return dispatch_gemv<BT>(ctx, a, b, out, m, k, n, addend, addend_mode);
     // A few rows of a small product (up to 32 rows in blocks of 8, at most
     // 2^26 multiply-adds): one launch of small_mfma_kernel up to k = 1024,

@@ -66,6 +66,10 @@ static void release_buffer(mhip_ctx* ctx, void* p) {
     else (void)hipFree(p);
 }
 
+bool workspace_short(const mhip_ctx* ctx, size_t bytes) {
+    return ctx->capturing && ctx->workspace_bytes < bytes;
+}
+
 mhip_status workspace(mhip_ctx* ctx, size_t bytes, void** out) {
     if (ctx->workspace_bytes < bytes) {
         mhip_status st = forbid_in_capture(ctx, "growing the workspace");
