@@ -12,18 +12,18 @@
 // in one launch and equal that many separate calls.
 //
 // Three kernels:
-//  - prefill (head dims 64 and 128): fp32 MFMA flash attention. A workgroup
-//    takes 128 queries of one (batch, head), four waves of 32, and walks the
-//    admitted keys in 32-key tiles loaded straight into LDS (direct
-//    global -> LDS loads, XOR-swizzled, double-buffered). Each wave computes S^T = K . Q^T with v_mfma_f32_32x32x2_f32
+//  - prefill (head dims 32, 64, 80, 96, 112 and 128): flash attention on the
+//    bf16 matrix cores with every operand split into three bf16 planes. A
+//    workgroup takes 256 queries of one (batch, head), eight waves of 32, and
+//    walks the admitted keys in 32-key tiles. Each wave computes S^T = K . Q^T
 //    (Q^T lives in registers, pre-scaled by scale * log2 e), so every lane
 //    owns one query column and 16 of the tile's keys: the online-softmax
 //    max/sum need one exchange with lane l ^ 32. The accumulator registers
 //    are then exactly the B operand of O^T = V^T . P^T, so the output stays
-//    per-lane too. Probabilities are normalised per tile and the running
-//    output rescaled, so it is always a convex combination of V rows and
-//    never overflows (the reference's 1e38 known answer,
-//    src/tests_conformance.rs:2215-2312).
+//    per-lane too. V is scaled down by a power of two above the sum of the
+//    weights, so the running output never overflows (the reference's 1e38
+//    known answer, src/tests_conformance.rs:2215-2312). Operands the split
+//    does not hold go to the f32 MFMA, wave by wave.
 //  - decode (one query row, head dim 4, 8, 16, ..., 256): split-KV. A
 //    workgroup takes one (batch, KV head, key chunk) and the query heads
 //    that share that KV head (up to 8; a larger group is split into slices
@@ -36,6 +36,7 @@
 #include "common.hpp"
 #include "decode_merge.hpp"
 #include "internal.hpp"
+#include "split_tile.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -90,104 +91,33 @@ __device__ __forceinline__ void key_range(const AttnArgs& a, uint64_t qpos, uint
 // Prefill: fp32 MFMA flash attention
 // ---------------------------------------------------------------------------
 
-template <int D, int VD>
-struct PrefillCfg {
-    static_assert(D >= 64 && VD >= 64, "rows of at least 16 chunks (the swizzle spans 16)");
-    static constexpr int kBQ = 128;            // queries per workgroup (4 waves x 32)
-    static constexpr int kBKV = 32;            // keys per tile
-    static constexpr int kKTile = kBKV * D;    // floats; rows unpadded, 16-byte chunks swizzled
-    static constexpr int kVTile = kBKV * VD;
-    static constexpr int kLdsFloats = 2 * kKTile + 2 * kVTile;  // K and V, double-buffered apart
-};
-
-typedef __attribute__((address_space(3))) void lds_void_t;
-// Word 3 of a raw (unformatted, unswizzled) buffer descriptor on gfx950.
-constexpr int kRawBufferWord3 = 0x00020000;
-
-// Rows [k0, k0 + 32) of a row-major [*, W] operand (leading dimension ld)
-// into an LDS tile of 32 x W floats, by direct loads into LDS: one
-// buffer_load_dwordx4 with the lds bit fills 1 KB of consecutive 16-byte
-// slots, lane i slot i. Slot (row, c) holds the row's chunk c ^ (row & 15)
-// (XOR swizzle instead of padding: 16-byte reads of one chunk position down
-// 16 rows, which the LDS serves 16 lanes at a time over its 64 banks, and
-// 4-byte reads across a row hit distinct banks). Rows at or past `rows`
-// repeat row rows - 1 (finite data the caller masks out). Completion is
-// tracked by vmcnt: wait for it before the tile's barrier.
-//
-// Each lane's byte offsets within a tile (row * ld + its chunk) are computed
-// once; a tile's loads address the buffer that starts at g + k0 * ld with
-// those 32-bit offsets. A tile spans 32 * ld * 4 bytes, below 2^32 (the
-// launch checks ld). Buffer loads rather than global_load_lds: the compiler
-// takes a pending global (FLAT) load into LDS for a possible LDS access and
-// then waits for all of a wave's LDS reads at once (1129-1130 -> 1117-1124
-// us at C4, the same bits).
-template <int W>
-struct TileDma {
-    static constexpr int kChunksPerRow = W / 4;
-    static constexpr int kInstrPerWave = 32 * W / 4 / 64 / 4;
-    static_assert((kChunksPerRow & (kChunksPerRow - 1)) == 0 && kChunksPerRow >= 16,
-                  "rows of a power-of-two number of chunks, at least 16");
-    uint32_t off[kInstrPerWave];
-
-    __device__ __forceinline__ TileDma(uint64_t ld, int wave, int lane) {
-#pragma unroll
-        for (int j = 0; j < kInstrPerWave; ++j) {
-            const int slot = (wave * kInstrPerWave + j) * 64 + lane;
-            const int row = slot / kChunksPerRow;
-            const int chunk = (slot % kChunksPerRow) ^ (row & 15);
-            off[j] = static_cast<uint32_t>((row * ld + chunk * 4) * sizeof(float));
-        }
-    }
-
-    __device__ __forceinline__ void load(const float* g, uint64_t ld, uint64_t k0, uint64_t rows,
-                                         float* tile, int wave, int lane) const {
-        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float*>(g + k0 * ld), 0,
-            static_cast<int>(static_cast<uint32_t>(32 * ld * sizeof(float))), kRawBufferWord3);
-        if (k0 + 32 <= rows) {
-#pragma unroll
-            for (int j = 0; j < kInstrPerWave; ++j) {
-                const int slot0 = (wave * kInstrPerWave + j) * 64;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_t*)(tile + slot0 * 4), 16, off[j],
-                                                         0, 0, 0);
-            }
-            return;
-        }
-        const uint32_t end = static_cast<uint32_t>(rows - 1 - k0);  // k0 < rows
-        const uint32_t row_bytes = static_cast<uint32_t>(ld * sizeof(float));
-#pragma unroll
-        for (int j = 0; j < kInstrPerWave; ++j) {
-            const int slot0 = (wave * kInstrPerWave + j) * 64;
-            const uint32_t row = static_cast<uint32_t>(slot0 + lane) / kChunksPerRow;
-            const uint32_t o = row > end ? off[j] - (row - end) * row_bytes : off[j];
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_t*)(tile + slot0 * 4), 16, o, 0, 0, 0);
-        }
-    }
-};
-
-// S^T[key][query] of one tile: A = the K rows (lane -> key l32), B = Q^T.
+// A head dimension of 16 n; the value columns go in blocks of 32 (the last one
+// partly past the row, its columns zero and never stored).
 template <int D>
-__device__ __forceinline__ v16f tile_scores(const float* sk, const float (&qf)[D / 2], int l32,
-                                            int half) {
-    v16f s;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = 0.0f;
-    const float* krow = sk + l32 * D;
-    const int swz = l32 & 15;
-#pragma unroll
-    for (int t = 0; t < D / 2; t += 4) {
-        const int chunk = (half * (D / 8) + t / 4) ^ swz;
-        // A native vector read: read through HIP's float4 struct, the compiler
-        // waited for the next tile's direct loads (vmcnt(0)) before the first
-        // score read, though they fill the other buffer.
-        const mhip::f32x4 kv = *reinterpret_cast<const mhip::f32x4*>(krow + chunk * 4);
-        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[0], qf[t], s, 0, 0, 0);
-        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[1], qf[t + 1], s, 0, 0, 0);
-        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[2], qf[t + 2], s, 0, 0, 0);
-        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[3], qf[t + 3], s, 0, 0, 0);
-    }
-    return s;
-}
+struct PrefillCfg {
+    static_assert(D % 16 == 0 && D <= 128, "whole MFMA steps, and the registers of 128");
+    static constexpr int kWaves = 8;
+    static constexpr int kThreads = 64 * kWaves;
+    static constexpr int kBQ = 32 * kWaves;    // queries per workgroup
+    static constexpr int kBKV = 32;            // keys per tile
+    static constexpr int kSteps = D / 16;      // of the scores' sum
+    static constexpr int kVB = (D + 31) / 32;  // blocks of value columns
+    // K planes: [plane][8 of d][key] 16-byte slots, the chunks 16 bytes apart
+    // in the banks (a row's 8-byte writes go down the chunks). V planes: [plane]
+    // [chunk][column], a chunk the 8 keys of one half of the wave in one step.
+    static constexpr int kKChunk = kBKV * 16 + 16;
+    static constexpr int kKPlane = D / 8 * kKChunk;
+    static constexpr int kVChunk = kVB * 32 * 16;
+    static constexpr int kVPlane = 4 * kVChunk;
+    // At 128 Q's third plane does not fit the registers: it stays in LDS.
+    static constexpr bool kQLds = D > 112;
+    static constexpr int kQBytes = kQLds ? kWaves * kSteps * 1024 : 0;
+    static constexpr int kLdsBytes = 3 * (kKPlane + kVPlane) + kQBytes;
+    // The f32 sum's tiles.
+    static constexpr int kLdF = D + 4;
+    static_assert(2 * kBKV * kLdF * 4 <= kLdsBytes, "its f32 tiles fit");
+    static constexpr int kKUnits = (kBKV * D / 4 + kThreads - 1) / kThreads;
+};
 
 // A wave's queries recomputed over their admitted keys only, on the VALU,
 // after its tile loop: taken when an edge tile of the wave held a non-finite
@@ -196,30 +126,32 @@ __device__ __forceinline__ v16f tile_scores(const float* sk, const float (&qf)[D
 // non-finite V there turns that 0 into NaN, where the reference never reads
 // the key (src/kernels.cu:1909-1920). Here each query visits only [lo, hi)
 // (within the workgroup's key chunk), one key at a time: the score from this
-// lane's half of Q^T (qf, pre-scaled to the log2 domain) and the other
-// half's in lane l ^ 32, an online softmax, and this lane's outputs
+// lane's half of Q^T (scaled to the log2 domain) and the other half's
+// in lane l ^ 32, an online softmax, and this lane's outputs
 // (register r of block vb: column vb*32 + 8*(r/4) + 4*half + r%4), so an
 // admitted inf or NaN gives what the reference's sum gives and a masked one
 // nothing. Slow (each query reads its keys from memory), and only for inputs
 // with non-finite values next to a mask edge; the tile loop's accumulators
 // are dead here, which keeps the kernel within its registers.
-template <int D, int VD>
-__device__ __forceinline__ void recompute_admitted(const float (&qf)[D / 2], const float* K,
+template <int D>
+__device__ __forceinline__ void recompute_admitted(const float* qhalf, float qscale, const float* K,
                                                    uint64_t k_ld, const float* V, uint64_t v_ld,
                                                    uint64_t lo, uint64_t hi, int half,
-                                                   v16f (&o)[VD / 32], float* m_out, float* l_out) {
+                                                   v16f (&o)[PrefillCfg<D>::kVB], float* m_out,
+                                                   float* l_out) {
+    constexpr int kVB = PrefillCfg<D>::kVB;
 #pragma unroll
-    for (int vb = 0; vb < VD / 32; ++vb)
+    for (int vb = 0; vb < kVB; ++vb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[vb][r] = 0.0f;
     float m = -INFINITY, l = 0.0f;
     for (uint64_t j = lo; j < hi; ++j) {
         const float* krow = K + j * k_ld + half * (D / 2);
         float part = 0.0f;
-#pragma unroll
         for (int t = 0; t < D / 2; t += 4) {
             const float4 k4 = *reinterpret_cast<const float4*>(krow + t);
-            part += qf[t] * k4.x + qf[t + 1] * k4.y + qf[t + 2] * k4.z + qf[t + 3] * k4.w;
+            const float4 q4 = *reinterpret_cast<const float4*>(qhalf + t);
+            part += q4.x * qscale * k4.x + q4.y * qscale * k4.y + q4.z * qscale * k4.z + q4.w * qscale * k4.w;
         }
         const float s = part + __shfl_xor(part, 32, 64);
         const float m_new = fmaxf(m, s);
@@ -229,10 +161,12 @@ __device__ __forceinline__ void recompute_admitted(const float (&qf)[D / 2], con
         l = l * alpha + w;
         const float* vrow = V + j * v_ld;
 #pragma unroll
-        for (int vb = 0; vb < VD / 32; ++vb)
+        for (int vb = 0; vb < kVB; ++vb)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const float4 v4 = *reinterpret_cast<const float4*>(vrow + vb * 32 + 8 * g + 4 * half);
+                const int c = vb * 32 + 8 * g + 4 * half;
+                if (D % 32 != 0 && c >= D) continue;
+                const float4 v4 = *reinterpret_cast<const float4*>(vrow + c);
                 o[vb][4 * g] = o[vb][4 * g] * alpha + w * v4.x;
                 o[vb][4 * g + 1] = o[vb][4 * g + 1] * alpha + w * v4.y;
                 o[vb][4 * g + 2] = o[vb][4 * g + 2] * alpha + w * v4.z;
@@ -242,7 +176,7 @@ __device__ __forceinline__ void recompute_admitted(const float (&qf)[D / 2], con
     }
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
 #pragma unroll
-    for (int vb = 0; vb < VD / 32; ++vb)
+    for (int vb = 0; vb < kVB; ++vb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[vb][r] *= inv;
     *m_out = m;
@@ -258,240 +192,526 @@ __device__ __forceinline__ void recompute_admitted(const float (&qf)[D / 2], con
 struct PrefillSplit {
     uint32_t nchunks;      // 1: no split, the kernel writes the output itself
     uint32_t chunk_tiles;
+    uint32_t qtiles, pairs, group;  // query tiles; (batch, head) pairs; query heads of a KV head
     float* part_o;         // [batch * seq][heads][nchunks][VD]
     float* part_ml;        // [batch * seq][heads][nchunks][2]
 };
 
-// The workgroup walks its key tiles double-buffered in LDS, each tile loaded
-// straight from global memory into LDS (no register staging), which keeps
-// the kernel within 256 registers: two waves per SIMD, one from each of the
-// two workgroups a CU holds, overlap each other's MFMA and softmax phases.
-template <int D, int VD>
-__global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnArgs a, PrefillSplit sp) {
-    apply_advance(a);
-    using Cfg = PrefillCfg<D, VD>;
-    extern __shared__ float lds[];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const int l32 = lane & 31, half = lane >> 5;
+// What a thread works on: its workgroup's operands and key tiles, its wave's
+// and its lane's key ranges. Keys count from the workgroup's first tile (32-bit:
+// the caller keeps key counts below 2^31).
+struct PrefillPlace {
+    const float *qrow, *K, *V;
+    float* out;            // the query's output row, or its chunk record's
+    float* ml;             // the chunk record's max and sum (nullptr: none)
+    uint64_t tile_begin;
+    int i_begin, i_end;    // tiles
+    bool q_live;
+    int lo, hi;            // keys the lane's query admits
+    int any_lo, any_hi;    // keys any query of the wave admits
+    int all_lo, all_hi;    // keys every query of the wave admits
+};
 
-    // Heaviest (latest) query tiles first over the whole grid: under a causal
-    // mask they see the most keys. Block ids are dealt round-robin to the 8
-    // XCDs, so consecutive ids take the same query tile of different (batch,
-    // head) pairs: every XCD gets an equal share of each weight class and runs
-    // it heaviest first (ids of one head's query tiles, dealt to XCDs by
-    // query tile, left XCDs with 2.4x the work of others).
-    const uint64_t qtiles = (a.seq + Cfg::kBQ - 1) / Cfg::kBQ;
-    const uint64_t chunk = blockIdx.x % sp.nchunks;
-    const uint64_t pairs = gridDim.x / sp.nchunks / qtiles;
-    const uint64_t bid = blockIdx.x / sp.nchunks;
-    const uint64_t qt = qtiles - 1 - bid / pairs;
-    const uint64_t bh = bid % pairs;
-    const uint64_t head = bh % a.heads, b = bh / a.heads;
-    const uint64_t kvh = head / (a.heads / a.kv_heads);
-
-    const float* Q = a.q + b * a.q_bs + head * D;
-    const float* K = a.k + b * a.k_bs + kvh * D;
-    const float* V = a.v + b * a.v_bs + kvh * VD;
-    float* O = a.out + b * a.o_bs + head * VD;
-    const uint64_t q_ld = a.heads * D, k_ld = a.kv_heads * D, v_ld = a.kv_heads * VD,
-                   o_ld = a.heads * VD;
-
-    // This lane's query and its Q^T operand: Q[q][half * D/2 + t], t < D/2.
-    const uint64_t q_first = qt * Cfg::kBQ;
-    const uint64_t q = q_first + wave * 32 + l32;
-    const bool q_live = q < a.seq;
-    float qf[D / 2];
-#pragma unroll
-    for (int t = 0; t < D / 2; t += 4) {
-        float4 v4 = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (q_live) v4 = *reinterpret_cast<const float4*>(Q + q * q_ld + half * (D / 2) + t);
-        qf[t] = v4.x * a.qscale;
-        qf[t + 1] = v4.y * a.qscale;
-        qf[t + 2] = v4.z * a.qscale;
-        qf[t + 3] = v4.w * a.qscale;
+// Heaviest (latest) query tiles first over the whole grid: under a causal
+// mask they see the most keys. Block ids are dealt round-robin to the 8
+// XCDs, so consecutive ids take the same query tile of different (batch,
+// head) pairs: every XCD gets an equal share of each weight class and runs
+// it heaviest first (ids of one head's query tiles, dealt to XCDs by
+// query tile, left XCDs with 2.4x the work of others).
+//
+// Block and key counts are below 2^31, so all of it is 32-bit, mostly scalar,
+// and a division that a call does not need (one query tile, one sequence, no
+// shared KV heads) is skipped: a prompt of 32 waits for each in turn.
+template <int D>
+__device__ __forceinline__ PrefillPlace prefill_place(const AttnArgs& a, const PrefillSplit& sp, uint32_t block,
+                                                      int thread) {
+    using Cfg = PrefillCfg<D>;
+    const int lane = thread & 63, wave = __builtin_amdgcn_readfirstlane(thread >> 6);
+    const uint32_t heads = static_cast<uint32_t>(a.heads);
+    uint32_t bh = block, chunk = 0, qt = sp.qtiles - 1;
+    if (sp.nchunks > 1) {
+        bh = block / sp.nchunks;
+        chunk = block - bh * sp.nchunks;
     }
-    uint64_t q_lo = 0, q_hi = 0;
-    if (q_live) key_range(a, a.offset + q, &q_lo, &q_hi);
-
-    // Key range of the whole workgroup and of this wave (for skipping tiles),
-    // and the keys every live query of the wave admits (tiles inside need no mask).
-    const uint64_t q_last = min(a.seq, q_first + Cfg::kBQ) - 1;
-    uint64_t blk_lo, blk_hi, tmp;
-    key_range(a, a.offset + q_first, &blk_lo, &tmp);
-    key_range(a, a.offset + q_last, &tmp, &blk_hi);
-    const uint64_t w_first = q_first + wave * 32;
-    const uint64_t w_last = min(a.seq, w_first + 32);
-    uint64_t wave_lo = 0, wave_hi = 0, all_lo = 0, all_hi = 0;
-    if (w_first < a.seq) {
-        key_range(a, a.offset + w_first, &wave_lo, &all_hi);
-        key_range(a, a.offset + w_last - 1, &all_lo, &wave_hi);
+    if (sp.qtiles > 1) {
+        const uint32_t back = bh / sp.pairs;
+        bh -= back * sp.pairs;
+        qt -= back;
     }
-    const uint64_t tile_begin = blk_lo / Cfg::kBKV * Cfg::kBKV;
-    const int ntiles = blk_hi > tile_begin
-                           ? static_cast<int>((blk_hi - tile_begin + Cfg::kBKV - 1) / Cfg::kBKV)
-                           : 0;
-    auto wave_in = [&](uint64_t k0) { return k0 < wave_hi && k0 + Cfg::kBKV > wave_lo; };
-    // This query's admitted keys relative to the first tile (32-bit: the
-    // caller keeps key counts below 2^31).
-    const int rel_lo = static_cast<int>(q_lo > tile_begin ? q_lo - tile_begin : 0);
-    const int rel_hi = static_cast<int>(q_hi > tile_begin ? q_hi - tile_begin : 0);
+    const uint32_t b = sp.pairs == heads ? 0 : bh / heads;
+    const uint32_t head = bh - b * heads;
+    const uint32_t kvh = sp.group == 1 ? head : head / sp.group;
+    PrefillPlace w{};
+    w.K = a.k + b * a.k_bs + static_cast<uint64_t>(kvh) * D;
+    w.V = a.v + b * a.v_bs + static_cast<uint64_t>(kvh) * D;
+    const int seq = static_cast<int>(a.seq), q_first = static_cast<int>(qt * Cfg::kBQ);
+    const int w_first = q_first + wave * 32, q = w_first + (lane & 31);
+    const uint64_t at = static_cast<uint64_t>(q) * (a.heads * D) + static_cast<uint64_t>(head) * D;
+    w.qrow = a.q + b * a.q_bs + at;
+    w.out = a.out + b * a.o_bs + at;
+    if (sp.nchunks > 1) {
+        const uint64_t rec = ((b * a.seq + q) * a.heads + head) * sp.nchunks + chunk;
+        w.out = sp.part_o + rec * D;
+        w.ml = sp.part_ml + 2 * rec;
+    }
+    w.q_live = q < seq;
 
-    float m = -INFINITY, l = 0.0f;
-    v16f o[VD / 32];
+    const int kv_seq = static_cast<int>(a.kv_seq), offset = static_cast<int>(a.offset);
+    const int back = a.window < 0 ? kv_seq : static_cast<int>(a.window < kv_seq ? a.window : kv_seq) - 1;
+    auto first = [&](int i) { return max(offset + i - max(back, 0), 0); };
+    auto past = [&](int i) { return a.causal ? offset + i + 1 : kv_seq; };
+    const int tile_begin = first(q_first) / Cfg::kBKV * Cfg::kBKV;
+    const int ntiles = (past(min(seq, q_first + Cfg::kBQ) - 1) - tile_begin + Cfg::kBKV - 1) / Cfg::kBKV;
+    w.tile_begin = tile_begin;
+    // All of the ntiles from tile_begin, or the part inside the key chunk.
+    w.i_end = ntiles;
+    if (sp.nchunks > 1) {
+        const int c0 = static_cast<int>(chunk * sp.chunk_tiles) - tile_begin / Cfg::kBKV;
+        w.i_begin = min(max(c0, 0), ntiles);
+        w.i_end = min(max(c0 + static_cast<int>(sp.chunk_tiles), 0), ntiles);
+    }
+    if (w.q_live) {
+        w.lo = first(q) - tile_begin;
+        w.hi = past(q) - tile_begin;
+    }
+    if (w_first < seq) {
+        const int w_last = min(seq, w_first + 32) - 1;
+        w.any_lo = first(w_first) - tile_begin;
+        w.all_hi = past(w_first) - tile_begin;
+        w.all_lo = first(w_last) - tile_begin;
+        w.any_hi = past(w_last) - tile_begin;
+    }
+    return w;
+}
+
+// One tile's masked scores: s[r] is key k0 + 8 (r / 4) + 4 half + r % 4 of the
+// lane's query, -inf where it is not admitted (rel_lo, rel_hi: its admitted
+// keys from the tile's first).
+__device__ __forceinline__ void mask_scores(v16f& s, int rel_lo, int rel_hi, int half) {
+    const int lo = min(max(rel_lo, 0), 32), hi = min(max(rel_hi, 0), 32);
+    const uint32_t mine = static_cast<uint32_t>(((1ull << hi) - 1ull) & ~((1ull << lo) - 1ull)) >> (4 * half);
 #pragma unroll
-    for (int vb = 0; vb < VD / 32; ++vb)
+    for (int r = 0; r < 16; ++r) {
+        const int key = 8 * (r / 4) + (r % 4);
+        s[r] = (mine >> key) & 1u ? s[r] : -INFINITY;
+    }
+}
+
+// The online softmax over one tile: s becomes the tile's weights 2^(s - m),
+// and the sums so far are to be scaled by the result. The reference m moves
+// only to a maximum more than 8 above it (weights reach 2^8), so that after the
+// first tiles the result is 1 for every query and nothing is scaled. Every
+// lane runs it (the MFMAs need the whole wave); a query with no admitted key
+// yet keeps m = -inf, l = 0.
+__device__ __forceinline__ float softmax_tile(v16f& s, float& m, float& l) {
+    float tile_max = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) tile_max = fmaxf(tile_max, s[r]);
+    tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, 64));
+    const float m_new = tile_max > m + 8.0f ? tile_max : m;
+    const float alpha = m_new == m ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);
+    const float base = m_new == -INFINITY ? 0.0f : m_new;
+    float psum = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        s[r] = __builtin_amdgcn_exp2f(s[r] - base);
+        psum += s[r];
+    }
+    l = l * alpha + (psum + __shfl_xor(psum, 32, 64));
+    m = m_new;
+    return alpha;
+}
+
+// The same with s the tile's probabilities over the sum so far: the output so
+// far, scaled by the result, stays a convex combination of V rows.
+__device__ __forceinline__ float softmax_tile_mean(v16f& s, float& m, float& l) {
+    const float m_old = m, l_old = l;
+    const float alpha = softmax_tile(s, m, l);
+    const float inv = l > 0.0f ? __builtin_amdgcn_rcpf(l) : 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] *= inv;
+    // A tile that adds nothing for this query leaves its output as it was.
+    return (l == l_old && m == m_old) || l == 0.0f ? 1.0f : (l_old * alpha) * inv;
+}
+
+// The workgroup's tiles [i_begin, i_end) with the f32 MFMA, for the waves
+// (`again`) that met inputs outside the bf16 split: values that are not
+// finite, scores' operands above 2^60, scaled values below 2^-100. Q is read
+// from memory, K and V tiles lie in LDS; a key that one query masks and another
+// admits enters P . V at weight 0, so a wave that met a V value that is not
+// finite in an edge tile sums its queries' admitted keys again on the VALU
+// (recompute_admitted).
+template <int D>
+__device__ __forceinline__ void prefill_f32(const AttnArgs& a, const PrefillPlace& w, int thread, bool again,
+                                            float* lds, v16f (&o)[PrefillCfg<D>::kVB], float& m, float& l) {
+    using Cfg = PrefillCfg<D>;
+    const int lane = thread & 63, l32 = lane & 31, half = lane >> 5;
+    const uint64_t kv_ld = a.kv_heads * D;
+    const float* const qhalf = w.qrow + half * (D / 2);
+    m = -INFINITY;
+    l = 0.0f;
+#pragma unroll
+    for (int vb = 0; vb < Cfg::kVB; ++vb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[vb][r] = 0.0f;
-
-    float* const kbuf0 = lds;
-    float* const vbuf0 = lds + 2 * Cfg::kKTile;
-    auto kbuf = [&](int i) { return kbuf0 + (i & 1) * Cfg::kKTile; };
-    auto vbuf = [&](int i) { return vbuf0 + (i & 1) * Cfg::kVTile; };
-    const TileDma<D> kdma(k_ld, wave, lane);
-    const TileDma<VD> vdma(v_ld, wave, lane);
-    auto load_k = [&](uint64_t k0, float* dst) { kdma.load(K, k_ld, k0, a.kv_seq, dst, wave, lane); };
-    auto load_v = [&](uint64_t k0, float* dst) { vdma.load(V, v_ld, k0, a.kv_seq, dst, wave, lane); };
-
-    // V reads: key row `key`, column vb*32 + l32 sits in chunk
-    // (vb*8 + l32/4) ^ (key & 15), and key & 15 = 8*((t/4) & 1) + 4*half +
-    // t%4 for step t: block vb ^ ((t/4) & 1), chunk (l32/4) ^ (4*half + t%4).
-    int vx[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) vx[j] = (((l32 >> 2) ^ (4 * half + j)) << 2) + (l32 & 3);
-
-    // This workgroup's tiles [i_begin, i_end) of the ntiles from tile_begin:
-    // all of them, or the part inside its key chunk.
-    int i_begin = 0, i_end = ntiles;
-    if (sp.nchunks > 1) {
-        const int64_t first = static_cast<int64_t>(tile_begin / Cfg::kBKV);
-        const int64_t c0 = static_cast<int64_t>(chunk) * sp.chunk_tiles - first;
-        i_begin = static_cast<int>(min<int64_t>(max<int64_t>(c0, 0), ntiles));
-        i_end = static_cast<int>(min<int64_t>(max<int64_t>(c0 + sp.chunk_tiles, 0), ntiles));
-    }
-
-    // The j-th tile walked sits in buffer j & 1 (K and V); the next one is
-    // loaded straight into the other buffer while it is used (that buffer
-    // held the previous tile, whose readers all passed the previous barrier).
-    bool redo = false;  // an edge tile of this wave held a non-finite V value
-    if (i_end > i_begin) {
-        load_k(tile_begin + static_cast<uint64_t>(i_begin) * Cfg::kBKV, kbuf(0));
-        load_v(tile_begin + static_cast<uint64_t>(i_begin) * Cfg::kBKV, vbuf(0));
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    for (int i = i_begin; i < i_end; ++i) {
-        const int j = i - i_begin;
-        const int cur = j & 1;
-        const uint64_t k0 = tile_begin + static_cast<uint64_t>(i) * Cfg::kBKV;
-        if (i + 1 < i_end) {
-            load_k(k0 + Cfg::kBKV, kbuf(cur ^ 1));
-            load_v(k0 + Cfg::kBKV, vbuf(cur ^ 1));
+    float* const sk = lds;
+    float* const sv = lds + Cfg::kBKV * Cfg::kLdF;
+    bool redo = false;
+    for (int i = w.i_begin; i < w.i_end; ++i) {
+        const uint64_t k0 = w.tile_begin + static_cast<uint64_t>(i) * Cfg::kBKV;
+        for (int f = thread; f < Cfg::kBKV * D / 4; f += Cfg::kThreads) {
+            const int row = f / (D / 4), c = f % (D / 4) * 4;
+            const uint64_t key = min(k0 + row, a.kv_seq - 1);
+            *reinterpret_cast<float4*>(sk + row * Cfg::kLdF + c) = *reinterpret_cast<const float4*>(w.K + key * kv_ld + c);
+            *reinterpret_cast<float4*>(sv + row * Cfg::kLdF + c) = *reinterpret_cast<const float4*>(w.V + key * kv_ld + c);
         }
-        if (wave_in(k0)) {
-            // A tile every query of the wave admits whole needs no mask.
-            const bool masked = !(k0 >= all_lo && k0 + Cfg::kBKV <= all_hi);
-            const float* sv = vbuf(cur);
-            // An edge tile checks its V for non-finite values (integer steps:
-            // an all-ones exponent gives e + 1 = 256, so (e + 1) >> 8 is 1; no
-            // compare masks to hold; four reads in flight), before the scores
-            // while fewer registers are live. One found sends the wave to
-            // recompute_admitted after the loop.
+        __syncthreads();
+        const int rel = i * Cfg::kBKV;
+        if (again && rel < w.any_hi && rel + Cfg::kBKV > w.any_lo) {
+            const bool masked = !(rel >= w.all_lo && rel + Cfg::kBKV <= w.all_hi);
             if (masked) {
                 uint32_t nonfinite = 0;
-                const mhip::f32x4* tile4 = reinterpret_cast<const mhip::f32x4*>(sv);
-#pragma unroll
-                for (int j = 0; j < Cfg::kVTile / 4 / 64; ++j) {
-                    const mhip::f32x4 v4 = tile4[j * 64 + lane];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        nonfinite |= (((__float_as_uint(v4[e]) >> 23) & 0xFFu) + 1u) >> 8;
-                    if ((j & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+                for (int f = lane; f < Cfg::kBKV * D; f += 64) {
+                    const float v = sv[f / D * Cfg::kLdF + f % D];
+                    nonfinite |= (((__float_as_uint(v) >> 23) & 0xFFu) + 1u) >> 8;
                 }
                 redo |= __builtin_amdgcn_ballot_w64(nonfinite != 0) != 0;
             }
-            v16f s_cur = tile_scores<D>(kbuf(cur), qf, l32, half);
-            // Register r holds key k0 + 8*(r/4) + 4*half + r%4 of query q; bit
-            // j of `span` says whether tile key j is admitted.
-            if (masked) {
-                const int lo_r = min(max(rel_lo - i * Cfg::kBKV, 0), Cfg::kBKV);
-                const int hi_r = min(max(rel_hi - i * Cfg::kBKV, 0), Cfg::kBKV);
-                const uint64_t span = ((1ull << hi_r) - 1ull) & ~((1ull << lo_r) - 1ull);
-                const uint32_t mine = static_cast<uint32_t>(span) >> (4 * half);
+            v16f s;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int key = 8 * (r / 4) + (r % 4);
-                    s_cur[r] = (mine >> key) & 1u ? s_cur[r] : -INFINITY;
-                }
+            for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+#pragma unroll 1
+            for (int t = 0; t < D / 2; t += 4) {
+                float4 v4 = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (w.q_live) v4 = *reinterpret_cast<const float4*>(qhalf + t);
+                const float q4[4] = {v4.x * a.qscale, v4.y * a.qscale, v4.z * a.qscale, v4.w * a.qscale};
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(sk[l32 * Cfg::kLdF + half * (D / 2) + t + e], q4[e], s, 0, 0, 0);
             }
-            float tile_max = -INFINITY;
+            if (masked) mask_scores(s, w.lo - rel, w.hi - rel, half);
+            const float keep = softmax_tile_mean(s, m, l);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) tile_max = fmaxf(tile_max, s_cur[r]);
-            tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, 64));
-            // Every lane runs the update (the MFMAs below need the whole wave);
-            // a query with no admitted key yet keeps m = -inf, l = 0, o = 0.
-            const float m_new = fmaxf(m, tile_max);
-            const float m_use = m_new == -INFINITY ? 0.0f : m_new;
-            const float alpha = __builtin_amdgcn_exp2f(m - m_use);
-            float psum = 0.0f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                s_cur[r] = __builtin_amdgcn_exp2f(s_cur[r] - m_use);
-                psum += s_cur[r];
-            }
-            psum += __shfl_xor(psum, 32, 64);
-            const float l_new = l * alpha + psum;
-            const float inv = l_new > 0.0f ? __builtin_amdgcn_rcpf(l_new) : 0.0f;
-            // A tile that adds nothing for this query leaves its output as it was.
-            const float keep = (psum == 0.0f && alpha == 1.0f) || l_new == 0.0f ? 1.0f : (l * alpha) * inv;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) s_cur[r] *= inv;
-#pragma unroll
-            for (int vb = 0; vb < VD / 32; ++vb) {
+            for (int vb = 0; vb < Cfg::kVB; ++vb) {
+                const int c = vb * 32 + l32;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) o[vb][r] *= keep;
-                // O^T += V^T . P^T: step t pairs key 8*(t/4) + 4*half + t%4 with register t.
 #pragma unroll
                 for (int t = 0; t < 16; ++t) {
-                    const int key_row = 8 * (t / 4) + 4 * half + (t % 4);
-                    const float v = sv[key_row * VD + (vb ^ ((t >> 2) & 1)) * 32 + vx[t % 4]];
-                    o[vb] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, s_cur[t], o[vb], 0, 0, 0);
+                    const int key = 8 * (t / 4) + 4 * half + (t % 4);
+                    const float v = D % 32 == 0 || c < D ? sv[key * Cfg::kLdF + c] : 0.0f;
+                    o[vb] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, s[t], o[vb], 0, 0, 0);
                 }
             }
-            m = m_new;
-            l = l_new;
         }
-        __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
     }
-
     if (redo) {
-        // This workgroup's keys (its tiles [i_begin, i_end)), the query's range within them.
-        const uint64_t c_lo = tile_begin + static_cast<uint64_t>(i_begin) * Cfg::kBKV;
-        const uint64_t c_hi = tile_begin + static_cast<uint64_t>(i_end) * Cfg::kBKV;
-        const uint64_t lo = max(q_lo, c_lo), hi = min(q_hi, c_hi);
-        recompute_admitted<D, VD>(qf, K, k_ld, V, v_ld, lo, hi > lo ? hi : lo, half, o, &m, &l);
+        const int lo = max(w.lo, w.i_begin * Cfg::kBKV), hi = min(w.hi, w.i_end * Cfg::kBKV);
+        recompute_admitted<D>(w.q_live ? qhalf : w.K, a.qscale, w.K, kv_ld, w.V, kv_ld,
+                              w.tile_begin + lo, w.tile_begin + max(lo, hi), half, o, &m, &l);
     }
+}
 
+// The range of operands as they are split (2 |x| as an integer, see kSplitTiny).
+struct SplitRange {
+    uint32_t big = 0, least = 0xFFFFFFFFu;
+    __device__ __forceinline__ void top(float x0, float x1) {
+        big = max(big, max(__float_as_uint(x0) << 1, __float_as_uint(x1) << 1));
+    }
+    __device__ __forceinline__ void bottom(float x0, float x1) { least = mhip::split_min(least, x0, x1); }
+};
+constexpr uint32_t kScoreTop = 2u * ((127u + 60u) << 23);   // 2^60
+constexpr uint32_t kValueTop = 2u * (254u << 23);           // (a scaled one is below 2^127 or not finite)
+
+// Flash attention of 256 queries of one (batch, head), eight waves of 32, on
+// the bf16 matrix cores: Q, K and V split exactly into three bf16 planes
+// (split_tile.hpp) and the probabilities too, six plane products a product.
+// Per tile of 32 keys a wave needs 96 MFMAs of 32 cycles (D 128) where the f32
+// MFMA needed 128 of 64.
+//
+// Q^T's planes live in registers, K's and V's in LDS, split once for the eight
+// waves. K is split row by row; V so that a lane's 8 keys of a step are the
+// ones whose scores the same half of the wave holds, so the probabilities feed
+// P . V from the registers they are computed in. Two barriers per tile: scores
+// and softmax while V is split into its buffer, then P . V while the next
+// tile's K is; both are loaded a tile ahead.
+//
+// Against the f32 MFMA kernel (four waves, 128 queries), causal, us: 4
+// sequences of 2048, 32 heads of 128, 1225 before and 837 now; one of 509 63
+// and 44; 1024 keys, 16 heads of 64, 4 sequences 172 and 139. Head dims 32, 80,
+// 96 and 112 ran on the generic kernel: 1024 keys, 32 heads of 80 5435 and 79.
+// Bound by the chain within a wave (scores, softmax, the split of the
+// probabilities, P . V) with two waves per SIMD to hide it: the registers of
+// Q's planes and the output allow no third.
+template <int D>
+__global__ __launch_bounds__(PrefillCfg<D>::kThreads, 2) void attn_prefill_kernel(AttnArgs a, PrefillSplit sp) {
+    apply_advance(a);
+    using Cfg = PrefillCfg<D>;
+    using mhip::bf16x8;
+    using mhip::u32x2;
+    using mhip::u32x4;
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    char* const lk = lds;
+    char* const lv = lds + 3 * Cfg::kKPlane;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    char* const lq = lv + 3 * Cfg::kVPlane + wave * Cfg::kSteps * 1024 + lane * 16;
+    const int l32 = lane & 31, half = lane >> 5;
+
+    const PrefillPlace w = prefill_place<D>(a, sp, blockIdx.x, threadIdx.x);
+    const float *const K = w.K, *const V = w.V, *const qrow = w.qrow;
+    const uint64_t kv_ld = a.kv_heads * D, tile_begin = w.tile_begin;
+    const int i_begin = w.i_begin, i_end = w.i_end;
+    float m = -INFINITY, l = 0.0f;
+    v16f o[Cfg::kVB];
+#pragma unroll
+    for (int vb = 0; vb < Cfg::kVB; ++vb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[vb][r] = 0.0f;
+    // A tile's loads: K, 4 of d of one key per unit; V, 8 keys of one column
+    // (the chunk of a pair of waves). Buffer loads whose range ends with the
+    // last key: keys past it read as zeros, which the mask takes out.
+    u32x4 kr[Cfg::kKUnits];
+    uint32_t vr[8];
+    const int v_chunk = wave >> 1;  // step v_chunk / 2, half v_chunk % 2
+    const int v_col = (wave & 1) * 64 + lane;
+    const bool v_on = v_col < Cfg::kVB * 32;
+    const bool v_in = v_col < D;
+    const uint32_t ld_bytes = static_cast<uint32_t>(kv_ld * sizeof(float));  // the launch checks 32 rows < 2^31
+    uint32_t k_off[Cfg::kKUnits];
+#pragma unroll
+    for (int u = 0; u < Cfg::kKUnits; ++u) {
+        const int f = min(static_cast<int>(threadIdx.x) + u * Cfg::kThreads, Cfg::kBKV * D / 4 - 1);
+        k_off[u] = f / (D / 4) * ld_bytes + f % (D / 4) * 16;
+    }
+    const uint32_t v_off = min(v_col, D - 1) * 4;
+    auto tile_rsrc = [&](const float* base, int i) {
+        const uint64_t k0 = tile_begin + static_cast<uint64_t>(i) * Cfg::kBKV;
+        const uint64_t bytes = ((a.kv_seq - 1 - k0) * kv_ld + D) * sizeof(float);
+        return __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float*>(base + k0 * kv_ld), 0,
+            static_cast<int>(static_cast<uint32_t>(bytes < 0xFFFFFFFFu ? bytes : 0xFFFFFFFFu)), 0x00020000);
+    };
+    auto load_k = [&](int i) {
+        const __amdgpu_buffer_rsrc_t rsrc = tile_rsrc(K, i);
+#pragma unroll
+        for (int u = 0; u < Cfg::kKUnits; ++u) kr[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, k_off[u], 0, 0);
+    };
+    auto load_v = [&](int i) {
+        const __amdgpu_buffer_rsrc_t rsrc = tile_rsrc(V, i);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            vr[e] = __builtin_amdgcn_raw_buffer_load_b32(
+                rsrc, v_off, (16 * (v_chunk >> 1) + 4 * (v_chunk & 1) + (e / 4) * 8 + e % 4) * ld_bytes, 0);
+    };
+    if (i_end > i_begin) {
+        load_k(i_begin);
+        load_v(i_begin);
+    }
+    SplitRange query;
+    // Whether a tile (by parity) holds K or V outside the split.
+    __shared__ int outside[2];
+    if (threadIdx.x < 2) outside[threadIdx.x] = 0;
+
+    // Q^T's planes, pre-scaled: step t, k = 16 t + 8 half + i of the query.
+    constexpr int kQRegs = Cfg::kQLds ? 2 : 3;
+    u32x4 qp[Cfg::kSteps][kQRegs];
+#pragma unroll
+    for (int t = 0; t < Cfg::kSteps; ++t) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; e += 4) {
+            float4 v4 = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (w.q_live) v4 = *reinterpret_cast<const float4*>(qrow + 16 * t + 8 * half + e);
+            x[e] = v4.x * a.qscale; x[e + 1] = v4.y * a.qscale; x[e + 2] = v4.z * a.qscale; x[e + 3] = v4.w * a.qscale;
+        }
+        u32x4 third;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            uint32_t p[3];
+            mhip::split_pair(x[2 * e], x[2 * e + 1], p);
+            query.top(x[2 * e], x[2 * e + 1]);
+            qp[t][0][e] = p[0];
+            qp[t][1][e] = p[1];
+            third[e] = p[2];
+        }
+        if constexpr (Cfg::kQLds) *reinterpret_cast<u32x4*>(lq + t * 1024) = third;
+        else qp[t][kQRegs - 1] = third;
+    }
+    // Whether the wave met operands outside the split (decided here for Q, or
+    // its values would be kept until the end).
+    bool again = __builtin_amdgcn_ballot_w64(query.big > kScoreTop) != 0;
+
+    auto store_k = [&](int i) {
+        SplitRange score;
+#pragma unroll
+        for (int u = 0; u < Cfg::kKUnits; ++u) {
+            const int f = threadIdx.x + u * Cfg::kThreads;
+            if (Cfg::kKUnits * Cfg::kThreads != Cfg::kBKV * D / 4 && f >= Cfg::kBKV * D / 4) continue;
+            const int row = f / (D / 4), c = f % (D / 4);
+            uint32_t p0[3], p1[3];
+            float x[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = __uint_as_float(kr[u][e]);
+            mhip::split_pair(x[0], x[1], p0);
+            mhip::split_pair(x[2], x[3], p1);
+            score.top(x[0], x[1]);
+            score.top(x[2], x[3]);
+            char* at = lk + c / 2 * Cfg::kKChunk + row * 16 + c % 2 * 8;
+#pragma unroll
+            for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x2*>(at + p * Cfg::kKPlane) = u32x2{p0[p], p1[p]};
+        }
+        if (score.big > kScoreTop) outside[i & 1] = 1;
+    };
+    // V is scaled by a power of two that keeps any sum of 2^8 kv_seq weighted
+    // rows finite, and the output by its inverse.
+    const int v_shift = 9 + 64 - __builtin_clzll(a.kv_seq);
+    const float v_scale = v_in ? __uint_as_float(static_cast<uint32_t>(127 - v_shift) << 23) : 0.0f;
+    auto store_v = [&](int i) {
+        if (!v_on) return;
+        SplitRange value;
+        u32x4 p[3];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float x0 = __uint_as_float(vr[2 * e]) * v_scale, x1 = __uint_as_float(vr[2 * e + 1]) * v_scale;
+            uint32_t q[3];
+            mhip::split_pair(x0, x1, q);
+            value.top(x0, x1);
+            value.bottom(x0, x1);
+            p[0][e] = q[0];
+            p[1][e] = q[1];
+            p[2][e] = q[2];
+        }
+        char* at = lv + v_chunk * Cfg::kVChunk + v_col * 16;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4*>(at + q * Cfg::kVPlane) = p[q];
+        if (value.big > kValueTop || value.least < mhip::kSplitTiny) outside[i & 1] = 1;
+    };
+    auto mfma = [](bf16x8 x, bf16x8 y, v16f c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, c, 0, 0, 0); };
+    auto as_bf16 = [](u32x4 v) { return __builtin_bit_cast(bf16x8, v); };
+
+    if (i_end > i_begin) {
+        __syncthreads();
+        store_k(i_begin);
+        if (i_begin + 1 < i_end) load_k(i_begin + 1);
+        mhip::lds_barrier<0>();
+        for (int i = i_begin; i < i_end; ++i) {
+            const int rel = i * Cfg::kBKV;  // the tile's first key, from tile_begin
+            const bool mine = rel < w.any_hi && rel + Cfg::kBKV > w.any_lo;
+            auto next_v = [&]() {
+                store_v(i);
+                if (i + 1 < i_end) load_v(i + 1);
+            };
+            auto next_k = [&]() {
+                if (i + 1 < i_end) store_k(i + 1);
+                if (i + 2 < i_end) load_k(i + 2);
+            };
+            // (Read last in the tile before, set next after this tile's barrier.)
+            if (threadIdx.x == 0) outside[(i + 1) & 1] = 0;
+            v16f s;
+            u32x4 pp[2][3];  // the probabilities' planes: step, plane
+            float alpha = 1.0f;
+            if (mine) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+#pragma unroll
+                for (int t = 0; t < Cfg::kSteps; ++t) {
+                    if (t == Cfg::kSteps / 2) next_v();
+                    bf16x8 kf[3];
+#pragma unroll
+                    for (int p = 0; p < 3; ++p)
+                        kf[p] = *reinterpret_cast<const bf16x8*>(lk + p * Cfg::kKPlane + (2 * t + half) * Cfg::kKChunk + l32 * 16);
+                    u32x4 q3;
+                    if constexpr (Cfg::kQLds) q3 = *reinterpret_cast<const u32x4*>(lq + t * 1024);
+                    else q3 = qp[t][kQRegs - 1];
+                    s = mfma(kf[0], as_bf16(q3), s);
+                    s = mfma(kf[2], as_bf16(qp[t][0]), s);
+                    s = mfma(kf[1], as_bf16(qp[t][1]), s);
+                    s = mfma(kf[0], as_bf16(qp[t][1]), s);
+                    s = mfma(kf[1], as_bf16(qp[t][0]), s);
+                    s = mfma(kf[0], as_bf16(qp[t][0]), s);
+                }
+                // A tile every query of the wave admits whole needs no mask.
+                if (!(rel >= w.all_lo && rel + Cfg::kBKV <= w.all_hi)) mask_scores(s, w.lo - rel, w.hi - rel, half);
+                alpha = softmax_tile(s, m, l);
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        uint32_t p[3];
+                        mhip::split_pair(s[8 * t + 2 * e], s[8 * t + 2 * e + 1], p);
+                        pp[t][0][e] = p[0];
+                        pp[t][1][e] = p[1];
+                        pp[t][2][e] = p[2];
+                    }
+            } else {
+                next_v();
+            }
+            mhip::lds_barrier<0>();
+            if (mine) {
+                again |= outside[i & 1] != 0;
+                if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
+#pragma unroll
+                    for (int vb = 0; vb < Cfg::kVB; ++vb)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) o[vb][r] *= alpha;
+                }
+#pragma unroll
+                for (int vb = 0; vb < Cfg::kVB; ++vb) {
+                    if (vb == Cfg::kVB / 2) next_k();
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        bf16x8 vf[3];
+#pragma unroll
+                        for (int p = 0; p < 3; ++p)
+                            vf[p] = *reinterpret_cast<const bf16x8*>(lv + p * Cfg::kVPlane + (2 * t + half) * Cfg::kVChunk +
+                                                                     (vb * 32 + l32) * 16);
+                        o[vb] = mfma(vf[0], as_bf16(pp[t][2]), o[vb]);
+                        o[vb] = mfma(vf[2], as_bf16(pp[t][0]), o[vb]);
+                        o[vb] = mfma(vf[1], as_bf16(pp[t][1]), o[vb]);
+                        o[vb] = mfma(vf[0], as_bf16(pp[t][1]), o[vb]);
+                        o[vb] = mfma(vf[1], as_bf16(pp[t][0]), o[vb]);
+                        o[vb] = mfma(vf[0], as_bf16(pp[t][0]), o[vb]);
+                    }
+                }
+            } else {
+                next_k();
+            }
+            mhip::lds_barrier<0>();
+        }
+    }
+    const float inv = l > 0.0f ? 1.0f / l * __uint_as_float(static_cast<uint32_t>(127 + v_shift) << 23) : 0.0f;
+#pragma unroll
+    for (int vb = 0; vb < Cfg::kVB; ++vb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[vb][r] *= inv;
+    // The thread's place once more from the kernel's arguments where the
+    // registers are short, so that none of it is kept through the loop.
+    uint32_t block = blockIdx.x;
+    int thread = threadIdx.x;
+    if constexpr (D > 64) __asm__ volatile("" : "+s"(block), "+v"(thread));
+    const PrefillPlace end = prefill_place<D>(a, sp, block, thread);
     // Register r of block vb holds O[q][vb*32 + 8*(r/4) + 4*half + r%4].
-    if (q_live && sp.nchunks > 1) {
-        const uint64_t rec = ((b * a.seq + q) * a.heads + head) * sp.nchunks + chunk;
-        float* po = sp.part_o + rec * VD;
+    auto store = [&]() {
+        if (!end.q_live) return;
+        const int first = 4 * (thread >> 5 & 1);
+        if (end.ml && first == 0) *reinterpret_cast<float2*>(end.ml) = make_float2(m, l);
 #pragma unroll
-        for (int vb = 0; vb < VD / 32; ++vb)
+        for (int vb = 0; vb < Cfg::kVB; ++vb)
 #pragma unroll
-            for (int g = 0; g < 4; ++g)
-                *reinterpret_cast<float4*>(po + vb * 32 + 8 * g + 4 * half) =
+            for (int g = 0; g < 4; ++g) {
+                const int c = vb * 32 + 8 * g + first;
+                if (D % 32 != 0 && c >= D) continue;
+                *reinterpret_cast<float4*>(end.out + c) =
                     make_float4(o[vb][4 * g], o[vb][4 * g + 1], o[vb][4 * g + 2], o[vb][4 * g + 3]);
-        if (half == 0) *reinterpret_cast<float2*>(sp.part_ml + 2 * rec) = make_float2(m, l);
-    } else if (q_live) {
-        float* orow = O + q * o_ld;
-#pragma unroll
-        for (int vb = 0; vb < VD / 32; ++vb)
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-                *reinterpret_cast<float4*>(orow + vb * 32 + 8 * g + 4 * half) =
-                    make_float4(o[vb][4 * g], o[vb][4 * g + 1], o[vb][4 * g + 2], o[vb][4 * g + 3]);
+            }
+    };
+    again = __builtin_amdgcn_ballot_w64(again) != 0;
+    if (!again) store();
+    if (__syncthreads_or(again)) {
+        prefill_f32<D>(a, end, thread, again, reinterpret_cast<float*>(lds), o, m, l);
+        if (again) store();
     }
 }
 
@@ -514,7 +734,7 @@ __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(AttnArgs a, u
     constexpr int kItems = 256 / kLanes;
     const uint64_t item = static_cast<uint64_t>(blockIdx.x) * kItems + threadIdx.x / kLanes;
     const int t = threadIdx.x % kLanes;
-    if (item >= rows * a.heads) return;
+    if (item >= rows * a.heads || threadIdx.x >= kItems * kLanes) return;
     const uint64_t row = item / a.heads, head = item % a.heads;
     const uint64_t b = row / a.seq, q = row % a.seq;
     const float* ml = sp.part_ml + 2 * item * sp.nchunks;
@@ -539,17 +759,17 @@ __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(AttnArgs a, u
     *reinterpret_cast<float4*>(a.out + b * a.o_bs + q * (a.heads * VD) + head * VD + 4 * t) = acc;
 }
 
-// Key chunks for a prefill whose query tiles (per sequence) fill under the
-// device's resident slots (two workgroups per CU): enough chunks of at
-// least 4 key tiles to fill them, at most 16.
-void prefill_split(const mhip_ctx* ctx, const AttnArgs& a, uint64_t qtiles, uint64_t kbkv,
+// Key chunks for a prefill whose query tiles (per sequence) do not give every
+// CU its workgroup: enough chunks of at least 4 key tiles to do so, at most 16.
+void prefill_split(const mhip_ctx* ctx, const AttnArgs& a, bool replayable, uint64_t qtiles, uint64_t kbkv,
                    uint32_t* nchunks, uint32_t* chunk_tiles) {
     *nchunks = 1;
     *chunk_tiles = 0;
     // A replayed key count may pass the captured one: chunks sized here from
-    // the captured count would leave the later keys to no workgroup.
-    if (a.advance) return;
-    const uint64_t slots = 2 * static_cast<uint64_t>(ctx->compute_units ? ctx->compute_units : 256);
+    // the captured count would leave the later keys to no workgroup. The call
+    // outside a capture sums the same way, so that a replay gives its bits.
+    if (replayable) return;
+    const uint64_t slots = ctx->compute_units ? ctx->compute_units : 256;
     const uint64_t per_sequence = a.heads * qtiles;
     const uint64_t kv_tiles = (a.kv_seq + kbkv - 1) / kbkv;
     if (per_sequence >= slots || kv_tiles < 8) return;
@@ -561,37 +781,45 @@ void prefill_split(const mhip_ctx* ctx, const AttnArgs& a, uint64_t qtiles, uint
     *nchunks = static_cast<uint32_t>((kv_tiles + per - 1) / per);
 }
 
-template <int D, int VD>
-mhip_status launch_prefill(mhip_ctx* ctx, const AttnArgs& a, uint64_t batch) {
-    using Cfg = PrefillCfg<D, VD>;
+template <int D>
+mhip_status launch_prefill(mhip_ctx* ctx, const AttnArgs& a, uint64_t batch, bool replayable) {
+    using Cfg = PrefillCfg<D>;
     const uint64_t qtiles = (a.seq + Cfg::kBQ - 1) / Cfg::kBQ;
     PrefillSplit sp{};
-    prefill_split(ctx, a, qtiles, Cfg::kBKV, &sp.nchunks, &sp.chunk_tiles);
+    prefill_split(ctx, a, replayable, qtiles, Cfg::kBKV, &sp.nchunks, &sp.chunk_tiles);
+    // A capture's workspace does not grow, which refuses it chunks. Head
+    // dimensions that need none on the generic kernel go without.
+    if (D != 64 && D != 128 && sp.nchunks > 1 &&
+        mhip::workspace_short(ctx, batch * a.seq * a.heads * sp.nchunks * (D + 2) * sizeof(float)))
+        sp.nchunks = 1;
     const uint64_t blocks = batch * a.heads * qtiles * sp.nchunks;
     if (blocks >= (1ULL << 31)) return mhip::fail(MHIP_SHAPE_UNSUPPORTED, "attention: too many query tiles");
+    sp.qtiles = static_cast<uint32_t>(qtiles);
+    sp.pairs = static_cast<uint32_t>(batch * a.heads);
+    sp.group = static_cast<uint32_t>(a.heads / a.kv_heads);
     const uint64_t rows = batch * a.seq;
     if (sp.nchunks > 1) {
         const uint64_t records = rows * a.heads * sp.nchunks;
         float* part = nullptr;
-        mhip_status st = attention_workspace(ctx, records * (VD + 2) * sizeof(float), &part);
+        mhip_status st = attention_workspace(ctx, records * (D + 2) * sizeof(float), &part);
         if (st != MHIP_OK) return st;
         sp.part_o = part;
-        sp.part_ml = part + records * VD;
+        sp.part_ml = part + records * D;
     }
-    const size_t lds = Cfg::kLdsFloats * sizeof(float);
+    const size_t lds = Cfg::kLdsBytes;
     static bool configured = false;
     if (!configured) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prefill_kernel<D, VD>),
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prefill_kernel<D>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
         configured = true;
     }
-    mhip::launch(ctx, (attn_prefill_kernel<D, VD>), dim3(static_cast<unsigned>(blocks)), dim3(256),
+    mhip::launch(ctx, (attn_prefill_kernel<D>), dim3(static_cast<unsigned>(blocks)), dim3(Cfg::kThreads),
                  lds, a, sp);
     mhip_status st = mhip::check_launch("attention (MFMA prefill)");
     if (st != MHIP_OK || sp.nchunks == 1) return st;
     const uint64_t items = rows * a.heads;
-    constexpr uint64_t kItems = 256 / (VD / 4);
-    mhip::launch(ctx, (attn_prefill_combine_kernel<VD>),
+    constexpr uint64_t kItems = 256 / (D / 4);
+    mhip::launch(ctx, (attn_prefill_combine_kernel<D>),
                  dim3(static_cast<unsigned>((items + kItems - 1) / kItems)), dim3(256), 0, a, rows,
                  sp);
     return mhip::check_launch("attention (prefill chunk merge)");
@@ -1081,9 +1309,19 @@ extern "C" mhip_status mhip_attention_f32(mhip_ctx* ctx, const float* q, const f
     }
     // The MFMA kernel's key arithmetic is 32-bit, and so are its byte
     // offsets within a 32-row K or V tile.
-    const bool small_keys = p->kv_rows < (1ULL << 31) && a.kv_heads * std::max(d, vd) < (1ULL << 25);
-    if (aligned && small_keys && vd == d && d == 128) return launch_prefill<128, 128>(ctx, a, batch);
-    if (aligned && small_keys && vd == d && d == 64) return launch_prefill<64, 64>(ctx, a, batch);
+    const bool small_keys = p->kv_rows < (1ULL << 31) - 512 && a.kv_heads * std::max(d, vd) < (1ULL << 24);
+    if (aligned && small_keys && vd == d && a.kv_seq > 0) {
+        const bool replayable = p->seq_len == 1 && p->bounded_key_count != 0;
+        switch (d) {
+            case 32: return launch_prefill<32>(ctx, a, batch, replayable);
+            case 64: return launch_prefill<64>(ctx, a, batch, replayable);
+            case 80: return launch_prefill<80>(ctx, a, batch, replayable);
+            case 96: return launch_prefill<96>(ctx, a, batch, replayable);
+            case 112: return launch_prefill<112>(ctx, a, batch, replayable);
+            case 128: return launch_prefill<128>(ctx, a, batch, replayable);
+            default: break;
+        }
+    }
     if (vd > 256) return mhip::fail(MHIP_SHAPE_UNSUPPORTED, "attention value dimension above 256");
     const uint64_t total = batch * p->seq_len * H;
     if (total / 4 >= (1ULL << 31)) return mhip::fail(MHIP_SHAPE_UNSUPPORTED, "attention: too many rows");

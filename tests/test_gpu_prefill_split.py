@@ -1,0 +1,138 @@
+"""GPU: prompt attention on the split bf16 matrix products at the edges of its
+tiles, head dimensions and operand ranges, replayed, and in a capture that has
+no room for its key chunks.
+
+Bound: a score is off by at most (d + 16) u |q| |k| scale (u = 2^-24: the f32
+sum of d products and the roundings of q's scaling, the split and the
+exponent), which moves every weight by that much relative to it and the output
+by twice the largest such error; the weighted mean itself adds (keys + 64) u.
+Both scale with the largest admitted |v| of the column.
+"""
+import numpy as np
+import pytest
+
+from conftest import bits
+
+pytestmark = pytest.mark.gpu
+
+U = 2.0 ** -24
+
+
+def inputs(seed, s, kv, h, hkv, d):
+    rng = np.random.default_rng(seed)
+    return [rng.standard_normal((r, c)).astype(np.float32) for r, c in ((s, h * d), (kv, hkv * d), (kv, hkv * d))]
+
+
+def attend(dev, q, k, v, s, kv, h, hkv, d, **kw):
+    from magnetar_hip import ops
+    p = ops.attention_params(s, kv, h, d, kv_head_count=hkv, **kw)
+    return ops.attention(dev, dev.upload(q), dev.upload(k), dev.upload(v), p).numpy()
+
+
+def check(got, q, k, v, s, kv, h, hkv, d, causal=False, window_size=None, rows=None):
+    """Every (row, head) against float64; rows: the ones with finite admitted values."""
+    pos, scale = np.arange(kv), 1.0 / np.sqrt(np.float64(d))
+    for i in range(s) if rows is None else rows:
+        at = kv - s + i
+        admitted = (pos <= at) if causal else np.full(kv, True)
+        if window_size:
+            admitted &= pos > at - window_size
+        for head in range(h):
+            g = head // (h // hkv)
+            Q = q[i, head * d:(head + 1) * d].astype(np.float64)
+            K = k[admitted, g * d:(g + 1) * d].astype(np.float64)
+            V = v[admitted, g * d:(g + 1) * d].astype(np.float64)
+            x = K @ Q * scale
+            w = np.exp(x - x.max())
+            want = (w / w.sum()) @ V
+            score_error = (d + 16) * U * (np.abs(K) @ np.abs(Q)).max() * scale
+            bound = (2 * score_error + (len(V) + 64) * U) * np.abs(V).max(axis=0)
+            err = np.abs(got[i, head * d:(head + 1) * d] - want)
+            assert np.all(err <= bound), (i, head, (err / bound).max())
+
+
+SHAPES = [  # s, kv, h, hkv, causal, window
+    (1, 1, 2, 1, True, None), (31, 31, 3, 3, True, None), (32, 33, 2, 2, False, None), (33, 64, 4, 2, True, 7),
+    (255, 300, 2, 1, True, None), (257, 257, 2, 2, True, 40), (5, 1030, 4, 2, True, None), (40, 700, 2, 2, True, 300)]
+
+
+@pytest.mark.parametrize("d", [32, 64, 80, 96, 112, 128])
+@pytest.mark.parametrize("s,kv,h,hkv,causal,window", SHAPES)
+def test_edges_of_tiles(dev, s, kv, h, hkv, causal, window, d):
+    q, k, v = inputs(s + d, s, kv, h, hkv, d)
+    got = attend(dev, q, k, v, s, kv, h, hkv, d, causal=causal, window_size=window)
+    check(got, q, k, v, s, kv, h, hkv, d, causal, window)
+
+
+@pytest.mark.parametrize("d", [32, 96, 128])
+def test_a_batch_is_its_sequences(dev, d):
+    from magnetar_hip import ops
+    s, kv, h = 70, 300, 4
+    q, k, v = inputs(d, 3 * s, 3 * kv, h, 2, d)
+    p = ops.attention_params(s, kv, h, d, kv_head_count=2, causal=True, batch=3)
+    got = ops.attention(dev, dev.upload(q), dev.upload(k), dev.upload(v), p).numpy()
+    for b in range(3):
+        rs, rk = slice(b * s, (b + 1) * s), slice(b * kv, (b + 1) * kv)
+        one = attend(dev, q[rs], k[rk], v[rk], s, kv, h, 2, d, causal=True)
+        assert np.array_equal(bits(got[rs]), bits(one))
+
+
+@pytest.mark.parametrize("d", [64, 80, 112, 128])
+@pytest.mark.parametrize("what", ["q 2^70", "k 2^65", "v 3e38", "v 1e-40", "v scale 1e-25", "one v 1e-30", "v inf"])
+def test_operands_outside_the_split(dev, d, what):
+    s, kv, h, hkv = 100, 300, 4, 2
+    q, k, v = inputs(d, s, kv, h, hkv, d)
+    rows = None
+    if what == "q 2^70":
+        q, k = q * np.float32(2.0 ** 70), k * np.float32(2.0 ** -70)
+    elif what == "k 2^65":
+        q, k = q * np.float32(2.0 ** -65), k * np.float32(2.0 ** 65)
+    elif what == "v 3e38":
+        v = np.sign(v) * np.float32(3e38)
+    elif what == "v 1e-40":
+        v[50:60] = 1e-40
+    elif what == "v scale 1e-25":
+        v *= np.float32(1e-25)
+    elif what == "one v 1e-30":
+        v[:, 3] = 1e-30
+    else:
+        v[210, 5] = np.inf  # first admitted by query 10, and 9 rows of its wave mask it
+        rows = range(10)
+    got = attend(dev, q, k, v, s, kv, h, hkv, d, causal=True)
+    check(got, q, k, v, s, kv, h, hkv, d, True, rows=rows)
+    if what == "v inf":
+        assert np.all(np.isinf(got[10:, 5]) & np.isinf(got[10:, d + 5])) and np.all(np.isfinite(got[:, :5]))
+
+
+@pytest.mark.parametrize("d", [80, 96, 128])
+def test_a_replayed_row_has_the_bits_of_the_call(dev, d):
+    from magnetar_hip import ops
+    from magnetar_hip.device import ADVANCE_KEY_COUNT
+    q, k, v = inputs(d, 1, 2000, 4, 2, d)
+    dq, dk, dv = dev.upload(q), dev.upload(k), dev.upload(v)
+    def call(keys, out=None):
+        p = ops.attention_params(1, 2000, 4, d, kv_head_count=2, causal=True, key_count=keys)
+        return ops.attention(dev, dq, dk, dv, p, out)
+    want = {keys: call(keys).numpy() for keys in (300, 301, 1999)}
+    out = dev.empty((1, 4 * d))
+    dev.capture_begin(ADVANCE_KEY_COUNT)
+    call(300, out)
+    graph = dev.capture_end()
+    for keys in (300, 1999, 301, 1999):
+        graph.launch(keys - 300)
+        assert np.array_equal(bits(out.numpy()), bits(want[keys]))
+
+
+def test_a_cold_capture_of_attention():
+    import magnetar_hip
+    from magnetar_hip import ops
+    q, k, v = inputs(1, 3, 2000, 4, 2, 96)
+    fresh = magnetar_hip.Device(0)
+    dq, dk, dv, out = fresh.upload(q), fresh.upload(k), fresh.upload(v), fresh.empty((3, 4 * 96))
+    p = ops.attention_params(3, 2000, 4, 96, kv_head_count=2, causal=True)
+    fresh.capture_begin(0)
+    ops.attention(fresh, dq, dk, dv, p, out)
+    graph = fresh.capture_end()
+    for _ in range(2):
+        graph.launch(0)
+        check(out.numpy(), q, k, v, 3, 2000, 4, 2, 96, True)
