@@ -836,17 +836,71 @@ constexpr int kMaxGroup = 8;  // query heads per workgroup; larger groups take s
 // a chunk is 32 KB of K plus 32 KB of V.
 // Calls whose default chunks give every CU 16 workgroups or more (many
 // batch rows or heads, long caches) take twice the steps: half the
-// workgroups and records (C4 decode, B8 KV 4096: 175 -> 171 us).
+// workgroups and records (B8 KV 4096, 32 heads on 32 KV heads: 175 -> 171 us;
+// on 8 57 -> 54 with twice the steps and 59 with more waves resident instead).
 __host__ __device__ constexpr int decode_steps(int d4) { return d4 >= 4 ? 8 : 2 * d4; }
 __host__ __device__ constexpr int decode_chunk(int d4, int steps) { return steps * 256 / d4; }
 __host__ __device__ constexpr int decode_chunk(int d4) { return decode_chunk(d4, decode_steps(d4)); }
 
+constexpr int log2_of(int n) { return n <= 1 ? 0 : 1 + log2_of(n / 2); }
+
+// A lane exchange of the VALU: quad_perm xor 1 and 2, row_half_mirror (l ^ 7),
+// row_mirror (l ^ 15), row_ror 4 and 8.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xF, 0xF, true));
+}
+
+// Lanes whose bit MASK (16 or 32) is clear get a of both sides, the others b.
+template <int MASK>
+__device__ __forceinline__ float swap_sum(float a, float b) {
+    const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
+    const auto r = MASK == 32 ? __builtin_amdgcn_permlane32_swap(ua, ub, false, false)
+                              : __builtin_amdgcn_permlane16_swap(ua, ub, false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// a summed over the lane and its partner in bit MASK where that bit is clear, b
+// where it is set. (The partner in bits 4 and 8 is the mirrored lane, which
+// differs in the lower bits too: they are summed over after it.)
+template <int MASK>
+__device__ __forceinline__ float deal(float a, float b, int lane) {
+    if constexpr (MASK >= 16) {
+        return swap_sum<MASK>(a, b);
+    } else {
+        constexpr int kCtrl = MASK == 8 ? 0x140 : MASK == 4 ? 0x141 : MASK == 2 ? 0x4E : 0xB1;
+        const bool upper = lane & MASK;
+        return (upper ? b : a) + dpp<kCtrl>(upper ? a : b);
+    }
+}
+
+// Sums x[0, NV) over the 2 MASK lanes of a group and deals the sums out: each
+// step halves the values a lane holds, its bit MASK choosing the half, until
+// one is left, which the further steps sum in every lane. NV values take NV - 1
+// exchanges and the remaining steps, where a butterfly a value takes NV log2.
+template <int MASK, int NV, int N>
+__device__ __forceinline__ void sum_dealt(float (&x)[N], int lane) {
+    if constexpr (MASK >= 1) {
+#pragma unroll
+        for (int i = 0; i < (NV + 1) / 2; ++i) x[i] = deal<MASK>(x[i], NV > 1 ? x[i + NV / 2] : x[i], lane);
+        sum_dealt<MASK / 2, (NV + 1) / 2>(x, lane);
+    }
+}
+
 // One workgroup per (batch, KV head, key chunk). Every thread issues all of
-// its K and V loads before any arithmetic (2 * kSteps dwordx4 in flight);
-// scores, the chunk max and the probabilities stay in registers, and only
-// the per-wave partial sums meet in LDS. Writes, per query head of the
-// group, the chunk's output normalised by its own weight sum, plus the
-// chunk max (log2 domain) and weight sum.
+// its K and V loads before any arithmetic (2 * kSteps dwordx4 in flight).
+// A wave's scores are summed and dealt out over the lanes (sum_dealt), so that
+// each of them is exponentiated once, and its probabilities return to the
+// lanes of their keys through LDS. A wave keeps its own maximum and weight
+// sum; the four meet at the end. Writes, per query head of the group, the
+// chunk's output normalised by its own weight sum, plus the chunk max (log2
+// domain) and weight sum.
+//
+// With five exchanges a head and key and every lane exponentiating every
+// score, grouped heads were bound by those, not by memory. One query over 4096
+// keys, 8 sequences, head dimension 128, us before and now: 32 heads on 8 KV
+// heads 68 and 54, on 4 68 and 40, on 32 175 and 172 (6.25 TB/s); 8192 keys of
+// one sequence, 32 on 8, 28 and 21; 16 heads of 64 on 2 25 and 17.
 template <int D4, int GT, int STEPS>
 __global__ __launch_bounds__(256) void attn_decode_partial_kernel(
     AttnArgs a, uint64_t key_base, uint64_t chunks, float* __restrict__ part_o,
@@ -856,8 +910,17 @@ __global__ __launch_bounds__(256) void attn_decode_partial_kernel(
     constexpr int kKPW = 4 * kKPS;        // keys per workgroup step
     constexpr int kSteps = STEPS;
     constexpr int D = 4 * D4;
+    // A wave's scores: N per lane, of which it ends with kLeft: those of kHeads
+    // heads and kKeys steps from value number `first`; 2^kCopies lanes hold the
+    // same ones.
+    constexpr int N = GT * kSteps;
+    constexpr int kDealt = log2_of(N < kLPK ? N : kLPK);
+    constexpr int kLeft = N >> kDealt, kCopies = log2_of(kLPK) - kDealt;
+    constexpr int kKeys = kLeft < kSteps ? kLeft : kSteps, kHeads = kLeft / kKeys;
+    constexpr int kRow = N + 4;  // (rows of a wave's subgroups in different banks)
     __shared__ float4 sq[GT][D4];
     __shared__ float4 red[4][GT][D4];
+    __shared__ float4 sp[4][kKPS][kRow / 4];
     __shared__ float wm[4][GT], wl[4][GT];
 
     // (batch, KV head) varies fastest: workgroups in flight together read
@@ -903,95 +966,146 @@ __global__ __launch_bounds__(256) void attn_decode_partial_kernel(
         }
     }
     const float* Qb = a.q + b * a.q_bs + head0 * D;
-    for (int i = threadIdx.x; i < group * D4; i += 256) {
-        float4 q4 = *reinterpret_cast<const float4*>(Qb + 4 * static_cast<uint64_t>(i));
+    for (int i = threadIdx.x; i < GT * D4; i += 256) {
+        float4 q4 = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (i < group * D4) q4 = *reinterpret_cast<const float4*>(Qb + 4 * static_cast<uint64_t>(i));
         q4.x *= a.qscale; q4.y *= a.qscale; q4.z *= a.qscale; q4.w *= a.qscale;
         sq[i / D4][i % D4] = q4;
     }
     __syncthreads();
 
-    // Scores (log2 domain) and the chunk max per head.
-    float s[GT][kSteps];
+    // Scores (log2 domain), the first step of the dealing as they come.
+    float s[N];
+    auto dot = [&](const float4& k4, const float4& q4) {
+        return k4.x * q4.x + k4.y * q4.y + k4.z * q4.z + k4.w * q4.w;
+    };
+    if constexpr (kLPK == 1) {
 #pragma unroll
-    for (int g = 0; g < GT; ++g) {
-        if (g >= group) break;
-        const float4 q4 = sq[g][sl];
+        for (int i = 0; i < N; ++i) s[i] = dot(kr[i % kSteps], sq[i / kSteps][0]);
+    } else {
+#pragma unroll
+        for (int g = 0; g < (GT + 1) / 2; ++g) {
+            const float4 q4 = sq[g][sl], other = sq[GT > 1 ? g + GT / 2 : g][sl];
+#pragma unroll
+            for (int u = 0; u < (GT > 1 ? kSteps : kSteps / 2); ++u)
+                s[g * kSteps + u] = deal<kLPK / 2>(dot(kr[u], q4), dot(kr[GT > 1 ? u : u + kSteps / 2], other), lane);
+        }
+        sum_dealt<kLPK / 4, N / 2>(s, lane);
+    }
+    const int first = (sl >> kCopies) * kLeft;
+
+    // The wave's maximum, probabilities and weight sum per head (heads past the
+    // group among them, unused).
+#pragma unroll
+    for (int g = 0; g < kHeads; ++g) {
+        float* const x = s + g * kKeys;
         float mx = -INFINITY;
 #pragma unroll
-        for (int u = 0; u < kSteps; ++u) {
-            float dot = kr[u].x * q4.x + kr[u].y * q4.y + kr[u].z * q4.z + kr[u].w * q4.w;
-#pragma unroll
-            for (int off = kLPK / 2; off >= 1; off >>= 1) dot += __shfl_xor(dot, off, 64);
-            const int j = u * kKPW + wave * kKPS + sub;
-            s[g][u] = j < n ? dot : -INFINITY;
-            mx = fmaxf(mx, s[g][u]);
+        for (int u = 0; u < kKeys; ++u) {
+            const int j = (first % kSteps + u) * kKPW + wave * kKPS + sub;
+            x[u] = j < n ? x[u] : -INFINITY;
+            mx = fmaxf(mx, x[u]);
         }
+        // Over the lanes that hold the head's other steps, then other keys.
+#pragma unroll
+        for (int off = 1 << kCopies; off < kSteps / kKeys << kCopies; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
 #pragma unroll
         for (int off = kLPK; off < 64; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-        if (lane == 0) wm[wave][g] = mx;
-    }
-    __syncthreads();
-
-    // Probabilities and the chunk's weight sum per head.
-#pragma unroll
-    for (int g = 0; g < GT; ++g) {
-        if (g >= group) break;
-        const float m = fmaxf(fmaxf(wm[0][g], wm[1][g]), fmaxf(wm[2][g], wm[3][g]));
         float l = 0.0f;
 #pragma unroll
-        for (int u = 0; u < kSteps; ++u) {
-            s[g][u] = m == -INFINITY ? 0.0f : exp2f(s[g][u] - m);
-            l += s[g][u];
+        for (int u = 0; u < kKeys; ++u) {
+            x[u] = x[u] == -INFINITY ? 0.0f : exp2f(x[u] - mx);
+            l += x[u];
         }
 #pragma unroll
+        for (int off = 1 << kCopies; off < kSteps / kKeys << kCopies; off <<= 1) l += __shfl_xor(l, off, 64);
+#pragma unroll
         for (int off = kLPK; off < 64; off <<= 1) l += __shfl_xor(l, off, 64);
-        if (lane == 0) wl[wave][g] = l;
+        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+#pragma unroll
+        for (int u = 0; u < kKeys; ++u) x[u] *= inv;
+        if (sub == 0 && (sl & ((1 << kCopies) - 1)) == 0 && first % kSteps == 0) {
+            wm[wave][first / kSteps + g] = mx;
+            wl[wave][first / kSteps + g] = l;
+        }
     }
-    __syncthreads();
+    if constexpr (kLPK > 1) {
+        float* const row = reinterpret_cast<float*>(sp[wave][sub]);
+        if ((sl & ((1 << kCopies) - 1)) == 0)
+#pragma unroll
+            for (int i = 0; i < kLeft; ++i) row[first + i] = s[i];
+        // The wave's own rows: its LDS operations are in order.
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
 
     // Weighted V rows with normalised probabilities: every partial sum is a
-    // convex combination of V rows, so none overflows.
+    // convex combination of V rows, so none overflows. The keys' lanes sum as
+    // above, and lane group `sub` of the first kParts stores its part of a float4.
+    constexpr int kParts = kKPS < 4 ? kKPS : 4;
 #pragma unroll
     for (int g = 0; g < GT; ++g) {
         if (g >= group) break;
-        const float l = (wl[0][g] + wl[1][g]) + (wl[2][g] + wl[3][g]);
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+        float p[kSteps];
+        if constexpr (kLPK > 1) {
+#pragma unroll
+            for (int u = 0; u < kSteps; u += 4) {
+                const float4 p4 = sp[wave][sub][(g * kSteps + u) / 4];
+                p[u] = p4.x; p[u + 1] = p4.y; p[u + 2] = p4.z; p[u + 3] = p4.w;
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < kSteps; ++u) p[u] = s[g * kSteps + u];
+        }
+        float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int u = 0; u < kSteps; ++u) {
-            const float p = s[g][u] * inv;
-            acc.x += p * vr[u].x;
-            acc.y += p * vr[u].y;
-            acc.z += p * vr[u].z;
-            acc.w += p * vr[u].w;
+            acc[0] += p[u] * vr[u].x;
+            acc[1] += p[u] * vr[u].y;
+            acc[2] += p[u] * vr[u].z;
+            acc[3] += p[u] * vr[u].w;
         }
-#pragma unroll
-        for (int off = kLPK; off < 64; off <<= 1) {
-            acc.x += __shfl_xor(acc.x, off, 64);
-            acc.y += __shfl_xor(acc.y, off, 64);
-            acc.z += __shfl_xor(acc.z, off, 64);
-            acc.w += __shfl_xor(acc.w, off, 64);
+        // Bit 32 of the lane chooses components 2 and 3, bit 16 the odd one.
+        if constexpr (kLPK <= 32) {
+            acc[0] = swap_sum<32>(acc[0], acc[2]);
+            acc[1] = swap_sum<32>(acc[1], acc[3]);
         }
-        if (sub == 0) red[wave][g][sl] = acc;
+        if constexpr (kLPK <= 16) acc[0] = swap_sum<16>(acc[0], acc[1]);
+        if constexpr (kLPK <= 8) acc[0] += dpp<0x128>(acc[0]);
+        if constexpr (kLPK <= 4) acc[0] += dpp<0x124>(acc[0]);
+        if constexpr (kLPK <= 2) acc[0] += dpp<0x4E>(acc[0]);
+        if constexpr (kLPK <= 1) acc[0] += dpp<0xB1>(acc[0]);
+        float* const out = reinterpret_cast<float*>(&red[wave][g][sl]);
+        if constexpr (kParts == 1) {
+            red[wave][g][sl] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+        } else if constexpr (kParts == 2) {
+            *reinterpret_cast<float2*>(out + 2 * sub) = make_float2(acc[0], acc[1]);
+        } else {
+            if (lane % 16 < kLPK) out[lane / 32 * 2 + lane / 16 % 2] = acc[0];
+        }
     }
     __syncthreads();
 
+    // The four waves by their weights; a NaN among the scores is one in l.
     const uint64_t bh0 = b * a.heads + head0;
     for (int i = threadIdx.x; i < group * D4; i += 256) {
         const int g = i / D4, t = i % D4;
-        float4 o = red[0][g][t];
+        const float m = fmaxf(fmaxf(wm[0][g], wm[1][g]), fmaxf(wm[2][g], wm[3][g]));
+        float f[4];
 #pragma unroll
-        for (int w = 1; w < 4; ++w) {
+        for (int w = 0; w < 4; ++w) f[w] = wm[w][g] == -INFINITY ? wl[w][g] : wl[w][g] * exp2f(wm[w][g] - m);
+        const float l = (f[0] + f[1]) + (f[2] + f[3]);
+        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
             const float4 r = red[w][g][t];
-            o.x += r.x; o.y += r.y; o.z += r.z; o.w += r.w;
+            const float share = f[w] * inv;
+            o.x += share * r.x; o.y += share * r.y; o.z += share * r.z; o.w += share * r.w;
         }
-        const float l = (wl[0][g] + wl[1][g]) + (wl[2][g] + wl[3][g]);
         const uint64_t rec = (bh0 + g) * chunks + c_idx;
         *reinterpret_cast<float4*>(part_o + rec * D + 4 * t) = o;
-        if (t == 0) {
-            const float m = fmaxf(fmaxf(wm[0][g], wm[1][g]), fmaxf(wm[2][g], wm[3][g]));
-            *reinterpret_cast<float2*>(part_ml + 2 * rec) = make_float2(m, l);
-        }
+        if (t == 0) *reinterpret_cast<float2*>(part_ml + 2 * rec) = make_float2(m, l);
     }
 }
 
@@ -1077,7 +1191,7 @@ mhip_status launch_decode_group(mhip_ctx* ctx, const AttnArgs& a, uint64_t batch
         hi = upper;
     }
     constexpr int kSteps = decode_steps(D4);
-    if constexpr (D4 >= 4 && GT <= 2) {
+    if constexpr (D4 >= 4 && GT <= 4) {
         // The choice follows the capacity for a bounded call, so its eager
         // run and a capture of it take the same chunks.
         const uint64_t span = bounded ? kv_rows : hi - lo;
