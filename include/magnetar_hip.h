@@ -179,9 +179,10 @@ mhip_status mhip_rope_f32(mhip_ctx* ctx, const float* in, float* out, uint64_t r
 /* out[m, n] = A . B with A [m, k] (or [k, m] stored when transpose_a) and
  * B [k, n] (or [n, k] when transpose_b), f32 accumulation; addend_mode 1 adds
  * addend[col] (matmul-bias), 2 adds addend[row * n + col] (matmul-residual)
- * to the finished sum. fp32 MFMA tiles for m > 8; an HBM-streaming split-k
- * kernel for m <= 8 (decode), whose partial sums use a grow-only workspace
- * owned by the context. */
+ * to the finished sum. For m > 8 matrix-core tiles, each f32 operand split
+ * exactly into three bf16 planes (six plane products, an error at or below the
+ * f32 matrix instructions'); HBM-streaming kernels for m <= 8 (decode). Partial
+ * sums use a grow-only workspace owned by the context. */
 mhip_status mhip_matmul_f32(mhip_ctx* ctx, const float* a, const float* b, float* out,
                             uint64_t m, uint64_t k, uint64_t n, int transpose_a,
                             int transpose_b, const float* addend, int addend_mode);
@@ -240,7 +241,8 @@ typedef struct {
  * Query i sits at position (kv_seq_len - seq_len) + i; a causal query admits
  * keys up to its own position, a window of w the last w of them. Softmax of
  * q.k * scale over the admitted keys weights V rows; no admitted key gives 0.
- * fp32 MFMA flash prefill for head dims 64/128, split-KV decode for one query
+ * Flash prefill on split bf16 planes for head dims 32, 64, 80, 96, 112 and 128,
+ * split-KV decode for one query
  * row (workspace owned by the context), a generic kernel otherwise. */
 mhip_status mhip_attention_f32(mhip_ctx* ctx, const float* q, const float* k, const float* v,
                                float* out, const mhip_attention_params* params);
