@@ -471,7 +471,9 @@ __global__ __launch_bounds__(PrefillCfg<D>::kThreads, 2) void attn_prefill_kerne
         for (int r = 0; r < 16; ++r) o[vb][r] = 0.0f;
     // A tile's loads: K, 4 of d of one key per unit; V, 8 keys of one column
     // (the chunk of a pair of waves). Buffer loads whose range ends with the
-    // last key: keys past it read as zeros, which the mask takes out.
+    // last key: keys past it read as zeros, which the mask takes out. The key
+    // goes into the vector offset: the range check takes a scalar offset off
+    // the range instead, which wraps where that key lies past the end.
     u32x4 kr[Cfg::kKUnits];
     uint32_t vr[8];
     const int v_chunk = wave >> 1;  // step v_chunk / 2, half v_chunk % 2
@@ -503,7 +505,7 @@ __global__ __launch_bounds__(PrefillCfg<D>::kThreads, 2) void attn_prefill_kerne
 #pragma unroll
         for (int e = 0; e < 8; ++e)
             vr[e] = __builtin_amdgcn_raw_buffer_load_b32(
-                rsrc, v_off, (16 * (v_chunk >> 1) + 4 * (v_chunk & 1) + (e / 4) * 8 + e % 4) * ld_bytes, 0);
+                rsrc, v_off + (16 * (v_chunk >> 1) + 4 * (v_chunk & 1) + (e / 4) * 8 + e % 4) * ld_bytes, 0, 0);
     };
     if (i_end > i_begin) {
         load_k(i_begin);

@@ -63,7 +63,9 @@ __global__ __launch_bounds__(64 * kPanelWaves, 4) void panel_kernel(
 
     // Step t of B: word i is k 16 t + 8 h + i, by buffer loads whose range ends
     // with the matrix (k past its end reads as zero; a slice that ends before
-    // it is whole steps). Steps past the slice repeat its last.
+    // it is whole steps). Steps past the slice repeat its last. The row goes
+    // into the vector offset: the range check takes a scalar offset off the
+    // range instead, which wraps where that row starts past the end.
     const uint32_t voff = (8 * h * n + col) * static_cast<uint32_t>(sizeof(BT));
     auto load = [&](uint32_t t, uint32_t (&r)[8]) {
         const uint64_t k0 = k_begin + min(t, steps - 1) * 16;
@@ -73,8 +75,8 @@ __global__ __launch_bounds__(64 * kPanelWaves, 4) void panel_kernel(
             0x00020000);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const uint32_t soff = i * n * static_cast<uint32_t>(sizeof(BT));
-            r[i] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, voff, soff, kStream);
+            const uint32_t row = i * n * static_cast<uint32_t>(sizeof(BT));
+            r[i] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, voff + row, 0, kStream);
         }
     };
 

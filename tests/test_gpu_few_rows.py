@@ -72,6 +72,26 @@ def test_values_outside_the_split(dev, m, k, n, tb, path, poison):
     check_products(dev, m, k, n, tb, path, poison)
 
 
+@pytest.mark.parametrize("m,k,n", [(9, 1, 2), (17, 33, 510), (12, 54, 258)])
+@pytest.mark.parametrize("compact", [False, True])
+def test_row_panel_reads_nothing_past_b(dev, m, k, n, compact):
+    """What lies behind B (here the next rows of the same allocation, 15 at
+    most of a last step of 16 k) leaves the bits alone, NaN or not: one read
+    would send the columns to the f32 MFMA's sums."""
+    import magnetar_hip
+    from magnetar_hip import ops
+    rng = np.random.default_rng(k)
+    a = dev.upload(rng.standard_normal((m, k)).astype(np.float32))
+    full = rng.standard_normal((k + 16, n)).astype(np.float32)
+    got = []
+    for behind in (0.0, np.nan):
+        full[k:] = behind
+        d = dev.upload((full.view(np.uint32) >> 16).astype(np.uint16) if compact else full)
+        b = magnetar_hip.DeviceArray(dev, d.ptr, (k, n), d.dtype, owned=False)
+        got.append((ops.matmul_bf16w if compact else ops.matmul)(dev, a, b).numpy().view(np.uint32))
+    assert np.array_equal(got[0], got[1])
+
+
 WIDTHS = [1, 63, 255, 1023, 1025, 4095, 4097, 16383, 16385, 16388, 32768, 32772, 49151, 49153, 65536, 65540, 70001,
           128000]
 

@@ -136,3 +136,21 @@ def test_a_cold_capture_of_attention():
     for _ in range(2):
         graph.launch(0)
         check(out.numpy(), q, k, v, 3, 2000, 4, 2, 96, True)
+
+
+@pytest.mark.parametrize("d", [32, 80, 128])
+@pytest.mark.parametrize("kv", [1, 33, 54])
+def test_nothing_is_read_past_the_last_key(dev, d, kv):
+    """What lies behind K and V (the next rows of the same allocation, 31 at
+    most of a last tile of 32 keys) leaves the bits alone, NaN or not."""
+    import magnetar_hip
+    from magnetar_hip import ops
+    q, k, v = inputs(kv, kv, kv + 32, 2, 2, d)
+    p = ops.attention_params(kv, kv, 2, d, kv_head_count=2, causal=True)
+    got = []
+    for behind in (0.0, np.nan):
+        k[kv:] = v[kv:] = behind
+        dk, dv = dev.upload(k), dev.upload(v)
+        views = [magnetar_hip.DeviceArray(dev, x.ptr, (kv, 2 * d), x.dtype, owned=False) for x in (dk, dv)]
+        got.append(ops.attention(dev, dev.upload(q), *views, p).numpy())
+    assert np.array_equal(bits(got[0]), bits(got[1]))
