@@ -21,7 +21,13 @@ namespace mhip {
 
 constexpr int kPanelRows = 32;
 constexpr int kPanelWaves = 8;
-constexpr int kPanelK = 256;    // k of A in LDS at a time (48 KB of planes)
+// k of A in LDS at a time: its planes take 72 KB, two workgroups per CU, or 48
+// KB with a compact B, whose second column block leaves no registers for the
+// 24 that 384 k are fetched into (they spilled: 12 x 4096 x 32000 54 -> 59 us).
+template <class BT>
+constexpr int kPanelK = sizeof(BT) == 2 ? 256 : 384;
+template <class BT>
+constexpr int kPanelLdsBytes = 3 * kPanelRows * kPanelK<BT> * 2;
 constexpr int kPanelDepth = 4;  // steps of 16 k that a wave reads ahead
 // Column blocks of 32 a wave takes: two of a compact B, read in pairs of
 // columns. The f32 tests and sums again 256 columns at a time.
@@ -38,7 +44,8 @@ constexpr int kPanelCols = kPanelWaves * 32 * kPanelBlocks<BT>;
 // What bounds it: the bytes in flight, so the waves a CU holds (two workgroups
 // at 128 registers). The 64 x 64 tiles that these products took before keep 8
 // KB of B in flight per workgroup; here each of 16 waves per CU keeps 8 KB.
-// 24 x 4096 x 11008: f32 MFMA tiles 149 us, split tiles 74, this 48-51.
+// 24 x 4096 x 11008: f32 MFMA tiles 149 us, split tiles 74, this 43 (4.2 TB/s);
+// compact 31.
 template <class BT, class Addend>
 __global__ __launch_bounds__(64 * kPanelWaves, 4) void panel_kernel(
     const float* __restrict__ A, const BT* __restrict__ B, float* __restrict__ C, uint64_t M, uint64_t K,
@@ -46,9 +53,10 @@ __global__ __launch_bounds__(64 * kPanelWaves, 4) void panel_kernel(
     constexpr bool kBf16 = sizeof(BT) == 2;
     constexpr int kBlocks = kPanelBlocks<BT>;
     constexpr int kPlanes = kBf16 ? 1 : 3;
-    constexpr int kChunkBytes = kPanelRows * 16, kPlaneBytes = kPanelK / 8 * kChunkBytes;
+    constexpr int kChunkBytes = kPanelRows * 16, kPlaneBytes = kPanelK<BT> / 8 * kChunkBytes;
     constexpr int kStream = 2;  // non-temporal
-    __shared__ __attribute__((aligned(16))) char lds[3 * kPlaneBytes];
+    static_assert(3 * kPlaneBytes == kPanelLdsBytes<BT>, "the launch's LDS");
+    extern __shared__ __attribute__((aligned(16))) char lds[];
     __shared__ int redo[2];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -87,36 +95,77 @@ __global__ __launch_bounds__(64 * kPanelWaves, 4) void panel_kernel(
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[b][r] = 0.0f;
     };
-    clear();
-    if (threadIdx.x < 2) redo[threadIdx.x] = 0;  // (the chunks' barriers follow)
     uint32_t tiny = 0xFFFFFFFFu;
-    uint32_t raw[kPanelDepth][8];
+    // A's chunk: 8 threads to a row and 32 k, zeros past the slice. Its loads
+    // are 16 bytes where A allows them; a k past the slice reads its first.
+    constexpr int kUnits = kPanelRows * kPanelK<BT> / 4 / (64 * kPanelWaves);
+    const bool wide = K % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0;
+    const int row_a = threadIdx.x / 8 % kPanelRows;
+    const uint32_t kk0 = threadIdx.x % 8 * 4 + threadIdx.x / (8 * kPanelRows) * 32;  // + 64 a unit
+    static_assert(64 * kPanelWaves == 16 * kPanelRows, "a unit is 64 k of every row");
+    const uint32_t len = static_cast<uint32_t>(k_end - k_begin);
+    const float* const a_row = A + (static_cast<uint64_t>(row_a) < M ? row_a : M - 1) * K + k_begin;
+    auto fetch = [&](uint32_t c0, float4 (&x)[kUnits]) {
 #pragma unroll
-    for (int d = 0; d < kPanelDepth; ++d) load(d, raw[d]);
-    constexpr uint32_t kChunkSteps = kPanelK / 16;
-    for (uint32_t c0 = 0; c0 < steps; c0 += kChunkSteps) {
-        // A's chunk: 8 threads to a row and 32 k, zeros past the slice.
-        __syncthreads();
+        for (int q = 0; q < kUnits; ++q) {
+            const uint32_t k = c0 * 16 + kk0 + 64 * q;
+            if (c0 * 16 + 64 * q >= len) break;  // (short slices: no step reads the unit)
+            if (wide) {  // (the slice ends on whole fours, too)
+                x[q] = *reinterpret_cast<const float4*>(a_row + (k < len ? k : 0));
+            } else {
+                x[q].x = a_row[k < len ? k : 0];
+                x[q].y = a_row[k + 1 < len ? k + 1 : 0];
+                x[q].z = a_row[k + 2 < len ? k + 2 : 0];
+                x[q].w = a_row[k + 3 < len ? k + 3 : 0];
+            }
+        }
+    };
+    auto put = [&](uint32_t c0, const float4 (&x)[kUnits]) {
         uint32_t tiny_a = 0xFFFFFFFFu;
 #pragma unroll
-        for (int q = 0; q < kPanelRows * kPanelK / 4 / (64 * kPanelWaves); ++q) {
-            const int f = threadIdx.x + q * 64 * kPanelWaves;
-            const int row = f / 8 % kPanelRows, kk = f % 8 * 4 + f / (8 * kPanelRows) * 32;
-            const uint64_t k = k_begin + c0 * 16 + kk;
-            const float* p = A + (row < M ? row : M - 1) * K;
-            float x[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) x[i] = k + i < k_end ? p[k + i] : 0.0f;
+        for (int q = 0; q < kUnits; ++q) {
+            const uint32_t k = c0 * 16 + kk0 + 64 * q, kk = kk0 + 64 * q;
+            if (c0 * 16 + 64 * q >= len) break;
+            const float y[4] = {k < len ? x[q].x : 0.0f, k + 1 < len ? x[q].y : 0.0f,
+                                k + 2 < len ? x[q].z : 0.0f, k + 3 < len ? x[q].w : 0.0f};
             uint32_t lo[3], hi[3];
-            split_pair(x[0], x[1], lo);
-            split_pair(x[2], x[3], hi);
-            tiny_a = split_min(split_min(tiny_a, x[0], x[1]), x[2], x[3]);
-            char* at = lds + kk / 8 * kChunkBytes + row * 16 + kk % 8 * 2;
+            split_pair(y[0], y[1], lo);
+            split_pair(y[2], y[3], hi);
+            tiny_a = split_min(split_min(tiny_a, y[0], y[1]), y[2], y[3]);
+            char* at = lds + kk / 8 * kChunkBytes + row_a * 16 + kk % 8 * 2;
 #pragma unroll
             for (int p3 = 0; p3 < 3; ++p3) *reinterpret_cast<u32x2*>(at + p3 * kPlaneBytes) = u32x2{lo[p3], hi[p3]};
         }
         if (tiny_a < kSplitTiny) redo[0] = redo[kBlocks - 1] = 1;
+    };
+    uint32_t raw[kPanelDepth][8];
+    if (threadIdx.x < 2) redo[threadIdx.x] = 0;
+    // A's first chunk ahead of an f32 B: loads come back in order, so behind
+    // B's it would wait for all of them (as the next chunks do). With 384 k a
+    // chunk 24 x 4096 x 11008 44.8 -> 42.9 us, 32 x 11008 x 4096 51 -> 48.
+    if constexpr (!kBf16) {
+        float4 x[kUnits];
+        fetch(0, x);
+#pragma unroll
+        for (int d = 0; d < kPanelDepth; ++d) load(d, raw[d]);
         __syncthreads();
+        put(0, x);
+        __syncthreads();
+    } else {
+#pragma unroll
+        for (int d = 0; d < kPanelDepth; ++d) load(d, raw[d]);
+    }
+    clear();
+    constexpr uint32_t kChunkSteps = kPanelK<BT> / 16;
+    for (uint32_t c0 = 0; c0 < steps; c0 += kChunkSteps) {
+        if (kBf16 || c0) {
+            float4 x[kUnits];
+            if constexpr (kBf16) __syncthreads();
+            fetch(c0, x);
+            if constexpr (!kBf16) __syncthreads();
+            put(c0, x);
+            __syncthreads();
+        }
         const uint32_t c_end = min(steps, c0 + kChunkSteps);
         for (uint32_t t0 = c0; t0 < c_end; t0 += kPanelDepth) {
 #pragma unroll

@@ -1466,9 +1466,15 @@ mhip_status launch_panel(mhip_ctx* ctx, const float* a, const BT* b, float* c, u
         mhip_status st = workspace(ctx, slices * m * n * sizeof(float), &target);
         if (st != MHIP_OK) return st;
     }
+    static bool configured = false;  // raise the dynamic-LDS cap above 64 KiB once
+    if (!configured) {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mhip::panel_kernel<BT, AddendEpilogue>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, mhip::kPanelLdsBytes<BT>);
+        configured = true;
+    }
     mhip::launch(ctx, (mhip::panel_kernel<BT, AddendEpilogue>),
                  dim3(static_cast<unsigned>((n + kCols - 1) / kCols), static_cast<unsigned>(slices)),
-                 dim3(64 * mhip::kPanelWaves), 0, a, b, target, m, k, n, k_slice,
+                 dim3(64 * mhip::kPanelWaves), mhip::kPanelLdsBytes<BT>, a, b, target, m, k, n, k_slice,
                  AddendEpilogue{addend, n, mode});
     mhip_status st = mhip::check_launch("matmul (row panel)");
     if (st != MHIP_OK || slices == 1) return st;
