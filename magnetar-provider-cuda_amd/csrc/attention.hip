@@ -109,8 +109,8 @@ struct PrefillCfg {
     static constexpr int kKPlane = D / 8 * kKChunk;
     static constexpr int kVChunk = kVB * 32 * 16;
     static constexpr int kVPlane = 4 * kVChunk;
-    // At 128 Q's third plane does not fit the registers: it stays in LDS.
-    static constexpr bool kQLds = D > 112;
+    // From 112 Q's third plane does not fit the registers: it stays in LDS.
+    static constexpr bool kQLds = D > 96;
     static constexpr int kQBytes = kQLds ? kWaves * kSteps * 1024 : 0;
     static constexpr int kLdsBytes = 3 * (kKPlane + kVPlane) + kQBytes;
     // The f32 sum's tiles.
