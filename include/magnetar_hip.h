@@ -240,7 +240,8 @@ typedef struct {
 /* q [seq, H*d], k [kv_rows, Hkv*d], v [kv_rows, Hkv*vd] -> out [seq, H*vd].
  * Query i sits at position (kv_seq_len - seq_len) + i; a causal query admits
  * keys up to its own position, a window of w the last w of them. Softmax of
- * q.k * scale over the admitted keys weights V rows; no admitted key gives 0.
+ * q.k * scale over the admitted keys weights V rows; a NaN or +inf score, and
+ * admitted scores that are all -inf, give NaN.
  * Flash prefill on split bf16 planes for head dims 32, 64, 80, 96, 112 and 128,
  * split-KV decode for one query
  * row (workspace owned by the context), a generic kernel otherwise. */

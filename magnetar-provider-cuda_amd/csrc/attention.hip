@@ -411,6 +411,12 @@ __device__ __forceinline__ void prefill_f32(const AttnArgs& a, const PrefillPlac
         recompute_admitted<D>(w.q_live ? qhalf : w.K, a.qscale, w.K, kv_ld, w.V, kv_ld,
                               w.tile_begin + lo, w.tile_begin + max(lo, hi), half, o, &m, &l);
     }
+    if (!w.ml && l == 0.0f) {  // every admitted score at -inf
+#pragma unroll
+        for (int vb = 0; vb < Cfg::kVB; ++vb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[vb][r] = NAN;
+    }
 }
 
 // The range of operands as they are split (2 |x| as an integer, see kSplitTiny).
@@ -683,7 +689,9 @@ __global__ __launch_bounds__(PrefillCfg<D>::kThreads, 2) void attn_prefill_kerne
             mhip::lds_barrier<0>();
         }
     }
-    const float inv = l > 0.0f ? 1.0f / l * __uint_as_float(static_cast<uint32_t>(127 + v_shift) << 23) : 0.0f;
+    // (No weight: a record's zeros, or, every admitted score at -inf, NaN.)
+    const float inv = l > 0.0f ? 1.0f / l * __uint_as_float(static_cast<uint32_t>(127 + v_shift) << 23)
+                               : sp.nchunks > 1 ? 0.0f : NAN;
 #pragma unroll
     for (int vb = 0; vb < Cfg::kVB; ++vb)
 #pragma unroll
@@ -727,8 +735,8 @@ mhip_status attention_workspace(mhip_ctx* ctx, size_t bytes, float** out) {
 
 // Merges a split prefill's chunk records per (query row, head): out = sum_c
 // w_c o_c with w_c = l_c 2^(m_c - M) / sum_c' l_c' 2^(m_c' - M), in chunk
-// order; no admitted key in any chunk gives zeros. VD / 4 threads per (row,
-// head), one float4 of the output each.
+// order; a chunk without weight (no admitted key, or every score at -inf) has
+// l_c = 0. VD / 4 threads per (row, head), one float4 of the output each.
 template <int VD>
 __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(AttnArgs a, uint64_t rows,
                                                                    PrefillSplit sp) {
@@ -744,15 +752,17 @@ __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(AttnArgs a, u
     float M = -INFINITY;
     for (uint32_t c = 0; c < sp.nchunks; ++c) M = fmaxf(M, ml[2 * c]);
     float total = 0.0f;
-    if (M != -INFINITY)
-        for (uint32_t c = 0; c < sp.nchunks; ++c)
-            if (ml[2 * c + 1] > 0.0f) total += ml[2 * c + 1] * exp2f(ml[2 * c] - M);
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (uint32_t c = 0; c < sp.nchunks; ++c)
+        if (ml[2 * c + 1] != 0.0f) total += ml[2 * c + 1] * exp2f(ml[2 * c] - M);
+    // Every query admits a key: no weight at all is every score at -inf, whose
+    // weights are NaN as those of a NaN or +inf score are.
+    float4 acc = make_float4(NAN, NAN, NAN, NAN);
     if (total > 0.0f) {
+        acc = make_float4(0.f, 0.f, 0.f, 0.f);
         const float inv_total = 1.0f / total;
         for (uint32_t c = 0; c < sp.nchunks; ++c) {
             const float l = ml[2 * c + 1];
-            if (!(l > 0.0f)) continue;
+            if (l == 0.0f) continue;
             const float w = l * exp2f(ml[2 * c] - M) * inv_total;
             const float4 o = *reinterpret_cast<const float4*>(po + c * VD);
             acc.x += w * o.x; acc.y += w * o.y; acc.z += w * o.z; acc.w += w * o.w;

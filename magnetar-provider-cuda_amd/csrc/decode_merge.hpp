@@ -5,13 +5,16 @@
 // Records of one (batch, head): chunk c holds its output o_c (normalised by
 // its own weight sum), its score max m_c (log2 domain) and weight sum l_c.
 // The merge is out = sum_c w_c o_c with w_c = l_c 2^(m_c - M) / sum_c' l_c'
-// 2^(m_c' - M) and M = max_c m_c; chunks with no admitted key (l_c = 0) weigh
-// nothing, and a head with none at all gives zeros. The same online-softmax
-// merge as src/kernels.cu:1868-1959 computes within one pass.
+// 2^(m_c' - M) and M = max_c m_c; chunks with no admitted key, or with every
+// score at -inf (l_c = 0), weigh nothing. A NaN or +inf score makes l_c NaN and
+// the output with it, and so does a query without any weight (it admits at
+// least its own key, so every score was -inf). The same online-softmax merge
+// as src/kernels.cu:1868-1959 computes within one pass.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdint>
 
 namespace mhip {
@@ -62,11 +65,11 @@ __device__ __forceinline__ float4 merge_decode_chunks(const float* __restrict__ 
     __syncthreads();
     const float M = fmaxf(fmaxf(rm[0], rm[1]), fmaxf(rm[2], rm[3]));
     float tot = 0.0f;
-    if (M != -INFINITY && threadIdx.x < chunks) {
-        if (mine.y > 0.0f) tot += mine.y * exp2f(mine.x - M);
+    if (threadIdx.x < chunks) {
+        if (mine.y != 0.0f) tot += mine.y * exp2f(mine.x - M);
         for (uint64_t c = threadIdx.x + 256; c < chunks; c += 256) {
             const float2 e = *reinterpret_cast<const float2*>(ml + 2 * c);
-            if (e.y > 0.0f) tot += e.y * exp2f(e.x - M);
+            if (e.y != 0.0f) tot += e.y * exp2f(e.x - M);
         }
     }
 #pragma unroll
@@ -118,6 +121,7 @@ __device__ __forceinline__ float4 merge_decode_chunks(const float* __restrict__ 
             const float4 r = red[g][threadIdx.x];
             v.x += r.x; v.y += r.y; v.z += r.z; v.w += r.w;
         }
+        if (!(total > 0.0f)) v = make_float4(NAN, NAN, NAN, NAN);
     }
     return v;
 }
