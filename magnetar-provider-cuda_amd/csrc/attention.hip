@@ -799,11 +799,8 @@ mhip_status launch_prefill(mhip_ctx* ctx, const AttnArgs& a, uint64_t batch, boo
     const uint64_t qtiles = (a.seq + Cfg::kBQ - 1) / Cfg::kBQ;
     PrefillSplit sp{};
     prefill_split(ctx, a, replayable, qtiles, Cfg::kBKV, &sp.nchunks, &sp.chunk_tiles);
-    // A capture's workspace does not grow, which refuses it chunks. Head
-    // dimensions that need none on the generic kernel go without.
-    if (D != 64 && D != 128 && sp.nchunks > 1 &&
-        mhip::workspace_short(ctx, batch * a.seq * a.heads * sp.nchunks * (D + 2) * sizeof(float)))
-        sp.nchunks = 1;
+    // (The other head dimensions ran on the generic kernel, without chunks.)
+    const mhip::CaptureGrowth growth(ctx, D != 64 && D != 128);
     const uint64_t blocks = batch * a.heads * qtiles * sp.nchunks;
     if (blocks >= (1ULL << 31)) return mhip::fail(MHIP_SHAPE_UNSUPPORTED, "attention: too many query tiles");
     sp.qtiles = static_cast<uint32_t>(qtiles);

@@ -52,6 +52,7 @@ struct mhip_ctx {
     // `max_offset`. `failure` keeps the first reason the capture cannot be
     // replayed (an allocation, a transfer, a synchronisation).
     bool capturing = false;
+    bool capture_growth = false;  // mhip::CaptureGrowth
     struct RecordedLaunch {
         const void* kernel = nullptr;
         dim3 grid, block;
@@ -234,10 +235,22 @@ void launch(mhip_ctx* ctx, void (*kernel)(P...), dim3 grid, dim3 block, size_t s
 
 // The context's grow-only scratch of at least `bytes` (split-k partials,
 // attention chunk records). Growing it waits for the stream; a buffer a live
-// graph may read is retired, not freed. Refused while capturing.
+// graph may read is retired, not freed. Refused while capturing, outside a
+// CaptureGrowth.
 mhip_status workspace(mhip_ctx* ctx, size_t bytes, void** out);
-// Whether that would be refused for a capture.
-bool workspace_short(const mhip_ctx* ctx, size_t bytes);
+
+// A call whose earlier kernel took no more scratch than the workspace holds,
+// and which a capture therefore takes: while it lives, the workspace may grow
+// for a capture too (a capture only records, so nothing it allocates is in the
+// way), and the captured call is the eager one, bit for bit. What the capture
+// has recorded may read the old buffer, which is retired.
+struct CaptureGrowth {
+    mhip_ctx* const ctx;
+    CaptureGrowth(mhip_ctx* c, bool allowed) : ctx(c) { ctx->capture_growth = allowed; }
+    ~CaptureGrowth() { ctx->capture_growth = false; }
+    CaptureGrowth(const CaptureGrowth&) = delete;
+    CaptureGrowth& operator=(const CaptureGrowth&) = delete;
+};
 
 // Looks up (once per device, with the context's device current) the device
 // address of the allocation-free matmul's fixed scratch array; called when a

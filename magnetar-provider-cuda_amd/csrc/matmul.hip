@@ -88,10 +88,6 @@ mhip_status workspace(mhip_ctx* ctx, size_t bytes, float** out) {
     return st;
 }
 
-// Whether a capture that would take a product of this size without partial
-// sums cannot have the bytes that its few-row kernel wants (choose_tiles).
-bool scratch_short(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n, size_t bytes);
-
 // ---------------------------------------------------------------------------
 // MFMA tiles
 // ---------------------------------------------------------------------------
@@ -1457,10 +1453,6 @@ mhip_status launch_panel(mhip_ctx* ctx, const float* a, const BT* b, float* c, u
     constexpr uint64_t kCols = mhip::kPanelCols<BT>;
     uint64_t slices, k_slice;
     panel_slicing(ctx, k, n, &slices, &k_slice);
-    if (slices > 1 && scratch_short(ctx, m, k, n, slices * m * n * sizeof(float))) {
-        slices = 1;
-        k_slice = (k + 15) / 16 * 16;
-    }
     float* target = c;
     if (slices > 1) {
         mhip_status st = workspace(ctx, slices * m * n * sizeof(float), &target);
@@ -1486,10 +1478,6 @@ mhip_status launch_ragged_gemv(mhip_ctx* ctx, const float* a, const BT* b, float
                                const float* addend, int mode) {
     uint64_t slices, k_per_slice;
     gemv_slicing(ctx, k, n, &slices, &k_per_slice);
-    if (slices > 1 && scratch_short(ctx, ROWS, k, n, slices * ROWS * n * sizeof(float))) {
-        slices = 1;
-        k_per_slice = k;
-    }
     float* target = c;
     if (slices > 1) {
         mhip_status st = workspace(ctx, slices * ROWS * n * sizeof(float), &target);
@@ -1622,12 +1610,12 @@ TileOption fastest_tiles(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n
 }
 
 // Which products the entry points with limited scratch take was settled by the
-// plans of the f32 MFMA kernels, whose fractions of the peak kF32 is:
+// plans of the f32 MFMA kernels, whose fractions of the peak kF32 is.
 // mhip_matmul_f32_noalloc, which gives mhip_matmul_f32's bits, refuses partial
-// sums beyond its array, and a capture those beyond the context's workspace,
-// which does not grow while recording. A product whose plan was within the
-// limit then stays within it, by the fastest option that does (for the array
-// one product in 500 over m 9-16384, k and n 1-65536).
+// sums beyond its array: a product whose plan was within it stays within, by
+// the fastest option that does (one product in 500 over m 9-16384, k and n
+// 1-65536). A capture refuses those beyond the context's workspace: for a
+// product whose plan was within it the workspace grows (mhip::CaptureGrowth).
 constexpr double kSplit[4] = {1.40, 1.30, 1.20, 0.76}, kF32[4] = {0.88, 0.82, 0.83, 0.65};
 
 bool within_before(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n, uint64_t limit) {
@@ -1638,13 +1626,7 @@ TileChoice choose_tiles(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n)
     TileOption best = fastest_tiles(ctx, m, k, n, kSplit, 4.0e12, UINT64_MAX);
     if (best.bytes > MHIP_NOALLOC_SCRATCH_BYTES && within_before(ctx, m, k, n, MHIP_NOALLOC_SCRATCH_BYTES))
         best = fastest_tiles(ctx, m, k, n, kSplit, 4.0e12, MHIP_NOALLOC_SCRATCH_BYTES);
-    if (!ctx->fixed_scratch && mhip::workspace_short(ctx, best.bytes) && within_before(ctx, m, k, n, ctx->workspace_bytes))
-        best = fastest_tiles(ctx, m, k, n, kSplit, 4.0e12, ctx->workspace_bytes);
     return best.choice;
-}
-
-bool scratch_short(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n, size_t bytes) {
-    return !ctx->fixed_scratch && mhip::workspace_short(ctx, bytes) && within_before(ctx, m, k, n, ctx->workspace_bytes);
 }
 
 // Few-row products by shape (few_rows.hpp), after the vector GEMV: up to 8
@@ -1752,12 +1734,12 @@ mhip_status matmul_impl(mhip_ctx* ctx, const float* a, const BT* b, float* out, 
     // multiple of 4 elements and an aligned base.
     const uintptr_t b_align = sizeof(BT) == 4 ? 15u : 7u;
     const bool b_aligned = (reinterpret_cast<uintptr_t>(b) & b_align) == 0;
-    // (One stored [k, 1] goes the way of ragged rows where a capture has no room.)
-    uint64_t slices = 1, per_slice = k;
-    if (transpose_a && m == 1) gemv_slicing(ctx, k, n, &slices, &per_slice);
-    const bool roomy = slices == 1 || !scratch_short(ctx, m, k, n, slices * n * sizeof(float));
-    if (m <= kGemvMaxRows && !ta && !tb && n % 4 == 0 && b_aligned && roomy)
+    // (A row of A stored [k, 1] took the tiles before.)
+    auto taken_before = [&] { return ctx->capturing && within_before(ctx, m, k, n, ctx->workspace_bytes); };
+    if (m <= kGemvMaxRows && !ta && !tb && n % 4 == 0 && b_aligned) {
+        const mhip::CaptureGrowth growth(ctx, transpose_a != 0 && taken_before());
         return dispatch_gemv<BT>(ctx, a, b, out, m, k, n, addend, addend_mode);
+    }
     // A few rows of a small product (up to 32 rows in blocks of 8, at most
     // 2^26 multiply-adds): one launch of small_mfma_kernel up to k = 1024,
     // else the GEMV's two short launches; both beat MFMA tiles that would be
@@ -1768,6 +1750,7 @@ mhip_status matmul_impl(mhip_ctx* ctx, const float* a, const BT* b, float* out, 
             return launch_small_mfma<BT>(ctx, a, b, out, m, k, n, addend, addend_mode);
         return launch_gemv<kGemvMaxRows, BT>(ctx, a, b, out, k, n, addend, addend_mode, m / kGemvMaxRows);
     }
+    const mhip::CaptureGrowth growth(ctx, taken_before());
     if (ragged_gemv_fits(m, n, ta, tb))
         return dispatch_ragged_gemv<BT>(ctx, a, b, out, m, k, n, addend, addend_mode);
     if (dot_fits(m, k, n, ta, tb, mhip::aligned16(b)) && mhip::aligned16(a))

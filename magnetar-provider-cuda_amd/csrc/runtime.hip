@@ -60,20 +60,27 @@ const uint64_t* advance_ptr(mhip_ctx* ctx, uint32_t bit, uint64_t max_offset) {
 }
 
 // Frees `p` now, or keeps it until the last live graph is destroyed.
+// (The launches of a capture in progress are a graph's to be.)
 static void release_buffer(mhip_ctx* ctx, void* p) {
     if (!p) return;
-    if (ctx->live_graphs > 0) ctx->retired.push_back(p);
+    if (ctx->live_graphs > 0 || ctx->capturing) ctx->retired.push_back(p);
     else (void)hipFree(p);
 }
 
-bool workspace_short(const mhip_ctx* ctx, size_t bytes) {
-    return ctx->capturing && ctx->workspace_bytes < bytes;
+// Frees the retired buffers once no graph is left to read them.
+static void free_retired(mhip_ctx* ctx) {
+    if (ctx->live_graphs > 0 || ctx->retired.empty()) return;
+    (void)hipStreamSynchronize(ctx->stream);
+    for (void* p : ctx->retired) (void)hipFree(p);
+    ctx->retired.clear();
 }
 
 mhip_status workspace(mhip_ctx* ctx, size_t bytes, void** out) {
     if (ctx->workspace_bytes < bytes) {
-        mhip_status st = forbid_in_capture(ctx, "growing the workspace");
-        if (st != MHIP_OK) return st;
+        if (!ctx->capture_growth) {
+            mhip_status st = forbid_in_capture(ctx, "growing the workspace");
+            if (st != MHIP_OK) return st;
+        }
         if (ctx->workspace) {
             (void)hipStreamSynchronize(ctx->stream);
             release_buffer(ctx, ctx->workspace);
@@ -460,6 +467,7 @@ mhip_status mhip_capture_end(mhip_ctx* ctx, mhip_graph** out, uint64_t* max_offs
         ctx->recorded.clear();
         (void)hipFree(ctx->capture_offset);
         ctx->capture_offset = nullptr;
+        mhip::free_retired(ctx);
         return mhip::fail(MHIP_CAPTURE_UNSUPPORTED, failure);
     }
     mhip_graph* g = new mhip_graph();
@@ -489,6 +497,7 @@ mhip_status mhip_capture_abort(mhip_ctx* ctx) {
     if (ctx->capture_offset) (void)hipFree(ctx->capture_offset);
     ctx->capture_offset = nullptr;
     ctx->capture_failure.clear();
+    mhip::free_retired(ctx);
     return MHIP_OK;
 }
 
@@ -539,10 +548,7 @@ mhip_status mhip_graph_destroy(mhip_graph* graph) {
     if (graph->table) (void)hipFree(graph->table);
     for (uint64_t* t : graph->old_tables) (void)hipFree(t);
     ctx->live_graphs -= 1;
-    if (ctx->live_graphs == 0) {
-        for (void* p : ctx->retired) (void)hipFree(p);
-        ctx->retired.clear();
-    }
+    mhip::free_retired(ctx);
     delete graph;
     return MHIP_OK;
 }

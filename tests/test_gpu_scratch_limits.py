@@ -35,6 +35,83 @@ def test_a_cold_capture_of_a_product(m, k, n, ta):
         assert np.all(np.abs(out.numpy() - a.astype(np.float64) @ wide) <= bound)
 
 
+# The same, a product whose partial sums are stream-K's, and prompts in key
+# chunks: a capture takes the eager call's plan, so its replays have its bits.
+CALLS = [("matmul", (1, 64, 10, False)), ("matmul", (20, 480, 640, False)), ("matmul", (1, 480, 64, True)),
+         ("matmul", (192, 3072, 5120, False)), ("matmul", (5, 500, 333, False)), ("matmul", (31, 500, 1030, False)),
+         ("attention", (3, 2000, 4, 2, 96)), ("attention", (300, 1000, 8, 8, 80)), ("attention", (40, 600, 2, 1, 32))]
+
+
+def call_of(kind, shape):
+    """make(device) -> (run, out): the call on that device, its inputs the same on every one."""
+    from magnetar_hip import ops
+    rng = np.random.default_rng(sum(shape))
+    normal = lambda *s: rng.standard_normal(s).astype(np.float32)
+    if kind == "matmul":
+        m, k, n, ta = shape
+        host = [normal(k, m) if ta else normal(m, k), normal(k, n)]
+        def make(device):
+            da, db, out = device.upload(host[0]), device.upload(host[1]), device.empty((m, n))
+            return (lambda: ops.matmul(device, da, db, ta, False, out=out)), out
+        return make
+    s, kv, h, hkv, d = shape
+    host = [normal(s, h * d), normal(kv, hkv * d), normal(kv, hkv * d)]
+    def make(device):
+        q, k, v, out = *map(device.upload, host), device.empty((s, h * d))
+        p = ops.attention_params(s, kv, h, d, kv_head_count=hkv, causal=True)
+        return (lambda: ops.attention(device, q, k, v, p, out)), out
+    return make
+
+
+@pytest.mark.parametrize("kind,shape", CALLS)
+def test_a_cold_capture_has_the_eager_bits(dev, kind, shape):
+    import magnetar_hip
+    make = call_of(kind, shape)
+    run, out = make(dev)
+    run()
+    want = bits(out.numpy())
+    fresh = magnetar_hip.Device(0)
+    run, out = make(fresh)
+    fresh.capture_begin(0)
+    run()
+    graph = fresh.capture_end()
+    for _ in range(2):
+        fresh.zeros(out.shape)  # (eager work between replays)
+        graph.launch(0)
+        assert np.array_equal(bits(out.numpy()), want)
+
+
+def test_growing_for_a_capture_leaves_earlier_launches_their_scratch():
+    """A workspace that grows while recording: the launches recorded before it,
+    in the same capture and in a live graph, keep theirs."""
+    import magnetar_hip
+    fresh, other = magnetar_hip.Device(0), magnetar_hip.Device(0)
+    calls = [call_of(*CALLS[i]) for i in (0, 1, 3, 7)]
+    runs, outs = zip(*(make(fresh) for make in calls))
+    wants = []
+    for make in calls:
+        run, out = make(other)
+        run()
+        wants.append(bits(out.numpy()))
+    graphs = []
+    for some in ((0,), (0, 1), (0, 1, 2, 3)):
+        fresh.capture_begin(0)
+        for i in some:
+            runs[i]()
+        graphs.append((some, fresh.capture_end()))
+    fresh.capture_begin(0)
+    runs[2]()
+    fresh.capture_abort()
+    for some, graph in graphs * 2:
+        graph.launch(0)
+        for i in some:
+            assert np.array_equal(bits(outs[i].numpy()), wants[i])
+    for _, graph in graphs:
+        graph.close()
+    runs[3]()
+    assert np.array_equal(bits(outs[3].numpy()), wants[3])
+
+
 def test_a_product_the_fixed_scratch_took_is_taken(dev):
     """The fastest tiles of 3392 x 5056 x 5952 want 162 MB of partial sums."""
     from magnetar_hip import _lib, ops
