@@ -29,8 +29,7 @@ constexpr int kPanelK = sizeof(BT) == 2 ? 256 : 384;
 template <class BT>
 constexpr int kPanelLdsBytes = 3 * kPanelRows * kPanelK<BT> * 2;
 constexpr int kPanelDepth = 4;  // steps of 16 k that a wave reads ahead
-// Column blocks of 32 a wave takes: two of a compact B, read in pairs of
-// columns. The f32 tests and sums again 256 columns at a time.
+// Column blocks of 32 a wave takes: two of a compact B, read in pairs of columns.
 template <class BT>
 constexpr int kPanelBlocks = sizeof(BT) == 2 ? 2 : 1;
 template <class BT>
@@ -57,7 +56,7 @@ __global__ __launch_bounds__(64 * kPanelWaves, 4) void panel_kernel(
     constexpr int kStream = 2;  // non-temporal
     static_assert(3 * kPlaneBytes == kPanelLdsBytes<BT>, "the launch's LDS");
     extern __shared__ __attribute__((aligned(16))) char lds[];
-    __shared__ int redo[2];
+    __shared__ int redo, any_tiny;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int l32 = lane & 31, h = lane >> 5;
@@ -86,6 +85,11 @@ __global__ __launch_bounds__(64 * kPanelWaves, 4) void panel_kernel(
             const uint32_t row = i * n * static_cast<uint32_t>(sizeof(BT));
             r[i] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, voff + row, 0, kStream);
         }
+    };
+
+    // The element of column block j in a word of B.
+    auto word = [](uint32_t r, int j) {
+        return !kBf16 ? __uint_as_float(r) : j == 0 ? bf16_lo(r) : bf16_hi(r);
     };
 
     f32x16 acc[kBlocks];
@@ -136,10 +140,10 @@ __global__ __launch_bounds__(64 * kPanelWaves, 4) void panel_kernel(
 #pragma unroll
             for (int p3 = 0; p3 < 3; ++p3) *reinterpret_cast<u32x2*>(at + p3 * kPlaneBytes) = u32x2{lo[p3], hi[p3]};
         }
-        if (tiny_a < kSplitTiny) redo[0] = redo[kBlocks - 1] = 1;
+        if (tiny_a < kSplitTiny) redo = any_tiny = 1;
     };
     uint32_t raw[kPanelDepth][8];
-    if (threadIdx.x < 2) redo[threadIdx.x] = 0;
+    if (threadIdx.x == 0) redo = any_tiny = 0;
     // A's first chunk ahead of an f32 B: loads come back in order, so behind
     // B's it would wait for all of them (as the next chunks do). With 384 k a
     // chunk 24 x 4096 x 11008 44.8 -> 42.9 us, 32 x 11008 x 4096 51 -> 48.
@@ -216,27 +220,120 @@ __global__ __launch_bounds__(64 * kPanelWaves, 4) void panel_kernel(
         }
     }
 
-    // Values outside the split (split_tile.hpp): the waves of 256 columns (the
-    // same whatever B's format) sum again with the f32 MFMA, straight from memory.
+    // Sums outside the split (split_tile.hpp), entry by entry, in waves that
+    // have any: again with the f32 MFMA, straight from memory. 24 x 4096 x 11008
+    // with a value below 2^-100 in 64 of A 72 us, 43 with none.
     float probe = 0.0f;
 #pragma unroll
     for (int j = 0; j < kBlocks; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(acc[j][r], 0.0f, probe);
-    const int part = wave / (kPanelWaves / kBlocks);
-    if (tiny < kSplitTiny || probe != 0.0f) redo[part] = 1;
+    if (probe != 0.0f) redo = 1;
+    if (tiny < kSplitTiny) redo = any_tiny = 1;
     __syncthreads();
-    if (redo[part]) {
-        clear();
-        const float* arow = A + (static_cast<uint64_t>(l32) < M ? l32 : M - 1) * K;
-        for (uint64_t k = k_begin; k < k_end; k += 2) {
-            const uint64_t kh = min(k + h, k_end - 1);
-            const bool on = k + h < k_end;
-            const float x = on ? arow[kh] : 0.0f;
+    if (redo) {
+        // The extents of the slice's 32 rows (in LDS, whose planes are done
+        // with) and of the lane's columns.
+        float2 col_line[kBlocks];
+#pragma unroll
+        for (int j = 0; j < kBlocks; ++j) col_line[j] = make_float2(0.f, 0.f);
+        uint32_t* const least_a = reinterpret_cast<uint32_t*>(lds);
+        uint32_t* const big_a = least_a + kPanelRows;
+        const float count = static_cast<float>(len);
+        if (any_tiny) {
+            if (threadIdx.x < kPanelRows) least_a[threadIdx.x] = 0xFFFFFFFFu, big_a[threadIdx.x] = 0;
+            __syncthreads();
+            constexpr int kRowThreads = 64 * kPanelWaves / kPanelRows;
+            const int row = threadIdx.x / kRowThreads;
+            const float* const x = A + (static_cast<uint64_t>(row) < M ? row : M - 1) * K + k_begin;
+            uint32_t least = 0xFFFFFFFFu, big = 0;
+            for (uint32_t k = threadIdx.x % kRowThreads; k < len; k += kRowThreads) {
+                least = split_min(least, x[k], 0.0f);
+                big = split_max(big, x[k], 0.0f);
+            }
+            atomicMin(least_a + row, least);
+            atomicMax(big_a + row, big);
+            uint32_t least_b[kBlocks], big_b[kBlocks];
+#pragma unroll
+            for (int j = 0; j < kBlocks; ++j) least_b[j] = 0xFFFFFFFFu, big_b[j] = 0;
+            for (uint32_t t = 0; t < steps; t += kPanelDepth) {
+#pragma unroll
+                for (int d = 0; d < kPanelDepth; ++d) load(t + d, raw[d]);
+#pragma unroll
+                for (int d = 0; d < kPanelDepth; ++d)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+#pragma unroll
+                        for (int j = 0; j < kBlocks; ++j) {
+                            const float y = word(raw[d][i], j);
+                            least_b[j] = split_min(least_b[j], y, 0.0f);
+                            big_b[j] = split_max(big_b[j], y, 0.0f);
+                        }
+            }
 #pragma unroll
             for (int j = 0; j < kBlocks; ++j)
-                acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, on ? elem(B + kh * N + col + j) : 0.0f,
-                                                              acc[j], 0, 0, 0);
+                col_line[j] = split_line(min(least_b[j], __shfl_xor(least_b[j], 32, 64)),
+                                         max(big_b[j], __shfl_xor(big_b[j], 32, 64)));
+            __syncthreads();
+        }
+        uint32_t again = 0, zero = 0;
+        auto line_of = [&](int row) {
+            return any_tiny ? split_line(least_a[row], big_a[row]) : make_float2(0.f, 0.f);
+        };
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float2 row_line = line_of(8 * (r / 4) + 4 * h + r % 4);
+#pragma unroll
+            for (int j = 0; j < kBlocks; ++j) {
+                const bool is = split_lost(acc[j][r], split_loss(row_line, col_line[j], count));
+                again |= (is ? 1u : 0u) << (j * 16 + r);
+                zero |= (is && acc[j][r] == 0.0f ? 1u : 0u) << (j * 16 + r);
+            }
+        }
+        for (uint64_t lanes; (lanes = __builtin_amdgcn_ballot_w64(zero != 0)) != 0;) {
+            const int l = __builtin_ctzll(lanes);
+            const int bit = __builtin_ctz(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(zero), l)));
+            const int r = bit % 16, row = 8 * (r / 4) + 4 * (l >> 5) + r % 4;
+            const float2 row_line = line_of(row);
+            float2 line = col_line[0];
+            if (bit / 16) line = col_line[kBlocks - 1];
+            line = make_float2(__shfl(line.x, l, 64), __shfl(line.y, l, 64));
+            const float* const x = A + (static_cast<uint64_t>(row) < M ? row : M - 1) * K;
+            const BT* const y = B + min(col0 + (l & 31) * kBlocks, n - kBlocks) + bit / 16;
+            const bool kept = split_cancelled(row_line, line, split_loss(row_line, line, count), k_begin, k_end,
+                                              [&](uint64_t k) { return x[k]; }, [&](uint64_t k) { return elem(y + k * N); });
+            if (lane == l) {
+                zero &= zero - 1;
+                if (kept) again &= ~(1u << bit);
+            }
+        }
+        if (__builtin_amdgcn_ballot_w64(again != 0)) {
+            f32x16 first[kBlocks];
+#pragma unroll
+            for (int j = 0; j < kBlocks; ++j) first[j] = acc[j];
+            clear();
+            const float* const x = A + (static_cast<uint64_t>(l32) < M ? l32 : M - 1) * K + k_begin;
+            for (uint32_t t = 0; t < steps; t += 2) {
+                // (A half of the wave sums k 8 h + i of a step, as it holds B.)
+                load(t, raw[0]);
+                load(t + 1, raw[1]);
+#pragma unroll
+                for (int d = 0; d < 2; ++d)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const uint32_t k = (t + d) * 16 + 8 * h + i;
+                        const float xa = k < len ? x[k] : 0.0f;
+#pragma unroll
+                        for (int j = 0; j < kBlocks; ++j)
+                            acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                                xa, k < len ? word(raw[d][i], j) : 0.0f, acc[j], 0, 0, 0);
+                    }
+            }
+#pragma unroll
+            for (int j = 0; j < kBlocks; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (!(again >> (j * 16 + r) & 1u)) acc[j][r] = first[j][r];
         }
     }
 

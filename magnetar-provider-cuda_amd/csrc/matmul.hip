@@ -151,7 +151,12 @@ __device__ __forceinline__ void gemm_tile(const float* __restrict__ A, const BT*
                                           const float* __restrict__ addend, int addend_mode) {
     using Tile = typename Shape::template Tile<A_T, B_T, BT>;
     Tile tile;
-    tile.sum(A, B, M, K, N, m0, n0, k_begin, k_end, access.wide_a, access.wide_b, access.short_rows, lds);
+    typename Tile::Mask again;
+    const bool redo = tile.sum(A, B, M, K, N, m0, n0, k_begin, k_end, access.wide_a, access.wide_b,
+                               access.short_rows, lds, again);
+    auto sum_again = [&]() {
+        tile.sum_f32(A, B, M, K, N, m0, n0, k_begin, k_end, access.wide_a, access.wide_b, access.short_rows, lds);
+    };
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int kg = wave / Tile::kTileWaves, wt = wave % Tile::kTileWaves;
@@ -159,8 +164,9 @@ __device__ __forceinline__ void gemm_tile(const float* __restrict__ A, const BT*
     const int lrow = lane & 31, lk = lane >> 5;
 
     // Accumulator r of lane l holds C[8*(r/4) + 4*(l/32) + r%4][l%32] of its
-    // 32x32 block; registers [R0, R1) are written.
-    auto store = [&](auto r0, auto r1) {
+    // 32x32 block; registers [R0, R1) are written, all of them or those whose
+    // bit of `again` is not `flip`.
+    auto store = [&](auto r0, auto r1, auto all, uint32_t flip) {
 #pragma unroll
         for (int i = 0; i < Tile::kMI; ++i) {
 #pragma unroll
@@ -170,6 +176,8 @@ __device__ __forceinline__ void gemm_tile(const float* __restrict__ A, const BT*
 #pragma unroll
                 for (int r = decltype(r0)::value; r < decltype(r1)::value; ++r) {
                     const uint64_t row = m0 + wm * Shape::WM + i * 32 + 8 * (r / 4) + 4 * lk + (r % 4);
+                    const int bit = (i * Tile::kNI + j) * 16 + r;
+                    if (!decltype(all)::value && (again[bit / 32] >> bit % 32 & 1u) == flip) continue;
                     if (row < M) {
                         float v = tile.acc[i][j][r];
                         if (addend_mode == 1) v = v + addend[col];
@@ -191,6 +199,23 @@ __device__ __forceinline__ void gemm_tile(const float* __restrict__ A, const BT*
     using R16 = std::integral_constant<int, 16>;
 
     if constexpr (Shape::KG == 2) {
+        if (redo) {
+            mhip::f32x16 first[Tile::kMI][Tile::kNI];
+#pragma unroll
+            for (int i = 0; i < Tile::kMI; ++i)
+#pragma unroll
+                for (int j = 0; j < Tile::kNI; ++j) first[i][j] = tile.acc[i][j];
+            sum_again();
+#pragma unroll
+            for (int i = 0; i < Tile::kMI; ++i)
+#pragma unroll
+                for (int j = 0; j < Tile::kNI; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int bit = (i * Tile::kNI + j) * 16 + r;
+                        if (!(again[bit / 32] >> bit % 32 & 1u)) tile.acc[i][j][r] = first[i][j][r];
+                    }
+        }
         // Two k groups: each finishes half of every block's rows, group 0
         // registers 0-7 (rows 0-15 of a 32x32 block), group 1 registers
         // 8-15, handing the other half to its partner through LDS, so both
@@ -226,10 +251,15 @@ __device__ __forceinline__ void gemm_tile(const float* __restrict__ A, const BT*
         if (kg == 0) take(R0{}, std::true_type{});
         else take(R8{}, std::false_type{});
         __syncthreads();  // LDS is free again
-        if (kg == 0) store(R0{}, R8{});
-        else store(R8{}, R16{});
+        if (kg == 0) store(R0{}, R8{}, std::true_type{}, 0);
+        else store(R8{}, R16{}, std::true_type{}, 0);
+    } else if (!redo) {
+        store(R0{}, R16{}, std::true_type{}, 0);
     } else {
-        store(R0{}, R16{});
+        // (The registers hold one set of sums: those that stay are written first.)
+        store(R0{}, R16{}, std::false_type{}, 1);
+        sum_again();
+        store(R0{}, R16{}, std::false_type{}, 0);
     }
 }
 

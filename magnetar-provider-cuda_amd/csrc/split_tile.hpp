@@ -19,10 +19,16 @@
 // the six with zero planes bit for bit.
 //
 // The split holds for zeros and 2^-100 <= |x| < the largest f32 that rounds
-// to a finite bf16. A tile that meets anything else (a nonzero below 2^-100,
-// seen while splitting; an infinity, a NaN or a value beyond, whose planes
-// turn every sum they enter into a NaN; a sum that overflows) is summed again
-// with the f32 MFMA from its start, so its results are an f32 sum's.
+// to a finite bf16; any other value that enters a sum costs it terms that the
+// f32 MFMA keeps. An entry whose sum may have lost any is summed again with
+// it, decided per entry from its own row of A and column of B, so that no
+// other row or column moves its bits:
+//  - a sum that is not finite (an infinity, a NaN or a value beyond turns the
+//    planes' sums into NaN; a sum may overflow);
+//  - a sum that a nonzero |x| < 2^-100 in its row or column may matter to.
+//    Such a value's planes are off by less than 2^-124 (planes below 2^-126
+//    may be flushed), its k products by 2^-124 k max|y| of the other operand's
+//    column or row. Sums of at least 2^26 times that keep theirs.
 #pragma once
 
 #include "common.hpp"
@@ -58,6 +64,44 @@ constexpr uint32_t kSplitTiny = 2u * ((127u - 100u) << 23) - 1u;
 __device__ __forceinline__ uint32_t split_min(uint32_t m, float x0, float x1) {
     const uint32_t t0 = (__float_as_uint(x0) << 1) - 1u, t1 = (__float_as_uint(x1) << 1) - 1u;
     return min(m, min(t0, t1));
+}
+
+// Largest magnitude seen, as 2 |x|.
+__device__ __forceinline__ uint32_t split_max(uint32_t m, float x0, float x1) {
+    return max(m, max(__float_as_uint(x0) << 1, __float_as_uint(x1) << 1));
+}
+// A row or column from its extents (least: split_min's, big: split_max's):
+// whether it holds a nonzero below 2^-100 (1 or 0), and its largest magnitude.
+__device__ __forceinline__ float2 split_line(uint32_t least, uint32_t big) {
+    return make_float2(least < kSplitTiny ? 1.0f : 0.0f, __uint_as_float(big >> 1));
+}
+// What such values may cost the sum of k products of a row and a column, times
+// 2^26. (0 times an infinite extent is NaN, taken for none: the sum is not
+// finite then.)
+__device__ __forceinline__ float split_loss(float2 row, float2 col, float k) {
+    return fmaxf(row.x * col.y, col.x * row.y) * (k * 0x1p-98f);
+}
+__device__ __forceinline__ bool split_lost(float sum, float loss) {
+    return !(fabsf(sum) < INFINITY) || fabsf(sum) < loss;
+}
+// A sum of exactly 0 where 0 < loss: one in some 2^24 sums cancels to that, and
+// has lost nothing if the magnitudes of its terms add up to the loss. The whole
+// wave asks for one entry; x(k) and y(k) are its row and column.
+template <class X, class Y>
+__device__ __forceinline__ bool split_cancelled(float2 row, float2 col, float loss, uint64_t k_begin, uint64_t k_end,
+                                                X x, Y y) {
+    // No terms can add up to the loss of values that small.
+    if ((row.x != 0.0f && row.y < 0x1p-98f) || (col.x != 0.0f && col.y < 0x1p-98f)) return false;
+    const int lane = threadIdx.x & 63;
+    float mine = 0.0f;
+    for (uint64_t k0 = k_begin; k0 < k_end; k0 += 64) {
+        const uint64_t k = k0 + lane;
+        if (k < k_end) mine += fabsf(x(k) * y(k));
+        if (__builtin_amdgcn_ballot_w64(mine >= loss)) return true;
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) mine += __shfl_xor(mine, off, 64);
+    return mine >= loss;
 }
 
 // Workgroup barrier that publishes LDS writes without waiting for the global
@@ -218,6 +262,54 @@ struct SplitOperand {
         else return (i & 1) ? bf16_hi(raw[2 * u + i / 2]) : bf16_lo(raw[2 * u + i / 2]);
     }
 
+    // The extents (split_min, split_max) of the tile's rows (columns) over k in
+    // [k_begin, k_end), into arrays in LDS: several stages' loads at a time, as
+    // the loop waits for nothing else.
+    template <int kAhead>
+    __device__ __forceinline__ void extents(uint64_t k_begin, uint64_t k_end, bool short_rows, uint32_t* least,
+                                            uint32_t* big) {
+        constexpr int kLines = KMAJOR ? kCols : kUnits;  // column i of a k-major thread, else unit i's row
+        uint32_t lo[kLines], hi[kLines];
+#pragma unroll
+        for (int i = 0; i < kLines; ++i) lo[i] = 0xFFFFFFFFu, hi[i] = 0;
+        auto gather = [&](const SplitOperand& o) {
+#pragma unroll
+            for (int u = 0; u < kUnits; ++u)
+#pragma unroll
+                for (int c = 0; c < kCols; ++c)
+#pragma unroll
+                    for (int i = 0; i < kUK; i += 2) {
+                        const float x0 = o.value(u, i, c), x1 = o.value(u, i + 1, c);
+                        lo[u + c] = split_min(lo[u + c], x0, x1);
+                        hi[u + c] = split_max(hi[u + c], x0, x1);
+                    }
+        };
+        uint64_t k0 = k_begin;
+        for (; short_rows && k0 + kAhead * BK <= k_end; k0 += kAhead * BK) {
+            SplitOperand ahead[kAhead];
+#pragma unroll
+            for (int d = 0; d < kAhead; ++d) {
+                ahead[d] = *this;
+#pragma unroll
+                for (int u = 0; u < kUnits; ++u) ahead[d].load(k0 + d * BK, u);
+            }
+#pragma unroll
+            for (int d = 0; d < kAhead; ++d) gather(ahead[d]);
+        }
+        for (; k0 < k_end; k0 += BK) {
+#pragma unroll
+            for (int u = 0; u < kUnits; ++u) load_edge(k0, k_end, u);
+            gather(*this);
+        }
+#pragma unroll
+        for (int i = 0; i < kLines; ++i) {
+            const int t = threadIdx.x;
+            const int row = KMAJOR ? t % (ROWS / kCols) * kCols + i : (t + i * THREADS) / (BK / 4);
+            atomicMin(least + row, lo[i]);
+            atomicMax(big + row, hi[i]);
+        }
+    }
+
     // Splits unit u and writes its planes to the stage at `lds`.
     __device__ __forceinline__ void store(char* lds, int u, uint32_t& tiny) const {
         const int t = threadIdx.x;
@@ -302,7 +394,7 @@ struct SplitTile {
     static constexpr int kMeetBytes = KG == 2 ? kWaves * kMI * kNI * 8 * 64 * 4 : 0;
     static constexpr int cmax(int a, int b) { return a > b ? a : b; }
     static constexpr int kLdsBytes =
-        cmax(kBufs * kStageBytes, cmax(OpA::kF32Bytes + OpB::kF32Bytes, kMeetBytes));
+        cmax(kBufs * kStageBytes, cmax(cmax(OpA::kF32Bytes + OpB::kF32Bytes, (BM + BN) * 16), kMeetBytes));
     static_assert(kLdsBytes <= 160 * 1024, "a workgroup's LDS");
     static_assert(KG == 1 || BK == 32, "each k group takes one 16 of a stage");
 
@@ -386,10 +478,12 @@ struct SplitTile {
     }
 
     // C[m0 .., n0 ..] summed over k in [k_begin, k_end) into acc (per k
-    // group). LDS is free on entry and on return.
-    __device__ __forceinline__ void sum(const float* __restrict__ A, const BT* __restrict__ B, uint64_t M,
+    // group) by the split's products; whether some of the sums in the workgroup
+    // are to be summed again (`again`: lost()). LDS is free on entry and on return.
+    __device__ __forceinline__ bool sum(const float* __restrict__ A, const BT* __restrict__ B, uint64_t M,
                                         uint64_t K, uint64_t N, uint64_t m0, uint64_t n0, uint64_t k_begin,
-                                        uint64_t k_end, bool wide_a, bool wide_b, bool short_rows, char* lds) {
+                                        uint64_t k_end, bool wide_a, bool wide_b, bool short_rows, char* lds,
+                                        uint32_t (&again)[(kMI * kNI * 16 + 31) / 32]) {
         const int lane = threadIdx.x & 63;
         const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
         const int kg = wave / kTileWaves, wt = wave % kTileWaves;
@@ -490,21 +584,140 @@ struct SplitTile {
             for (int j = 0; j < kNI; ++j)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(acc[i][j][r], 0.0f, probe);
-        if (!__syncthreads_or(tiny < kSplitTiny || probe != 0.0f)) return;
+        if (!__syncthreads_or(tiny < kSplitTiny || probe != 0.0f)) return false;
+        const bool any_tiny = __syncthreads_or(tiny < kSplitTiny);
+        return lost(A, B, M, K, N, m0, n0, k_begin, k_end, wide_a, wide_b, short_rows, any_tiny, lds, again);
+    }
 
-        // The f32 sum.
+    // The sums to be summed again, bit (i * kNI + j) * 16 + r of `again` for
+    // register r of block (i, j); whether the workgroup has any. With values
+    // below 2^-100 about (any_tiny) the extents of the tile's rows and columns
+    // are read first. 4096^3 with one such value in 64 of A: 802 us, 688 with
+    // none (1773 when such tiles were summed again, 985 on f32 MFMA kernels);
+    // with every value of A at 1e-35, whose sums need it, 1875.
+    static constexpr int kExtentsAhead = kMI * kNI >= 8 ? 2 : 4;  // (registers)
+    static constexpr int kWords = (kMI * kNI * 16 + 31) / 32;
+    using Mask = uint32_t[kWords];
+    __device__ __forceinline__ bool lost(const float* __restrict__ A, const BT* __restrict__ B, uint64_t M,
+                                         uint64_t K, uint64_t N, uint64_t m0, uint64_t n0, uint64_t k_begin,
+                                         uint64_t k_end, bool wide_a, bool wide_b, bool short_rows, bool any_tiny,
+                                         char* lds, Mask& again) {
+        uint32_t* const least_a = reinterpret_cast<uint32_t*>(lds);
+        uint32_t* const big_a = least_a + BM;
+        uint32_t* const least_b = big_a + BM;
+        uint32_t* const big_b = least_b + BN;
+        float2* const lines = reinterpret_cast<float2*>(big_b + BN);
+        if (any_tiny) {
+            for (int i = threadIdx.x; i < BM; i += kThreads) least_a[i] = 0xFFFFFFFFu, big_a[i] = 0;
+            for (int i = threadIdx.x; i < BN; i += kThreads) least_b[i] = 0xFFFFFFFFu, big_b[i] = 0;
+            __syncthreads();
+            OpA oa;
+            oa.init(A, A_T ? M : K, m0, M, wide_a);
+            oa.template extents<kExtentsAhead>(k_begin, k_end, short_rows, least_a, big_a);
+            OpB ob;
+            ob.init(B, B_T ? K : N, n0, N, wide_b);
+            ob.template extents<kExtentsAhead>(k_begin, k_end, short_rows, least_b, big_b);
+            __syncthreads();
+            for (int i = threadIdx.x; i < BM; i += kThreads) lines[i] = split_line(least_a[i], big_a[i]);
+            for (int i = threadIdx.x; i < BN; i += kThreads) lines[BM + i] = split_line(least_b[i], big_b[i]);
+            __syncthreads();
+        }
+        const int lane = threadIdx.x & 63;
+        const int wt = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)) % kTileWaves;
+        const int row0 = wt / kWavesN * WM + 4 * (lane >> 5), col0 = wt % kWavesN * WN + (lane & 31);
+        const float count = static_cast<float>(k_end - k_begin);
+        float2 col[kNI];
+#pragma unroll
+        for (int j = 0; j < kNI; ++j) col[j] = any_tiny ? lines[BM + col0 + j * 32] : make_float2(0.f, 0.f);
+        Mask zero;
+#pragma unroll
+        for (int w = 0; w < kWords; ++w) again[w] = zero[w] = 0;
+#pragma unroll
+        for (int i = 0; i < kMI; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float2 row = any_tiny ? lines[row0 + i * 32 + 8 * (r / 4) + r % 4] : make_float2(0.f, 0.f);
+#pragma unroll
+                for (int j = 0; j < kNI; ++j) {
+                    const int bit = (i * kNI + j) * 16 + r;
+                    const float sum = acc[i][j][r];
+                    const bool is = split_lost(sum, split_loss(row, col[j], count));
+                    again[bit / 32] |= (is ? 1u : 0u) << bit % 32;
+                    zero[bit / 32] |= (is && sum == 0.0f ? 1u : 0u) << bit % 32;
+                }
+                // (All of the rows and comparisons at once spill.)
+#pragma unroll
+                for (int w = 0; w < kWords; ++w)
+                    __asm__ volatile("" : "+v"(again[w]), "+v"(zero[w]) : : "memory");
+            }
+        // The zeros one at a time, lane by lane.
+#pragma unroll
+        for (int w = 0; w < kWords; ++w)
+            for (uint64_t lanes; (lanes = __builtin_amdgcn_ballot_w64(zero[w] != 0)) != 0;) {
+                const int l = __builtin_ctzll(lanes);
+                const uint32_t mask = __builtin_amdgcn_readlane(static_cast<int>(zero[w]), l);
+                const int bit = w * 32 + __builtin_ctz(mask), r = bit % 16;
+                const int row = wt / kWavesN * WM + bit / 16 / kNI * 32 + 8 * (r / 4) + 4 * (l >> 5) + r % 4;
+                const int column = wt % kWavesN * WN + bit / 16 % kNI * 32 + (l & 31);
+                const float2 row_line = lines[row], col_line = lines[BM + column];
+                const uint64_t m = min(m0 + row, M - 1), n = min(n0 + column, N - 1);
+                const bool kept = split_cancelled(
+                    row_line, col_line, split_loss(row_line, col_line, count), k_begin, k_end,
+                    [&](uint64_t k) { return A_T ? A[k * M + m] : A[m * K + k]; },
+                    [&](uint64_t k) { return elem(B + (B_T ? n * K + k : k * N + n)); });
+                if (lane == l) {
+                    zero[w] &= zero[w] - 1;
+                    if (kept) again[w] &= ~(1u << bit % 32);
+                }
+            }
+        uint32_t any = 0;
+#pragma unroll
+        for (int w = 0; w < kWords; ++w) any |= again[w];
+        return __syncthreads_or(any != 0);  // (LDS is free again)
+    }
+
+    // The same sums with the f32 MFMA.
+    __device__ __forceinline__ void sum_f32(const float* __restrict__ A, const BT* __restrict__ B, uint64_t M,
+                                            uint64_t K, uint64_t N, uint64_t m0, uint64_t n0, uint64_t k_begin,
+                                            uint64_t k_end, bool wide_a, bool wide_b, bool short_rows, char* lds) {
+        const int lane = threadIdx.x & 63;
+        const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+        const int kg = wave / kTileWaves, wt = wave % kTileWaves;
+        const int wm = wt / kWavesN, wn = wt % kWavesN;
+        OpA oa;
+        OpB ob;
+        oa.init(A, A_T ? M : K, m0, M, wide_a);
+        ob.init(B, B_T ? K : N, n0, N, wide_b);
         clear();
         float* const fa = reinterpret_cast<float*>(lds);
         float* const fb = reinterpret_cast<float*>(lds + OpA::kF32Bytes);
         const int l32 = lane & 31, h = lane >> 5;
+        // A stage's loads are in flight while the one before is summed, where
+        // the registers allow it.
+        constexpr bool kAhead = kMI * kNI < 8;
+        auto load = [&](uint64_t k0) {
+            if (short_rows && k0 + BK <= k_end) {
+#pragma unroll
+                for (int u = 0; u < OpA::kUnits; ++u) oa.load(k0, u);
+#pragma unroll
+                for (int u = 0; u < OpB::kUnits; ++u) ob.load(k0, u);
+            } else {
+#pragma unroll
+                for (int u = 0; u < OpA::kUnits; ++u) oa.load_edge(k0, k_end, u);
+#pragma unroll
+                for (int u = 0; u < OpB::kUnits; ++u) ob.load_edge(k0, k_end, u);
+            }
+        };
+        if (kAhead) load(k_begin);
         for (uint64_t k0 = k_begin; k0 < k_end; k0 += BK) {
-            if (short_rows && k0 + BK <= k_end) load(k0);
-            else load_edge(k0);
+            if (!kAhead) load(k0);
 #pragma unroll
             for (int u = 0; u < OpA::kUnits; ++u) oa.store_f32(fa, u);
 #pragma unroll
             for (int u = 0; u < OpB::kUnits; ++u) ob.store_f32(fb, u);
-            __syncthreads();
+            lds_barrier<0>();
+            if (kAhead && k0 + BK < k_end) load(k0 + BK);
+#pragma unroll 1
             for (int s = 0; s < BK / KG; s += 2) {
                 const int k = kg * (BK / KG) + s + h;
                 float af[kMI], bf[kNI];
@@ -518,7 +731,7 @@ struct SplitTile {
                     for (int j = 0; j < kNI; ++j)
                         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i], bf[j], acc[i][j], 0, 0, 0);
             }
-            __syncthreads();
+            lds_barrier<0>();
         }
     }
 };

@@ -1,7 +1,8 @@
 """GPU: the f32 products summed as bf16 plane products (csrc/split_tile.hpp),
 one shape per tile configuration, at the values where the split does not hold:
 infinities, NaN, the largest and the smallest f32, and rows so small that
-their planes would underflow. Such tiles are summed again with the f32 MFMA.
+their planes would underflow. The sums that these may matter to, and no other,
+are summed again with the f32 MFMA.
 
 Bound, entry by entry: |C - C64| <= (k + 8) u (|A| |B|) with u = 2^-24, the
 forward-error bound of any order of f32 additions (Higham, Accuracy and
@@ -106,3 +107,51 @@ def test_compact_weights_give_the_f32_bits(dev, m, k, n):
         got = ops.matmul_bf16w(dev, da, dev.upload(bits)).numpy()
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
         check(want, a, wide)
+
+
+# One shape per tile configuration, k split over workgroups, stream-K, row panels.
+PLACES = SHAPES[:5] + [(509, 1100, 1500), (192, 3072, 5120), (512, 1024, 11008), (20, 480, 640), (31, 200, 258)]
+
+
+@pytest.mark.parametrize("m,k,n", PLACES)
+@pytest.mark.parametrize("value", [np.inf, np.nan, 3.4e38, 1e-44])
+def test_a_value_moves_its_own_row_and_column_only(dev, m, k, n, value):
+    """The other entries keep the bits they have without it."""
+    from magnetar_hip import ops
+    a, b = operands(m, k, n, m + 23)
+    want = ops.matmul(dev, dev.upload(a), dev.upload(b)).numpy().view(np.uint32)
+    row, col = m // 3, n // 2
+    a[row, k // 2] = b[k // 3, col] = value
+    got = ops.matmul(dev, dev.upload(a), dev.upload(b)).numpy().view(np.uint32)
+    others = np.ones((m, n), bool)
+    others[row, :] = others[:, col] = False
+    assert np.array_equal(got[others], want[others])
+
+
+@pytest.mark.parametrize("m,k,n", PLACES)
+@pytest.mark.parametrize("tiny", [1e-31, 1e-35, 1e-42])
+def test_a_tiny_value_that_cannot_matter_sums_nothing_again(dev, m, k, n, tiny):
+    """Values below 2^-100 among ordinary ones: the bits are those with zeros
+    in their place (the f32 MFMA's sums differ in their rounding)."""
+    from magnetar_hip import ops
+    a, b = operands(m, k, n, m + 29)
+    got = []
+    for value in (0.0, tiny):
+        a.reshape(-1)[:: 61] = value
+        b[k // 2, 1::7] = value
+        got.append(ops.matmul(dev, dev.upload(a), dev.upload(b)).numpy().view(np.uint32))
+    assert np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("m,k,n", [(20, 480, 640), (31, 200, 258)])
+@pytest.mark.parametrize("down", [-100, -108, -120])
+@pytest.mark.parametrize("compact", [False, True])
+def test_small_rows_of_a_panel_keep_their_precision(dev, m, k, n, down, compact):
+    from magnetar_hip import ops
+    a, b = operands(m, k, n, m + 31)
+    a[::3] *= np.float32(2.0 ** down)
+    b = (b * np.float32(2.0 ** 90)).view(np.uint32) & np.uint32(0xFFFF0000)
+    half = (b >> 16).astype(np.uint16)
+    b = b.view(np.float32)
+    da = dev.upload(a)
+    check(ops.matmul_bf16w(dev, da, dev.upload(half)).numpy() if compact else ops.matmul(dev, da, dev.upload(b)).numpy(), a, b)
