@@ -143,7 +143,7 @@ __global__ __launch_bounds__(64 * kPanelWaves, 4) void panel_kernel(
         if (tiny_a < kSplitTiny) redo = any_tiny = 1;
     };
     uint32_t raw[kPanelDepth][8];
-    if (threadIdx.x == 0) redo = any_tiny = 0;
+    if (threadIdx.x == 0) redo = K < kSplitMinK, any_tiny = 0;
     // A's first chunk ahead of an f32 B: loads come back in order, so behind
     // B's it would wait for all of them (as the next chunks do). With 384 k a
     // chunk 24 x 4096 x 11008 44.8 -> 42.9 us, 32 x 11008 x 4096 51 -> 48.
@@ -307,6 +307,7 @@ __global__ __launch_bounds__(64 * kPanelWaves, 4) void panel_kernel(
                 if (kept) again &= ~(1u << bit);
             }
         }
+        if (K < kSplitMinK) again = 0xFFFFFFFFu;
         if (__builtin_amdgcn_ballot_w64(again != 0)) {
             f32x16 first[kBlocks];
 #pragma unroll

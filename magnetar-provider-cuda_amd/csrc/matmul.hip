@@ -152,8 +152,15 @@ __device__ __forceinline__ void gemm_tile(const float* __restrict__ A, const BT*
     using Tile = typename Shape::template Tile<A_T, B_T, BT>;
     Tile tile;
     typename Tile::Mask again;
-    const bool redo = tile.sum(A, B, M, K, N, m0, n0, k_begin, k_end, access.wide_a, access.wide_b,
-                               access.short_rows, lds, again);
+    bool redo = true;
+    if (K >= mhip::kSplitMinK) {
+        redo = tile.sum(A, B, M, K, N, m0, n0, k_begin, k_end, access.wide_a, access.wide_b, access.short_rows, lds,
+                        again);
+    } else {
+        tile.clear();
+#pragma unroll
+        for (int w = 0; w < Tile::kWords; ++w) again[w] = 0xFFFFFFFFu;
+    }
     auto sum_again = [&]() {
         tile.sum_f32(A, B, M, K, N, m0, n0, k_begin, k_end, access.wide_a, access.wide_b, access.short_rows, lds);
     };

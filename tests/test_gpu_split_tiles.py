@@ -6,9 +6,10 @@ are summed again with the f32 MFMA.
 
 Bound, entry by entry: |C - C64| <= (k + 8) u (|A| |B|) with u = 2^-24, the
 forward-error bound of any order of f32 additions (Higham, Accuracy and
-Stability of Numerical Algorithms, eq. 3.5) plus 8 u for the split (its
-dropped products are below 4 u / 16 of |A| |B|, its planes exact) and the
-first-order bound's remainder. Entries that are not finite in f64 rounded to
+Stability of Numerical Algorithms, eq. 3.5) plus 8 u for the split (its planes
+are exact, its dropped products a2 b3 + a3 b2 + a3 b3 below 1.01 u of |A| |B|:
+|x2| <= 2^-8 |x|, |x3| <= 2^-17 |x|; six roundings a product where there are
+few) and the first-order bound's remainder. Entries that are not finite in f64 rounded to
 f32 are compared exactly.
 """
 import numpy as np
@@ -155,3 +156,37 @@ def test_small_rows_of_a_panel_keep_their_precision(dev, m, k, n, down, compact)
     b = b.view(np.float32)
     da = dev.upload(a)
     check(ops.matmul_bf16w(dev, da, dev.upload(half)).numpy() if compact else ops.matmul(dev, da, dev.upload(b)).numpy(), a, b)
+
+
+@pytest.mark.parametrize("m,n", [(70, 70), (64, 2050), (2000, 2030), (4000, 4060), (20, 640), (9, 2), (31, 258)])
+@pytest.mark.parametrize("compact", [False, True])
+def test_one_and_two_products_keep_the_f32_error(dev, m, n, compact):
+    """k 1 is a single rounded product, k 2 at most two products and a sum
+    (an fma chain rounds less): bit for bit, and within 3 u of the terms."""
+    from magnetar_hip import ops
+    for k in (1, 2):
+        a, b = operands(m, k, n, m + 37)
+        if compact:
+            b = (b.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
+        half = (b.view(np.uint32) >> 16).astype(np.uint16)
+        da = dev.upload(a)
+        got = ops.matmul_bf16w(dev, da, dev.upload(half)).numpy() if compact else ops.matmul(dev, da, dev.upload(b)).numpy()
+        if k == 1:
+            assert np.array_equal(got.view(np.uint32), (a * b).view(np.uint32))
+        scale = np.abs(a).astype(np.float64) @ np.abs(b)
+        assert np.all(np.abs(got - a.astype(np.float64) @ b.astype(np.float64)) <= k * 1.5 * 2.0 ** -24 * scale)
+
+
+WORST = np.float32(1 + 2.0 ** -8 - 2.0 ** -17)  # its square's dropped products are 0.99 u of it
+
+
+@pytest.mark.parametrize("m,k,n", [(70, 1, 70), (70, 3, 70), (2000, 16, 2030), (20, 3, 640), (4000, 72, 4060), (20, 480, 640),
+                                   (300, 4096, 300)])
+def test_operands_whose_dropped_products_are_largest(dev, m, k, n):
+    """Every dropped product of the same sign and as large as any. Nothing but
+    their sum and the rounding of the kept ones: (k / 16 * 6 + 2) u of the sum."""
+    from magnetar_hip import ops
+    a, b = np.full((m, k), WORST), np.full((k, n), WORST)
+    got = ops.matmul(dev, dev.upload(a), dev.upload(b)).numpy()
+    exact = k * np.float64(WORST) ** 2
+    assert np.all(np.abs(got - exact) <= (k / 16 * 6 + 2) * 2.0 ** -24 * exact)
