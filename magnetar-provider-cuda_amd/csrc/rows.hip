@@ -280,22 +280,26 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_loop_kernel(
 }
 
 // Rows that softmax_vec_kernel does not take -- longer than 16384, or no whole
-// 16-byte vectors -- on one workgroup of T threads each: E vectors of V floats
-// per thread, all loaded before any is used, then as softmax_vec_kernel. A
-// loop that read the row three times with one load in flight per thread took
-// 59-93 us for one row of 32000 (a vocabulary), 526 for 4096 of them and 90 for
-// 8192 rows of 4095; this takes 9, 201 and 43.
+// 16-byte vectors -- on T threads each (a wave of several in a workgroup, or a
+// workgroup): E vectors of V floats per thread, all loaded before any is used,
+// then as softmax_vec_kernel. A loop that read the row three times with one
+// load in flight per thread took 59-93 us for one row of 32000 (a vocabulary),
+// 526 for 4096 of them and 90 for 8192 rows of 4095; this takes 9, 201 and 43.
+// Short rows on a workgroup each took 167 us for 131072 rows of 31 (92 in that
+// loop) and 139 for 8192 of 4097 on 1024 threads (89); now 25 and 49.
 template <int T, int V, int E>
-__global__ __launch_bounds__(T) void softmax_wide_kernel(const float* in, float* out, uint64_t cols,
-                                                         uint32_t* flags) {
+__global__ __launch_bounds__(T < 256 ? 256 : T) void softmax_wide_kernel(const float* in, float* out, uint64_t rows,
+                                                                         uint64_t cols, uint32_t* flags) {
     __shared__ float2 scratch[T / 64];
-    const uint64_t row = blockIdx.x;
+    const int thread = threadIdx.x % T;
+    const uint64_t row = T < 256 ? blockIdx.x * static_cast<uint64_t>(256 / T) + threadIdx.x / T : blockIdx.x;
+    if (T < 256 && row >= rows) return;
     const float* x = in + row * cols;
     float v[E][V];
     float mt = -INFINITY;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-        const uint64_t c = (threadIdx.x + static_cast<uint64_t>(e) * T) * V;
+        const uint64_t c = (thread + static_cast<uint64_t>(e) * T) * V;
 #pragma unroll
         for (int i = 0; i < V; ++i) v[e][i] = -INFINITY;
         if (c < cols) {
@@ -311,6 +315,8 @@ __global__ __launch_bounds__(T) void softmax_wide_kernel(const float* in, float*
     for (int e = 0; e < E; ++e)
 #pragma unroll
         for (int i = 0; i < V; ++i) mt = fmaxf(mt, v[e][i]);
+    // (A wave's own row: its maximum costs less than merging 64 states.)
+    if constexpr (T == 64) mt = wave_reduce(mt, mhip::MaxOp{});
     const float base = mt == -INFINITY ? 0.0f : mt;
     float st = 0.0f;
 #pragma unroll
@@ -321,16 +327,17 @@ __global__ __launch_bounds__(T) void softmax_wide_kernel(const float* in, float*
             st += v[e][i];
         }
     float M = mt, S = st;
-    block_merge<T>(M, S, scratch);
+    if constexpr (T == 64) S = wave_reduce(S, SumOp{});
+    else block_merge<T>(M, S, scratch);
     if (!isfinite(M)) {
-        if (threadIdx.x == 0) atomicOr(flags, MHIP_FLAG_SOFTMAX_NON_FINITE);
+        if (thread == 0) atomicOr(flags, MHIP_FLAG_SOFTMAX_NON_FINITE);
         return;
     }
     const float scale = expf(mt - M) * (1.0f / S);
     float* y = out + row * cols;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-        const uint64_t c = (threadIdx.x + static_cast<uint64_t>(e) * T) * V;
+        const uint64_t c = (thread + static_cast<uint64_t>(e) * T) * V;
         if (c >= cols) continue;
         if constexpr (V == 4)
             *reinterpret_cast<float4*>(y + c) =
@@ -488,17 +495,24 @@ mhip_status mhip_softmax_rows_f32(mhip_ctx* ctx, const float* in, float* out, ui
     const bool vec = cols % 4 == 0 && mhip::aligned16(in) && mhip::aligned16(out);
     if (vec && dispatch_vec<RowKind::Softmax>(ctx, rows, in, nullptr, out, cols, 0, 0.0f))
         return mhip::check_launch("softmax");
-    const dim3 grid(static_cast<unsigned>(rows));
-    // The fewest registers per thread that hold the row; unaligned rows of more
-    // than 32 floats a thread would spill.
-    auto wide = [&](auto kernel, int threads) { mhip::launch(ctx, kernel, grid, dim3(threads), 0, in, out, cols, ctx->flags); };
-    if (vec && cols <= 1024 * 4 * 8) wide(softmax_wide_kernel<1024, 4, 8>, 1024);
-    else if (vec && cols <= 1024 * 4 * 16) wide(softmax_wide_kernel<1024, 4, 16>, 1024);
-    else if (cols <= 256 * 4) wide(softmax_wide_kernel<256, 1, 4>, 256);
-    else if (cols <= 256 * 16) wide(softmax_wide_kernel<256, 1, 16>, 256);
-    else if (cols <= 1024 * 16) wide(softmax_wide_kernel<1024, 1, 16>, 1024);
-    else if (cols <= 1024 * 32) wide(softmax_wide_kernel<1024, 1, 32>, 1024);
-    else wide(softmax_loop_kernel, 1024);
+    // The fewest threads, then registers, that hold the row; unaligned rows of
+    // more than 32 floats a thread would spill.
+    auto wide = [&](auto kernel, int threads, int row_threads) {
+        const dim3 grid(static_cast<unsigned>(mhip::ceil_div(rows, threads / row_threads)));
+        mhip::launch(ctx, kernel, grid, dim3(threads), 0, in, out, rows, cols, ctx->flags);
+    };
+    if (vec && cols <= 1024 * 4 * 8) wide(softmax_wide_kernel<1024, 4, 8>, 1024, 1024);
+    else if (vec && cols <= 1024 * 4 * 16) wide(softmax_wide_kernel<1024, 4, 16>, 1024, 1024);
+    else if (cols <= 64) wide(softmax_wide_kernel<64, 1, 1>, 256, 64);
+    else if (cols <= 64 * 4) wide(softmax_wide_kernel<64, 1, 4>, 256, 64);
+    else if (cols <= 64 * 8) wide(softmax_wide_kernel<64, 1, 8>, 256, 64);
+    else if (cols <= 64 * 16) wide(softmax_wide_kernel<64, 1, 16>, 256, 64);
+    else if (cols <= 256 * 8) wide(softmax_wide_kernel<256, 1, 8>, 256, 256);
+    else if (cols <= 256 * 16) wide(softmax_wide_kernel<256, 1, 16>, 256, 256);
+    else if (cols <= 256 * 32) wide(softmax_wide_kernel<256, 1, 32>, 256, 256);
+    else if (cols <= 1024 * 16) wide(softmax_wide_kernel<1024, 1, 16>, 1024, 1024);
+    else if (cols <= 1024 * 32) wide(softmax_wide_kernel<1024, 1, 32>, 1024, 1024);
+    else mhip::launch(ctx, softmax_loop_kernel, dim3(static_cast<unsigned>(rows)), dim3(1024), 0, in, out, cols, ctx->flags);
     return mhip::check_launch("softmax");
 }
 

@@ -96,11 +96,16 @@ WIDTHS = [1, 63, 255, 1023, 1025, 4095, 4097, 16383, 16385, 16388, 32768, 32772,
           128000]
 
 
-@pytest.mark.parametrize("cols", WIDTHS)
-def test_softmax_of_wide_and_ragged_rows(dev, cols):
+# Around the edges of the rows that a wave, several of it in a workgroup, or a
+# small workgroup holds.
+SHORT = [2, 65, 257, 509, 513, 2047, 2049, 8191, 8193]
+
+
+@pytest.mark.parametrize("cols,rows", [(c, 3) for c in WIDTHS] + [(c, 9) for c in SHORT])
+def test_softmax_of_wide_and_ragged_rows(dev, cols, rows):
     from magnetar_hip import ops
     rng = np.random.default_rng(cols)
-    x = (4 * rng.standard_normal((3, cols))).astype(np.float32)
+    x = (4 * rng.standard_normal((rows, cols))).astype(np.float32)
     if cols > 2:
         x[1, : cols // 2] = -np.inf
         x[2, cols - 1] = 80.0
@@ -116,7 +121,7 @@ def test_softmax_of_wide_and_ragged_rows(dev, cols):
     assert np.array_equal(d.numpy().view(np.uint32), got.view(np.uint32))
 
 
-@pytest.mark.parametrize("cols", WIDTHS[3:])
+@pytest.mark.parametrize("cols", WIDTHS[3:] + SHORT[1:])
 def test_softmax_keeps_nan_and_flags_rows_without_a_finite_entry(dev, cols):
     import magnetar_hip
     from magnetar_hip import ops
