@@ -1676,8 +1676,17 @@ TileChoice choose_tiles(const mhip_ctx* ctx, uint64_t m, uint64_t k, uint64_t n)
 bool ragged_gemv_fits(uint64_t m, uint64_t n, bool ta, bool tb) {
     return m <= kGemvMaxRows && !ta && !tb && m * n < (1ULL << 31);
 }
+// A wave's lanes run along k: a short k leaves them idle before many outputs'
+// butterflies (8 x 32 x 11008 9.1 us, tiles 4.8; 8 x 128 x 11008 9.4 and 7.9; 8
+// x 128 x 4096 5.2 and 6.1), and where a few hundred columns give each CU hardly
+// a wave, a very long k is a chain of its loads (8 x 65536 x 256 149, tiles 75;
+// 3 x 65536 x 256 109 and 74). Both sides measured over m 1-8, k 32-65536, n
+// 32-32000.
 bool dot_fits(uint64_t m, uint64_t k, uint64_t n, bool ta, bool tb, bool b_aligned) {
-    return m <= kGemvMaxRows && !ta && tb && k % 8 == 0 && b_aligned && n < (1ULL << 31);
+    const bool lanes = m == 1 || k >= 256 || m * n <= std::max<uint64_t>(512 * k, 24576);
+    const bool chain = k > (m <= 4 && n >= 128 ? 32768 : n >= 128 ? 16384 : m <= 4 ? UINT64_MAX : 32768);
+    return m <= kGemvMaxRows && !ta && tb && k % 8 == 0 && b_aligned && n < (1ULL << 31) && lanes &&
+           !(chain && n < 1024);
 }
 // (Pairs of a compact B's columns; 32-bit offsets over 16 rows of B.)
 bool panel_fits(uint64_t m, uint64_t n, bool ta, bool tb) {

@@ -58,6 +58,13 @@ def test_row_dots(dev, m, k, n):
     check_products(dev, m, k, n, True, "row_dots")
 
 
+@pytest.mark.parametrize("m,k,n,path", [(1, 32, 32001, "row_dots"), (3, 32, 8193, "tiles"), (8, 128, 8193, "tiles"),
+                                        (8, 128, 8192, "row_dots"), (8, 16392, 130, "tiles"), (8, 16384, 130, "row_dots"),
+                                        (4, 32768, 128, "row_dots"), (5, 32776, 33, "tiles")])
+def test_row_dots_where_they_are_faster(dev, m, k, n, path):
+    check_products(dev, m, k, n, True, path)
+
+
 @pytest.mark.parametrize("m,k,n", [(9, 1, 2), (9, 15, 30), (10, 257, 258), (17, 1000, 510), (31, 4100, 514),
                                    (32, 4096, 11008), (25, 2050, 4098), (12, 33, 32),
                                    (30, 65, 4094)])
