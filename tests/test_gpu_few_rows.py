@@ -47,7 +47,7 @@ def check_products(dev, m, k, n, tb, path, poison=None):
 
 
 @pytest.mark.parametrize("m", [1, 2, 5, 8])
-@pytest.mark.parametrize("k,n", [(1, 1), (31, 255), (4096, 257), (1030, 1029), (300, 50257)])
+@pytest.mark.parametrize("k,n", [(1, 1), (31, 255), (64, 33), (65, 33), (4096, 257), (1030, 1029), (300, 50257)])
 def test_ragged_gemv(dev, m, k, n):
     check_products(dev, m, k, n, False, "gemv_ragged")
 
