@@ -426,11 +426,76 @@ __global__ __launch_bounds__(256) void splitk_reduce_scalar_kernel(const float* 
     C[e] = v;
 }
 
+// The same for many splits of few outputs (row panels and ragged GEMVs of a
+// long k): 16 waves of 64 V outputs each add a run of the splits in order, eight
+// loads in flight, and the runs meet in LDS, in order. What bounds it: the
+// chain of loads. 17 x 65536 x 256, 512 splits: the product 151 us with a
+// thread per output running through all of them, 28 so.
+constexpr int kDeepWaves = 16;
+template <int V>
+__global__ __launch_bounds__(64 * kDeepWaves) void splitk_reduce_deep_kernel(const float* __restrict__ partial,
+                                                                             float* __restrict__ C, uint64_t M,
+                                                                             uint64_t N, uint32_t splits,
+                                                                             const float* __restrict__ addend,
+                                                                             int addend_mode) {
+    __shared__ float red[kDeepWaves][V][64];
+    const uint64_t total = M * N;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint64_t e = (static_cast<uint64_t>(blockIdx.x) * 64 + lane) * V;
+    const uint32_t run = (splits + kDeepWaves - 1) / kDeepWaves;
+    const uint32_t s0 = min(splits, wave * run), s1 = min(splits, s0 + run);
+    float v[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) v[i] = 0.0f;
+    if (e < total) {  // (V 4: whole vectors)
+        constexpr int kU = 8;
+        for (uint32_t s = s0; s < s1; s += kU) {
+            float p[kU][V];
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                const float* const at = partial + min(s + u, s1 - 1) * total + e;
+                if constexpr (V == 4) {
+                    const float4 t = *reinterpret_cast<const float4*>(at);
+                    p[u][0] = t.x; p[u][1] = t.y; p[u][2] = t.z; p[u][3] = t.w;
+                } else {
+                    p[u][0] = *at;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+#pragma unroll
+                for (int i = 0; i < V; ++i)
+                    if (s + u < s1) v[i] += p[u][i];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i) red[wave][i][lane] = v[i];
+    __syncthreads();
+    if (wave != 0 || e >= total) return;
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        float t = red[0][i][lane];
+#pragma unroll
+        for (int w = 1; w < kDeepWaves; ++w) t += red[w][i][lane];
+        if (addend_mode == 1) t = t + addend[(e + i) % N];
+        else if (addend_mode >= 2) t = apply_addend(t, addend[e + i], addend_mode);
+        v[i] = t;
+    }
+    if constexpr (V == 4) *reinterpret_cast<float4*>(C + e) = make_float4(v[0], v[1], v[2], v[3]);
+    else C[e] = v[0];
+}
+
 // Adds a product's partial results (splits of m x n at `partial`) into c.
 mhip_status launch_splitk_reduce(mhip_ctx* ctx, const float* partial, float* c, uint64_t m, uint64_t n,
                                  uint64_t splits, const float* addend, int mode, const char* what) {
     // dwordx4: whole rows of 4 and 16-byte aligned output and addend.
-    if (n % 4 == 0 && mhip::aligned16(c) && (mode == 0 || mhip::aligned16(addend)))
+    const bool vec = n % 4 == 0 && mhip::aligned16(c) && (mode == 0 || mhip::aligned16(addend));
+    if (splits >= 64) {
+        const uint64_t per = vec ? 256 : 64;
+        mhip::launch(ctx, vec ? splitk_reduce_deep_kernel<4> : splitk_reduce_deep_kernel<1>,
+                     dim3(static_cast<unsigned>((m * n + per - 1) / per)), dim3(64 * kDeepWaves), 0, partial, c, m, n,
+                     static_cast<uint32_t>(splits), addend, mode);
+    } else if (vec)
         mhip::launch(ctx, splitk_reduce_kernel, dim3(static_cast<unsigned>((m * n + 1023) / 1024)), dim3(256), 0,
                      partial, c, m, n, static_cast<uint32_t>(splits), addend, mode);
     else

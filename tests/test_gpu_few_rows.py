@@ -72,6 +72,15 @@ def test_row_panel(dev, m, k, n):
     check_products(dev, m, k, n, False, "row_panel")
 
 
+# 64 and more partial results of a long k, whole vectors of them and not.
+@pytest.mark.parametrize("m,k,n,path", [(17, 8200, 66, "row_panel"), (9, 9000, 64, "row_panel"), (32, 65536, 130, "row_panel"),
+                                        (3, 20000, 7, "gemv_ragged"), (8, 2049, 253, "gemv_ragged")])
+def test_sums_of_many_slices(dev, m, k, n, path):
+    from magnetar_hip import ops
+    assert ops.matmul_plan(dev, m, k, n)["splits"] >= 64
+    check_products(dev, m, k, n, False, path)
+
+
 @pytest.mark.parametrize("poison", [np.inf, np.nan, -3.4e38, 1e-44])
 @pytest.mark.parametrize("m,k,n,tb,path", [(9, 100, 258, False, "row_panel"), (31, 1030, 600, False, "row_panel"),
                                            (2, 520, 100, True, "row_dots"), (4, 77, 99, False, "gemv_ragged")])
