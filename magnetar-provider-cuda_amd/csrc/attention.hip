@@ -284,12 +284,17 @@ __device__ __forceinline__ PrefillPlace prefill_place(const AttnArgs& a, const P
     return w;
 }
 
+// The keys [rel_lo, rel_hi) of a tile of 32, a bit each.
+__device__ __forceinline__ uint32_t tile_keys(int rel_lo, int rel_hi) {
+    const int lo = min(max(rel_lo, 0), 32), hi = min(max(rel_hi, 0), 32);
+    return static_cast<uint32_t>(((1ull << hi) - 1ull) & ~((1ull << lo) - 1ull));
+}
+
 // One tile's masked scores: s[r] is key k0 + 8 (r / 4) + 4 half + r % 4 of the
 // lane's query, -inf where it is not admitted (rel_lo, rel_hi: its admitted
 // keys from the tile's first).
 __device__ __forceinline__ void mask_scores(v16f& s, int rel_lo, int rel_hi, int half) {
-    const int lo = min(max(rel_lo, 0), 32), hi = min(max(rel_hi, 0), 32);
-    const uint32_t mine = static_cast<uint32_t>(((1ull << hi) - 1ull) & ~((1ull << lo) - 1ull)) >> (4 * half);
+    const uint32_t mine = tile_keys(rel_lo, rel_hi) >> (4 * half);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int key = 8 * (r / 4) + (r % 4);
@@ -335,8 +340,9 @@ __device__ __forceinline__ float softmax_tile_mean(v16f& s, float& m, float& l) 
 }
 
 // The workgroup's tiles [i_begin, i_end) with the f32 MFMA, for the waves
-// (`again`) that met inputs outside the bf16 split: values that are not
-// finite, scores' operands above 2^60, scaled values below 2^-100. Q is read
+// (`again`) with outputs that the bf16 split does not hold: values that are not
+// finite, scores' operands above 2^60, outputs that scaled values below 2^-100
+// matter to. Q is read
 // from memory, K and V tiles lie in LDS; a key that one query masks and another
 // admits enters P . V at weight 0, so a wave that met a V value that is not
 // finite in an edge tile sums its queries' admitted keys again on the VALU
@@ -518,9 +524,14 @@ __global__ __launch_bounds__(PrefillCfg<D>::kThreads, 2) void attn_prefill_kerne
         load_v(i_begin);
     }
     SplitRange query;
-    // Whether a tile (by parity) holds K or V outside the split.
-    __shared__ int outside[2];
-    if (threadIdx.x < 2) outside[threadIdx.x] = 0;
+    // A tile's (by parity) keys whose K is outside the split, and whether some V
+    // of it is not finite; the value columns with a nonzero below 2^-100 (scaled).
+    __shared__ uint32_t far_keys[2];
+    __shared__ int bad_values[2], any_tiny;
+    __shared__ uint8_t tiny_values[Cfg::kVB * 32];
+    if (threadIdx.x < 2) far_keys[threadIdx.x] = bad_values[threadIdx.x] = 0;
+    if (threadIdx.x == 2) any_tiny = 0;
+    if (threadIdx.x < Cfg::kVB * 32) tiny_values[threadIdx.x] = 0;
 
     // Q^T's planes, pre-scaled: step t, k = 16 t + 8 half + i of the query.
     constexpr int kQRegs = Cfg::kQLds ? 2 : 3;
@@ -547,14 +558,15 @@ __global__ __launch_bounds__(PrefillCfg<D>::kThreads, 2) void attn_prefill_kerne
         if constexpr (Cfg::kQLds) *reinterpret_cast<u32x4*>(lq + t * 1024) = third;
         else qp[t][kQRegs - 1] = third;
     }
-    // Whether the wave met operands outside the split (decided here for Q, or
-    // its values would be kept until the end).
-    bool again = __builtin_amdgcn_ballot_w64(query.big > kScoreTop) != 0;
+    // Whether the lane's query met operands outside the split (decided here for
+    // Q, or its values would be kept until the end). Two lanes hold a query.
+    const uint64_t far_q = __builtin_amdgcn_ballot_w64(query.big > kScoreTop);
+    bool again = (far_q | far_q >> 32) >> l32 & 1;
 
     auto store_k = [&](int i) {
-        SplitRange score;
 #pragma unroll
         for (int u = 0; u < Cfg::kKUnits; ++u) {
+            SplitRange score;
             const int f = threadIdx.x + u * Cfg::kThreads;
             if (Cfg::kKUnits * Cfg::kThreads != Cfg::kBKV * D / 4 && f >= Cfg::kBKV * D / 4) continue;
             const int row = f / (D / 4), c = f % (D / 4);
@@ -569,24 +581,26 @@ __global__ __launch_bounds__(PrefillCfg<D>::kThreads, 2) void attn_prefill_kerne
             char* at = lk + c / 2 * Cfg::kKChunk + row * 16 + c % 2 * 8;
 #pragma unroll
             for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x2*>(at + p * Cfg::kKPlane) = u32x2{p0[p], p1[p]};
+            if (score.big > kScoreTop) atomicOr(&far_keys[i & 1], 1u << row);
         }
-        if (score.big > kScoreTop) outside[i & 1] = 1;
     };
     // V is scaled by a power of two that keeps any sum of 2^8 kv_seq weighted
     // rows finite, and the output by its inverse.
     const int v_shift = 9 + 64 - __builtin_clzll(a.kv_seq);
     const float v_scale = v_in ? __uint_as_float(static_cast<uint32_t>(127 - v_shift) << 23) : 0.0f;
+    const uint32_t v_tiny = mhip::kSplitTiny + (static_cast<uint32_t>(v_shift) << 24);  // unscaled
     auto store_v = [&](int i) {
         if (!v_on) return;
         SplitRange value;
         u32x4 p[3];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float x0 = __uint_as_float(vr[2 * e]) * v_scale, x1 = __uint_as_float(vr[2 * e + 1]) * v_scale;
+            const float y0 = __uint_as_float(vr[2 * e]), y1 = __uint_as_float(vr[2 * e + 1]);
+            const float x0 = y0 * v_scale, x1 = y1 * v_scale;
             uint32_t q[3];
             mhip::split_pair(x0, x1, q);
             value.top(x0, x1);
-            value.bottom(x0, x1);
+            value.bottom(y0, y1);
             p[0][e] = q[0];
             p[1][e] = q[1];
             p[2][e] = q[2];
@@ -594,13 +608,14 @@ __global__ __launch_bounds__(PrefillCfg<D>::kThreads, 2) void attn_prefill_kerne
         char* at = lv + v_chunk * Cfg::kVChunk + v_col * 16;
 #pragma unroll
         for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4*>(at + q * Cfg::kVPlane) = p[q];
-        if (value.big > kValueTop || value.least < mhip::kSplitTiny) outside[i & 1] = 1;
+        if (value.big > kValueTop) bad_values[i & 1] = 1;
+        if (value.least < v_tiny) tiny_values[v_col] = any_tiny = 1;
     };
     auto mfma = [](bf16x8 x, bf16x8 y, v16f c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, c, 0, 0, 0); };
     auto as_bf16 = [](u32x4 v) { return __builtin_bit_cast(bf16x8, v); };
 
+    __syncthreads();
     if (i_end > i_begin) {
-        __syncthreads();
         store_k(i_begin);
         if (i_begin + 1 < i_end) load_k(i_begin + 1);
         mhip::lds_barrier<0>();
@@ -616,7 +631,7 @@ __global__ __launch_bounds__(PrefillCfg<D>::kThreads, 2) void attn_prefill_kerne
                 if (i + 2 < i_end) load_k(i + 2);
             };
             // (Read last in the tile before, set next after this tile's barrier.)
-            if (threadIdx.x == 0) outside[(i + 1) & 1] = 0;
+            if (threadIdx.x == 0) far_keys[(i + 1) & 1] = bad_values[(i + 1) & 1] = 0;
             v16f s;
             u32x4 pp[2][3];  // the probabilities' planes: step, plane
             float alpha = 1.0f;
@@ -658,7 +673,10 @@ __global__ __launch_bounds__(PrefillCfg<D>::kThreads, 2) void attn_prefill_kerne
             }
             mhip::lds_barrier<0>();
             if (mine) {
-                again |= outside[i & 1] != 0;
+                // (A value that is not finite reaches every query of the wave.)
+                const uint32_t far = far_keys[i & 1];
+                const int bad = bad_values[i & 1];
+                if (far | bad) again |= bad || (far & tile_keys(w.lo - rel, w.hi - rel));
                 if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
 #pragma unroll
                     for (int vb = 0; vb < Cfg::kVB; ++vb)
@@ -703,9 +721,9 @@ __global__ __launch_bounds__(PrefillCfg<D>::kThreads, 2) void attn_prefill_kerne
     if constexpr (D > 64) __asm__ volatile("" : "+s"(block), "+v"(thread));
     const PrefillPlace end = prefill_place<D>(a, sp, block, thread);
     // Register r of block vb holds O[q][vb*32 + 8*(r/4) + 4*half + r%4].
+    const int first = 4 * (thread >> 5 & 1);
     auto store = [&]() {
         if (!end.q_live) return;
-        const int first = 4 * (thread >> 5 & 1);
         if (end.ml && first == 0) *reinterpret_cast<float2*>(end.ml) = make_float2(m, l);
 #pragma unroll
         for (int vb = 0; vb < Cfg::kVB; ++vb)
@@ -717,11 +735,40 @@ __global__ __launch_bounds__(PrefillCfg<D>::kThreads, 2) void attn_prefill_kerne
                     make_float4(o[vb][4 * g], o[vb][4 * g + 1], o[vb][4 * g + 2], o[vb][4 * g + 3]);
             }
     };
-    again = __builtin_amdgcn_ballot_w64(again) != 0;
-    if (!again) store();
-    if (__syncthreads_or(again)) {
-        prefill_f32<D>(a, end, thread, again, reinterpret_cast<float*>(lds), o, m, l);
-        if (again) store();
+    // What is to be summed again: a query whose own row or keys lie outside the
+    // split, and an output so small that its column's tiny values (planes off
+    // by less than 2^-124 of the scaled mean) can have cost it a rounding.
+    uint32_t redo[2] = {0, 0};
+    if (any_tiny) {
+        const float least = __uint_as_float(static_cast<uint32_t>(127 + v_shift - 98) << 23);
+#pragma unroll
+        for (int vb = 0; vb < Cfg::kVB; ++vb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int c = vb * 32 + 8 * (r / 4) + first + r % 4;
+                if (tiny_values[c] && fabsf(o[vb][r]) < least) redo[vb / 2] |= 1u << (vb % 2 * 16 + r);
+            }
+    }
+    if (again) redo[0] = redo[1] = 0xFFFFFFFFu;
+    if (!end.q_live) redo[0] = redo[1] = 0;
+    const bool some = __builtin_amdgcn_ballot_w64((redo[0] | redo[1]) != 0) != 0;
+    auto store_some = [&](uint32_t flip) {
+        if (!end.q_live) return;
+        if (end.ml && first == 0 && again == (flip == 0)) *reinterpret_cast<float2*>(end.ml) = make_float2(m, l);
+#pragma unroll
+        for (int vb = 0; vb < Cfg::kVB; ++vb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int c = vb * 32 + 8 * (r / 4) + first + r % 4;
+                if (D % 32 != 0 && c >= D) continue;
+                if ((redo[vb / 2] >> (vb % 2 * 16 + r) & 1u) != flip) end.out[c] = o[vb][r];
+            }
+    };
+    if (!some) store();
+    else store_some(1);
+    if (__syncthreads_or(some)) {
+        prefill_f32<D>(a, end, thread, some, reinterpret_cast<float*>(lds), o, m, l);
+        if (some) store_some(0);
     }
 }
 

@@ -104,6 +104,45 @@ def test_operands_outside_the_split(dev, d, what):
         assert np.all(np.isinf(got[10:, 5]) & np.isinf(got[10:, d + 5])) and np.all(np.isfinite(got[:, :5]))
 
 
+@pytest.mark.parametrize("d", [32, 64, 80, 112, 128])
+@pytest.mark.parametrize("kv", [270, 1000])  # whole, and in key chunks
+def test_what_lies_outside_moves_its_own_queries_only(dev, d, kv):
+    """A key beyond 2^60 moves the queries that admit it, a query that one, and a
+    tiny value among ordinary ones no output."""
+    s, h, hkv = 260 if kv == 270 else 40, 4, 2
+    q, k, v = inputs(d + kv, s, kv, h, hkv, d)
+    want = bits(attend(dev, q, k, v, s, kv, h, hkv, d, causal=True))
+    at = kv - s + s // 2  # first admitted by query s // 2
+    far = k.copy()
+    far[at] = np.float32(2.0 ** 61)
+    got = bits(attend(dev, q, far, v, s, kv, h, hkv, d, causal=True))
+    assert np.array_equal(got[:s // 2], want[:s // 2]) and not np.array_equal(got[s // 2:], want[s // 2:])
+    big = q.copy()
+    big[s // 3] *= np.float32(2.0 ** 61)
+    got = bits(attend(dev, big, k, v, s, kv, h, hkv, d, causal=True))
+    others = np.arange(s) != s // 3
+    assert np.array_equal(got[others], want[others])
+    got = []
+    for value in (0.0, 1e-30, 1e-44):
+        few = v.copy()
+        few[5::17, ::3] = value
+        got.append(bits(attend(dev, q, k, few, s, kv, h, hkv, d, causal=True)))
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+
+
+@pytest.mark.parametrize("d", [32, 80, 128])
+@pytest.mark.parametrize("kv", [270, 1000])
+def test_columns_of_tiny_values(dev, d, kv):
+    """Each column at its own scale, down to values that vanish when scaled."""
+    s, h, hkv = 40, 4, 2
+    q, k, v = inputs(d, s, kv, h, hkv, d)
+    v *= (2.0 ** -np.linspace(60.0, 124.0, hkv * d)).astype(np.float32)
+    check(attend(dev, q, k, v, s, kv, h, hkv, d, causal=True), q, k, v, s, kv, h, hkv, d, True)
+    v[:, 3] = np.float32(1e-43)  # a denormal's mean is itself, to a few of the least f32
+    got = attend(dev, q, k, v, s, kv, h, hkv, d, causal=True)
+    assert np.all(np.abs(got[:, [3, 3 + d]] - np.float32(1e-43)) <= 64 * 2.0 ** -149)
+
+
 @pytest.mark.parametrize("d", [80, 96, 128])
 def test_a_replayed_row_has_the_bits_of_the_call(dev, d):
     from magnetar_hip import ops
