@@ -943,6 +943,12 @@ __device__ __forceinline__ void sum_dealt(float (&x)[N], int lane) {
     }
 }
 
+// The power of two p with l p in [0.5, 1), for a normal l > 0.
+__device__ __forceinline__ float half_over(float l) { return __uint_as_float((253u - (__float_as_uint(l) >> 23)) << 23); }
+
+// Its inverse.
+__device__ __forceinline__ float twice_under(float l) { return __uint_as_float(((__float_as_uint(l) >> 23) + 1u) << 23); }
+
 // One workgroup per (batch, KV head, key chunk). Every thread issues all of
 // its K and V loads before any arithmetic (2 * kSteps dwordx4 in flight).
 // A wave's scores are summed and dealt out over the lanes (sum_dealt), so that
@@ -1077,9 +1083,9 @@ __global__ __launch_bounds__(256) void attn_decode_partial_kernel(
         for (int off = 1 << kCopies; off < kSteps / kKeys << kCopies; off <<= 1) l += __shfl_xor(l, off, 64);
 #pragma unroll
         for (int off = kLPK; off < 64; off <<= 1) l += __shfl_xor(l, off, 64);
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        const float scale = l > 0.0f ? half_over(l) : 0.0f;
 #pragma unroll
-        for (int u = 0; u < kKeys; ++u) x[u] *= inv;
+        for (int u = 0; u < kKeys; ++u) x[u] *= scale;
         if (sub == 0 && (sl & ((1 << kCopies) - 1)) == 0 && first % kSteps == 0) {
             wm[wave][first / kSteps + g] = mx;
             wl[wave][first / kSteps + g] = l;
@@ -1095,8 +1101,8 @@ __global__ __launch_bounds__(256) void attn_decode_partial_kernel(
         __builtin_amdgcn_wave_barrier();
     }
 
-    // Weighted V rows with normalised probabilities: every partial sum is a
-    // convex combination of V rows, so none overflows. The keys' lanes sum as
+    // V rows weighted by the probabilities over a power of two above their sum:
+    // no partial sum overflows, and none of the weights is rounded again. The keys' lanes sum as
     // above, and lane group `sub` of the first kParts stores its part of a float4.
     constexpr int kParts = kKPS < 4 ? kKPS : 4;
 #pragma unroll
@@ -1147,18 +1153,25 @@ __global__ __launch_bounds__(256) void attn_decode_partial_kernel(
     for (int i = threadIdx.x; i < group * D4; i += 256) {
         const int g = i / D4, t = i % D4;
         const float m = fmaxf(fmaxf(wm[0][g], wm[1][g]), fmaxf(wm[2][g], wm[3][g]));
-        float f[4];
+        float e[4], f[4];
 #pragma unroll
-        for (int w = 0; w < 4; ++w) f[w] = wm[w][g] == -INFINITY ? wl[w][g] : wl[w][g] * exp2f(wm[w][g] - m);
+        for (int w = 0; w < 4; ++w) {
+            e[w] = wm[w][g] == -INFINITY ? 0.0f : exp2f(wm[w][g] - m);
+            f[w] = wm[w][g] == -INFINITY ? wl[w][g] : wl[w][g] * e[w];
+        }
         const float l = (f[0] + f[1]) + (f[2] + f[3]);
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        // (Their weights over a power of two above the sum of them, the rest of
+        // the division last.)
+        const float scale = l > 0.0f ? half_over(l) : 0.0f;
+        const float rest = l > 0.0f ? 1.0f / (l * scale) : 0.0f;
         float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
             const float4 r = red[w][g][t];
-            const float share = f[w] * inv;
+            const float share = wl[w][g] > 0.0f ? e[w] * twice_under(wl[w][g]) * scale : 0.0f;
             o.x += share * r.x; o.y += share * r.y; o.z += share * r.z; o.w += share * r.w;
         }
+        o.x *= rest; o.y *= rest; o.z *= rest; o.w *= rest;
         const uint64_t rec = (bh0 + g) * chunks + c_idx;
         *reinterpret_cast<float4*>(part_o + rec * D + 4 * t) = o;
         if (t == 0) *reinterpret_cast<float2*>(part_ml + 2 * rec) = make_float2(m, l);
