@@ -93,10 +93,18 @@ __device__ __forceinline__ void key_range(const AttnArgs& a, uint64_t qpos, uint
 
 // A head dimension of 16 n; the value columns go in blocks of 32 (the last one
 // partly past the row, its columns zero and never stored).
-template <int D>
+//
+// Four waves, two workgroups per CU, for up to 128 queries of a head dimension
+// of up to 64 (above, K's, V's and Q's planes fill more than half of the LDS):
+// half of eight waves would have no query, and batches of few queries whose
+// chunks pass one round of workgroups wait for a second (8 x 20 queries over
+// 2000 keys, 8 heads of 64 on 2, 63 us with eight, 44 with four; 8 x 128 over
+// 1000, 32 on 8, 119 and 87). A single prompt of 64-128 takes 3-7 % longer.
+template <int D, int WAVES = 8>
 struct PrefillCfg {
     static_assert(D % 16 == 0 && D <= 128, "whole MFMA steps, and the registers of 128");
-    static constexpr int kWaves = 8;
+    static_assert(WAVES == 8 || (WAVES == 4 && D <= 64), "one or two waves split a chunk of V");
+    static constexpr int kWaves = WAVES;
     static constexpr int kThreads = 64 * kWaves;
     static constexpr int kBQ = 32 * kWaves;    // queries per workgroup
     static constexpr int kBKV = 32;            // keys per tile
@@ -222,10 +230,10 @@ struct PrefillPlace {
 // Block and key counts are below 2^31, so all of it is 32-bit, mostly scalar,
 // and a division that a call does not need (one query tile, one sequence, no
 // shared KV heads) is skipped: a prompt of 32 waits for each in turn.
-template <int D>
+template <int D, int WAVES>
 __device__ __forceinline__ PrefillPlace prefill_place(const AttnArgs& a, const PrefillSplit& sp, uint32_t block,
                                                       int thread) {
-    using Cfg = PrefillCfg<D>;
+    using Cfg = PrefillCfg<D, WAVES>;
     const int lane = thread & 63, wave = __builtin_amdgcn_readfirstlane(thread >> 6);
     const uint32_t heads = static_cast<uint32_t>(a.heads);
     uint32_t bh = block, chunk = 0, qt = sp.qtiles - 1;
@@ -347,10 +355,10 @@ __device__ __forceinline__ float softmax_tile_mean(v16f& s, float& m, float& l) 
 // admits enters P . V at weight 0, so a wave that met a V value that is not
 // finite in an edge tile sums its queries' admitted keys again on the VALU
 // (recompute_admitted).
-template <int D>
+template <int D, int WAVES>
 __device__ __forceinline__ void prefill_f32(const AttnArgs& a, const PrefillPlace& w, int thread, bool again,
                                             float* lds, v16f (&o)[PrefillCfg<D>::kVB], float& m, float& l) {
-    using Cfg = PrefillCfg<D>;
+    using Cfg = PrefillCfg<D, WAVES>;
     const int lane = thread & 63, l32 = lane & 31, half = lane >> 5;
     const uint64_t kv_ld = a.kv_heads * D;
     const float* const qhalf = w.qrow + half * (D / 2);
@@ -456,10 +464,10 @@ constexpr uint32_t kValueTop = 2u * (254u << 23);           // (a scaled one is 
 // Bound by the chain within a wave (scores, softmax, the split of the
 // probabilities, P . V) with two waves per SIMD to hide it: the registers of
 // Q's planes and the output allow no third.
-template <int D>
-__global__ __launch_bounds__(PrefillCfg<D>::kThreads, 2) void attn_prefill_kernel(AttnArgs a, PrefillSplit sp) {
+template <int D, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, 2) void attn_prefill_kernel(AttnArgs a, PrefillSplit sp) {
     apply_advance(a);
-    using Cfg = PrefillCfg<D>;
+    using Cfg = PrefillCfg<D, WAVES>;
     using mhip::bf16x8;
     using mhip::u32x2;
     using mhip::u32x4;
@@ -471,7 +479,7 @@ __global__ __launch_bounds__(PrefillCfg<D>::kThreads, 2) void attn_prefill_kerne
     char* const lq = lv + 3 * Cfg::kVPlane + wave * Cfg::kSteps * 1024 + lane * 16;
     const int l32 = lane & 31, half = lane >> 5;
 
-    const PrefillPlace w = prefill_place<D>(a, sp, blockIdx.x, threadIdx.x);
+    const PrefillPlace w = prefill_place<D, WAVES>(a, sp, blockIdx.x, threadIdx.x);
     const float *const K = w.K, *const V = w.V, *const qrow = w.qrow;
     const uint64_t kv_ld = a.kv_heads * D, tile_begin = w.tile_begin;
     const int i_begin = w.i_begin, i_end = w.i_end;
@@ -488,8 +496,8 @@ __global__ __launch_bounds__(PrefillCfg<D>::kThreads, 2) void attn_prefill_kerne
     // the range instead, which wraps where that key lies past the end.
     u32x4 kr[Cfg::kKUnits];
     uint32_t vr[8];
-    const int v_chunk = wave >> 1;  // step v_chunk / 2, half v_chunk % 2
-    const int v_col = (wave & 1) * 64 + lane;
+    const int v_chunk = WAVES == 8 ? wave >> 1 : wave;  // step v_chunk / 2, half v_chunk % 2
+    const int v_col = WAVES == 8 ? (wave & 1) * 64 + lane : lane;
     const bool v_on = v_col < Cfg::kVB * 32;
     const bool v_in = v_col < D;
     const uint32_t ld_bytes = static_cast<uint32_t>(kv_ld * sizeof(float));  // the launch checks 32 rows < 2^31
@@ -719,7 +727,7 @@ __global__ __launch_bounds__(PrefillCfg<D>::kThreads, 2) void attn_prefill_kerne
     uint32_t block = blockIdx.x;
     int thread = threadIdx.x;
     if constexpr (D > 64) __asm__ volatile("" : "+s"(block), "+v"(thread));
-    const PrefillPlace end = prefill_place<D>(a, sp, block, thread);
+    const PrefillPlace end = prefill_place<D, WAVES>(a, sp, block, thread);
     // Register r of block vb holds O[q][vb*32 + 8*(r/4) + 4*half + r%4].
     const int first = 4 * (thread >> 5 & 1);
     auto store = [&]() {
@@ -767,7 +775,7 @@ __global__ __launch_bounds__(PrefillCfg<D>::kThreads, 2) void attn_prefill_kerne
     if (!some) store();
     else store_some(1);
     if (__syncthreads_or(some)) {
-        prefill_f32<D>(a, end, thread, some, reinterpret_cast<float*>(lds), o, m, l);
+        prefill_f32<D, WAVES>(a, end, thread, some, reinterpret_cast<float*>(lds), o, m, l);
         if (some) store_some(0);
     }
 }
@@ -819,16 +827,16 @@ __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(AttnArgs a, u
 }
 
 // Key chunks for a prefill whose query tiles (per sequence) do not give every
-// CU its workgroup: enough chunks of at least 4 key tiles to do so, at most 16.
+// CU its workgroups: enough chunks of at least 4 key tiles to do so, at most 16.
 void prefill_split(const mhip_ctx* ctx, const AttnArgs& a, bool replayable, uint64_t qtiles, uint64_t kbkv,
-                   uint32_t* nchunks, uint32_t* chunk_tiles) {
+                   uint64_t per_cu, uint32_t* nchunks, uint32_t* chunk_tiles) {
     *nchunks = 1;
     *chunk_tiles = 0;
     // A replayed key count may pass the captured one: chunks sized here from
     // the captured count would leave the later keys to no workgroup. The call
     // outside a capture sums the same way, so that a replay gives its bits.
     if (replayable) return;
-    const uint64_t slots = ctx->compute_units ? ctx->compute_units : 256;
+    const uint64_t slots = per_cu * (ctx->compute_units ? ctx->compute_units : 256);
     const uint64_t per_sequence = a.heads * qtiles;
     const uint64_t kv_tiles = (a.kv_seq + kbkv - 1) / kbkv;
     if (per_sequence >= slots || kv_tiles < 8) return;
@@ -840,12 +848,14 @@ void prefill_split(const mhip_ctx* ctx, const AttnArgs& a, bool replayable, uint
     *nchunks = static_cast<uint32_t>((kv_tiles + per - 1) / per);
 }
 
-template <int D>
+template <int D, int WAVES = 8>
 mhip_status launch_prefill(mhip_ctx* ctx, const AttnArgs& a, uint64_t batch, bool replayable) {
-    using Cfg = PrefillCfg<D>;
+    using Cfg = PrefillCfg<D, WAVES>;
+    if constexpr (D <= 64 && WAVES == 8)
+        if (a.seq <= PrefillCfg<D, 4>::kBQ) return launch_prefill<D, 4>(ctx, a, batch, replayable);
     const uint64_t qtiles = (a.seq + Cfg::kBQ - 1) / Cfg::kBQ;
     PrefillSplit sp{};
-    prefill_split(ctx, a, replayable, qtiles, Cfg::kBKV, &sp.nchunks, &sp.chunk_tiles);
+    prefill_split(ctx, a, replayable, qtiles, Cfg::kBKV, 8 / WAVES, &sp.nchunks, &sp.chunk_tiles);
     // (The other head dimensions ran on the generic kernel, without chunks.)
     const mhip::CaptureGrowth growth(ctx, D != 64 && D != 128);
     const uint64_t blocks = batch * a.heads * qtiles * sp.nchunks;
@@ -865,11 +875,11 @@ mhip_status launch_prefill(mhip_ctx* ctx, const AttnArgs& a, uint64_t batch, boo
     const size_t lds = Cfg::kLdsBytes;
     static bool configured = false;
     if (!configured) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prefill_kernel<D>),
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prefill_kernel<D, WAVES>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
         configured = true;
     }
-    mhip::launch(ctx, (attn_prefill_kernel<D>), dim3(static_cast<unsigned>(blocks)), dim3(Cfg::kThreads),
+    mhip::launch(ctx, (attn_prefill_kernel<D, WAVES>), dim3(static_cast<unsigned>(blocks)), dim3(Cfg::kThreads),
                  lds, a, sp);
     mhip_status st = mhip::check_launch("attention (MFMA prefill)");
     if (st != MHIP_OK || sp.nchunks == 1) return st;

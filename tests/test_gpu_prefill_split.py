@@ -64,6 +64,16 @@ def test_edges_of_tiles(dev, s, kv, h, hkv, causal, window, d):
     check(got, q, k, v, s, kv, h, hkv, d, causal, window)
 
 
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("window", [None, 50])
+def test_128_queries_have_the_bits_of_129(dev, d, window):
+    """Workgroups of four waves and of eight: the same queries, the same bits."""
+    kv, h, hkv = 200, 4, 2
+    q, k, v = inputs(d, 129, kv, h, hkv, d)
+    got = [attend(dev, q[129 - s:], k, v, s, kv, h, hkv, d, causal=True, window_size=window) for s in (128, 129)]
+    assert np.array_equal(bits(got[0]), bits(got[1][1:]))
+
+
 @pytest.mark.parametrize("d", [32, 96, 128])
 def test_a_batch_is_its_sequences(dev, d):
     from magnetar_hip import ops
