@@ -179,9 +179,11 @@ mhip_status mhip_rope_f32(mhip_ctx* ctx, const float* in, float* out, uint64_t r
 /* out[m, n] = A . B with A [m, k] (or [k, m] stored when transpose_a) and
  * B [k, n] (or [n, k] when transpose_b), f32 accumulation; addend_mode 1 adds
  * addend[col] (matmul-bias), 2 adds addend[row * n + col] (matmul-residual)
- * to the finished sum. For m > 8 matrix-core tiles, each f32 operand split
- * exactly into three bf16 planes (six plane products, an error at or below the
- * f32 matrix instructions'); HBM-streaming kernels for m <= 8 (decode). Partial
+ * to the finished sum. Matrix-core tiles, each f32 operand split exactly into
+ * three bf16 planes (six plane products; products of k 1 and 2, and sums that a
+ * value outside the split matters to, on the f32 matrix instructions); up to 32
+ * rows of b [k, n], and up to 8 rows of b [n, k] with 16-byte rows, take
+ * HBM-streaming kernels. An entry's bits depend on its own row and column. Partial
  * sums use a grow-only workspace owned by the context. */
 mhip_status mhip_matmul_f32(mhip_ctx* ctx, const float* a, const float* b, float* out,
                             uint64_t m, uint64_t k, uint64_t n, int transpose_a,
@@ -243,8 +245,8 @@ typedef struct {
  * q.k * scale over the admitted keys weights V rows; a NaN or +inf score, and
  * admitted scores that are all -inf, give NaN.
  * Flash prefill on split bf16 planes for head dims 32, 64, 80, 96, 112 and 128,
- * split-KV decode for one query
- * row (workspace owned by the context), a generic kernel otherwise. */
+ * split-KV decode for one query row of head dims 4, 8, 16, 32, 64, 128 and 256
+ * (workspace owned by the context), a generic kernel otherwise. */
 mhip_status mhip_attention_f32(mhip_ctx* ctx, const float* q, const float* k, const float* v,
                                float* out, const mhip_attention_params* params);
 
@@ -306,7 +308,9 @@ mhip_status mhip_kv_write_f32(mhip_ctx* ctx, float* store, uint64_t capacity, ui
  * written must stay inside K/V and the store). Nothing that allocates,
  * transfers, clears memory or synchronises can be captured: such a call
  * returns CaptureUnsupported and fails the capture (mhip_capture_end then
- * reports the first reason). Multi-row attention replays only at offset 0. */
+ * reports the first reason). Growing the workspace is such an allocation, but
+ * for products and prompt attention that could run without that scratch: for
+ * them it grows while recording, so that a capture takes the eager call's plan. Multi-row attention replays only at offset 0. */
 typedef enum {
     MHIP_ADVANCE_POSITION_OFFSET = 1,
     MHIP_ADVANCE_KEY_COUNT = 2,

@@ -14,7 +14,8 @@
 // Three kernels:
 //  - prefill (head dims 32, 64, 80, 96, 112 and 128): flash attention on the
 //    bf16 matrix cores with every operand split into three bf16 planes. A
-//    workgroup takes 256 queries of one (batch, head), eight waves of 32, and
+//    workgroup takes 256 queries of one (batch, head), eight waves of 32 (four
+//    for short prompts of head dims 32 and 64), and
 //    walks the admitted keys in 32-key tiles. Each wave computes S^T = K . Q^T
 //    (Q^T lives in registers, pre-scaled by scale * log2 e), so every lane
 //    owns one query column and 16 of the tile's keys: the online-softmax
@@ -22,8 +23,8 @@
 //    are then exactly the B operand of O^T = V^T . P^T, so the output stays
 //    per-lane too. V is scaled down by a power of two above the sum of the
 //    weights, so the running output never overflows (the reference's 1e38
-//    known answer, src/tests_conformance.rs:2215-2312). Operands the split
-//    does not hold go to the f32 MFMA, wave by wave.
+//    known answer, src/tests_conformance.rs:2215-2312). Outputs that operands
+//    outside the split matter to are summed again with the f32 MFMA.
 //  - decode (one query row, head dim 4, 8, 16, ..., 256): split-KV. A
 //    workgroup takes one (batch, KV head, key chunk) and the query heads
 //    that share that KV head (up to 8; a larger group is split into slices
@@ -88,7 +89,7 @@ __device__ __forceinline__ void key_range(const AttnArgs& a, uint64_t qpos, uint
 }
 
 // ---------------------------------------------------------------------------
-// Prefill: fp32 MFMA flash attention
+// Prefill: flash attention on split bf16 planes
 // ---------------------------------------------------------------------------
 
 // A head dimension of 16 n; the value columns go in blocks of 32 (the last one
@@ -458,8 +459,10 @@ constexpr uint32_t kValueTop = 2u * (254u << 23);           // (a scaled one is 
 // tile's K is; both are loaded a tile ahead.
 //
 // Against the f32 MFMA kernel (four waves, 128 queries), causal, us: 4
-// sequences of 2048, 32 heads of 128, 1225 before and 837 now; one of 509 63
-// and 44; 1024 keys, 16 heads of 64, 4 sequences 172 and 139. Head dims 32, 80,
+// sequences of 2048, 32 heads of 128, 1127 before and 727 now; one of 509 60
+// and 42; 1024 keys, 16 heads of 64 53 and 38. (Batches of few queries of 128
+// wait for a second round of workgroups: 8 of 20 over 2000, 8 heads on 2, 72 and
+// 89, 6 of 7 over 420 31 and 40.) Head dims 32, 80,
 // 96 and 112 ran on the generic kernel: 1024 keys, 32 heads of 80 5435 and 79.
 // Bound by the chain within a wave (scores, softmax, the split of the
 // probabilities, P . V) with two waves per SIMD to hide it: the registers of

@@ -43,8 +43,8 @@ constexpr int kPanelCols = kPanelWaves * 32 * kPanelBlocks<BT>;
 // What bounds it: the bytes in flight, so the waves a CU holds (two workgroups
 // at 128 registers). The 64 x 64 tiles that these products took before keep 8
 // KB of B in flight per workgroup; here each of 16 waves per CU keeps 8 KB.
-// 24 x 4096 x 11008: f32 MFMA tiles 149 us, split tiles 74, this 43 (4.2 TB/s);
-// compact 31.
+// 24 x 4096 x 11008: f32 MFMA tiles 149 us, split tiles 74, this 43 (37 at 5.2
+// TB/s and the slices' sum); compact 27.
 template <class BT, class Addend>
 __global__ __launch_bounds__(64 * kPanelWaves, 4) void panel_kernel(
     const float* __restrict__ A, const BT* __restrict__ B, float* __restrict__ C, uint64_t M, uint64_t K,

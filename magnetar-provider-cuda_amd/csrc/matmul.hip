@@ -1666,19 +1666,20 @@ __global__ void fill_addend_kernel(float* C, uint64_t M, uint64_t N, const float
 // The tile configurations, picked per shape by the time model. What bounds
 // them, and TFLOP/s at 4096^3 and 2048^3 (f32 MFMA kernels before: 146, 134 us
 // at 2048^3):
-//  - kBig: 256 x 256 tiles, 8 waves of 64 x 128: 230-237 TFLOP/s, 580-615 us
-//    at 4096^3 (938 before), 400 with compact weights. The card's power limit
-//    bounds it: MFMAs are busy 75 % of the cycles at 1.77 GHz, and a loop of
-//    nothing but these MFMAs runs at 1.76 GHz. Three buffers and the barrier
+//  - kBig: 256 x 256 tiles, 8 waves of 64 x 128: 218-231 TFLOP/s, 595-630 us
+//    at 4096^3 by the inputs (938 before), 400 with compact weights. The card's
+//    power limit bounds it: MFMAs are busy 68 % of the cycles at 1.85 GHz, and a
+//    loop of nothing but these MFMAs runs at 1.79 GHz. Three buffers and the barrier
 //    that leaves the next stage's reads in flight took 1.17 M cycles to 1.05 M
 //    and 606 us to 591.
 //  - kSmall: 128 x 128 tiles, 4 waves of 64 x 64, two workgroups per CU: 190;
-//  - kMid: 128 x 128 tiles, 8 waves of 32 x 64: 185, 114-120 us at 2048^3,
-//    bound by issue: 5.7 VALU instructions (the split) per MFMA, of which
+//  - kMid: 128 x 128 tiles, 8 waves of 32 x 64: 167-185, 103-120 us at 2048^3,
+//    bound by issue: 5.9 VALU instructions (the split) per MFMA, of which
 //    about 4 hide behind it, and 96 bytes of LDS reads per cycle;
-//  - kTiny: 64 x 64 tiles, 8 waves of 32 x 32 in two k groups: 130; products
+//  - kTiny: 64 x 64 tiles, 8 waves of 32 x 32 in two k groups: 93-130; products
 //    of about one such tile per CU (1024^3: 256 tiles), which then need no k
-//    split and no second launch.
+//    split and no second launch. Bound by the split's VALU, 13 instructions per
+//    MFMA, and by its waits: 23.0 us at 1024^3 where the f32 MFMA took 21.0.
 enum class TileChoice { kBig, kSmall, kMid, kTiny };
 
 using BigShape = TileShape<256, 256, 64, 128, 1, 16, 3>;

@@ -8,10 +8,11 @@
 // products the six of at least 2^-18 of x y are summed, smallest first, in
 // the f32 accumulators:
 //     a1 b3 + a3 b1 + a2 b2 + a1 b2 + a2 b1 + a1 b1;
-// the other three are below 2^-26 of x y, under a quarter of the rounding of
-// a single f32 addition. An accumulator is rounded 6 times per 16 k rather
-// than about 16, so sums come out closer to the exact product than with the
-// f32 MFMA: 2-norm errors against f64 of 32 x 32 tiles, f32 MFMA and split,
+// the other three add up to at most 1.01 x 2^-24 of |x y| (|x2| <= 2^-8 |x|, |x3|
+// <= 2^-17 |x|; 2^-27.5 as the rms over mantissas), the largest rounding of one
+// product. An accumulator is rounded 6 times per 16 k rather than about 16, so
+// from k 3 on sums come out closer to the exact product than with the f32 MFMA
+// on every distribution measured (kSplitMinK has the shorter ones): 2-norm errors against f64 of 32 x 32 tiles, f32 MFMA and split,
 // N(0,1) x N(0,0.02): K 64 1.45e-7 and 1.10e-7, 256 2.9e-7 and 2.4e-7, 4096
 // 1.15e-6 and 0.99e-6, 16384 2.3e-6 and 2.1e-6; U(0,1): K 4096 8.4e-7 and
 // 5.3e-7; log-normal: 1.1e-6 and 6.1e-7. A compact bf16 B is its own single
