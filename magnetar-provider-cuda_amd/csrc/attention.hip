@@ -96,11 +96,12 @@ __device__ __forceinline__ void key_range(const AttnArgs& a, uint64_t qpos, uint
 // partly past the row, its columns zero and never stored).
 //
 // Four waves, two workgroups per CU, for up to 128 queries of a head dimension
-// of up to 64 (above, K's, V's and Q's planes fill more than half of the LDS):
-// half of eight waves would have no query, and batches of few queries whose
-// chunks pass one round of workgroups wait for a second (8 x 20 queries over
-// 2000 keys, 8 heads of 64 on 2, 63 us with eight, 44 with four; 8 x 128 over
-// 1000, 32 on 8, 119 and 87). A single prompt of 64-128 takes 3-7 % longer.
+// of up to 64 (above, K's, V's and Q's planes fill more than half of the LDS)
+// where eight would take a second round of workgroups, half of their waves
+// without a query: 8 x 20 queries over 2000 keys, 8 heads of 64 on 2, 63 us with
+// eight, 44 with four; 8 x 128 over 1000, 32 on 8, 119 and 87. In one round four
+// take 3-7 % longer for 64-128 queries, and less for up to 32, one wave's (32 of
+// 4 heads 6.3 and 6.0). Either way the same chunks and the same bits.
 template <int D, int WAVES = 8>
 struct PrefillCfg {
     static_assert(D % 16 == 0 && D <= 128, "whole MFMA steps, and the registers of 128");
@@ -830,16 +831,16 @@ __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(AttnArgs a, u
 }
 
 // Key chunks for a prefill whose query tiles (per sequence) do not give every
-// CU its workgroups: enough chunks of at least 4 key tiles to do so, at most 16.
+// CU its workgroup: enough chunks of at least 4 key tiles to do so, at most 16.
 void prefill_split(const mhip_ctx* ctx, const AttnArgs& a, bool replayable, uint64_t qtiles, uint64_t kbkv,
-                   uint64_t per_cu, uint32_t* nchunks, uint32_t* chunk_tiles) {
+                   uint32_t* nchunks, uint32_t* chunk_tiles) {
     *nchunks = 1;
     *chunk_tiles = 0;
     // A replayed key count may pass the captured one: chunks sized here from
     // the captured count would leave the later keys to no workgroup. The call
     // outside a capture sums the same way, so that a replay gives its bits.
     if (replayable) return;
-    const uint64_t slots = per_cu * (ctx->compute_units ? ctx->compute_units : 256);
+    const uint64_t slots = ctx->compute_units ? ctx->compute_units : 256;
     const uint64_t per_sequence = a.heads * qtiles;
     const uint64_t kv_tiles = (a.kv_seq + kbkv - 1) / kbkv;
     if (per_sequence >= slots || kv_tiles < 8) return;
@@ -854,14 +855,15 @@ void prefill_split(const mhip_ctx* ctx, const AttnArgs& a, bool replayable, uint
 template <int D, int WAVES = 8>
 mhip_status launch_prefill(mhip_ctx* ctx, const AttnArgs& a, uint64_t batch, bool replayable) {
     using Cfg = PrefillCfg<D, WAVES>;
-    if constexpr (D <= 64 && WAVES == 8)
-        if (a.seq <= PrefillCfg<D, 4>::kBQ) return launch_prefill<D, 4>(ctx, a, batch, replayable);
     const uint64_t qtiles = (a.seq + Cfg::kBQ - 1) / Cfg::kBQ;
     PrefillSplit sp{};
-    prefill_split(ctx, a, replayable, qtiles, Cfg::kBKV, 8 / WAVES, &sp.nchunks, &sp.chunk_tiles);
+    prefill_split(ctx, a, replayable, qtiles, Cfg::kBKV, &sp.nchunks, &sp.chunk_tiles);
     // (The other head dimensions ran on the generic kernel, without chunks.)
     const mhip::CaptureGrowth growth(ctx, D != 64 && D != 128);
     const uint64_t blocks = batch * a.heads * qtiles * sp.nchunks;
+    if constexpr (D <= 64 && WAVES == 8)
+        if (a.seq <= 32 || (a.seq <= PrefillCfg<D, 4>::kBQ && blocks > (ctx->compute_units ? ctx->compute_units : 256)))
+            return launch_prefill<D, 4>(ctx, a, batch, replayable);
     if (blocks >= (1ULL << 31)) return mhip::fail(MHIP_SHAPE_UNSUPPORTED, "attention: too many query tiles");
     sp.qtiles = static_cast<uint32_t>(qtiles);
     sp.pairs = static_cast<uint32_t>(batch * a.heads);

@@ -67,11 +67,31 @@ def test_edges_of_tiles(dev, s, kv, h, hkv, causal, window, d):
 @pytest.mark.parametrize("d", [32, 64])
 @pytest.mark.parametrize("window", [None, 50])
 def test_128_queries_have_the_bits_of_129(dev, d, window):
-    """Workgroups of four waves and of eight: the same queries, the same bits."""
-    kv, h, hkv = 200, 4, 2
+    """Workgroups of four waves (more than one round of them) and of eight: the
+    same queries, the same bits."""
+    from magnetar_hip import ops
+    kv, h, hkv, batch = 200, 4, 2, 65
     q, k, v = inputs(d, 129, kv, h, hkv, d)
-    got = [attend(dev, q[129 - s:], k, v, s, kv, h, hkv, d, causal=True, window_size=window) for s in (128, 129)]
-    assert np.array_equal(bits(got[0]), bits(got[1][1:]))
+    want = attend(dev, q, k, v, 129, kv, h, hkv, d, causal=True, window_size=window)[1:]
+    p = ops.attention_params(128, kv, h, d, kv_head_count=hkv, causal=True, window_size=window, batch=batch)
+    many = [dev.upload(np.tile(x, (batch, 1))) for x in (q[1:], k, v)]
+    got = ops.attention(dev, *many, p).numpy().reshape(batch, 128, h * d)
+    for one in (attend(dev, q[1:], k, v, 128, kv, h, hkv, d, causal=True, window_size=window), got[0], got[64]):
+        assert np.array_equal(bits(one), bits(want))
+    check(got[33], q[1:], k, v, 128, kv, h, hkv, d, True, window)
+
+
+@pytest.mark.parametrize("s,kv", [(1, 33), (7, 420), (31, 64), (127, 300)])
+def test_batches_of_few_queries(dev, s, kv):
+    """Four waves a workgroup, a batch its separate calls bit for bit."""
+    from magnetar_hip import ops
+    d, h, hkv, batch = 32, 16, 4, 17
+    q, k, v = inputs(s, s, kv, h, hkv, d)
+    p = ops.attention_params(s, kv, h, d, kv_head_count=hkv, causal=True, batch=batch)
+    got = ops.attention(dev, *[dev.upload(np.tile(x, (batch, 1))) for x in (q, k, v)], p).numpy().reshape(batch, s, h * d)
+    one = attend(dev, q, k, v, s, kv, h, hkv, d, causal=True)
+    check(one, q, k, v, s, kv, h, hkv, d, True)
+    assert all(np.array_equal(bits(got[b]), bits(one)) for b in range(batch))
 
 
 @pytest.mark.parametrize("d", [32, 96, 128])
