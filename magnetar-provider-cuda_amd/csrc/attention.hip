@@ -446,6 +446,21 @@ struct SplitRange {
 constexpr uint32_t kScoreTop = 2u * ((127u + 60u) << 23);   // 2^60
 constexpr uint32_t kValueTop = 2u * (254u << 23);           // (a scaled one is below 2^127 or not finite)
 
+// Whether a lane's query admits a key, among its workgroup's, with a K beyond
+// the scores' range. Its two lanes look at a half of each row. (Slow, as
+// recompute_admitted is: only where a tile held such a key.)
+template <int D>
+__device__ __forceinline__ bool admits_far_key(const PrefillPlace& w, uint64_t kv_ld, int half) {
+    const int lo = max(w.lo, w.i_begin * 32), hi = min(w.hi, w.i_end * 32);
+    uint32_t big = 0;
+    for (int j = lo; j < hi; ++j) {
+        const float* const row = w.K + (w.tile_begin + j) * kv_ld + half * (D / 2);
+        for (int t = 0; t < D / 2; ++t) big = max(big, __float_as_uint(row[t]) << 1);
+    }
+    const uint64_t far = __builtin_amdgcn_ballot_w64(big > kScoreTop);
+    return (far | far >> 32) >> (threadIdx.x & 31) & 1;
+}
+
 // Flash attention of 256 queries of one (batch, head), eight waves of 32, on
 // the bf16 matrix cores: Q, K and V split exactly into three bf16 planes
 // (split_tile.hpp) and the probabilities too, six plane products a product.
@@ -536,13 +551,12 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_prefill_kernel(AttnArgs a,
         load_v(i_begin);
     }
     SplitRange query;
-    // A tile's (by parity) keys whose K is outside the split, and whether some V
-    // of it is not finite; the value columns with a nonzero below 2^-100 (scaled).
-    __shared__ uint32_t far_keys[2];
-    __shared__ int bad_values[2], any_tiny;
+    // What a tile (by parity) holds outside the split; the value columns with a
+    // nonzero below 2^-100 (scaled).
+    constexpr uint32_t kFarKey = 1, kBadValue = 2, kTinyValue = 4;
+    __shared__ uint32_t outside[2];
     __shared__ uint8_t tiny_values[Cfg::kVB * 32];
-    if (threadIdx.x < 2) far_keys[threadIdx.x] = bad_values[threadIdx.x] = 0;
-    if (threadIdx.x == 2) any_tiny = 0;
+    if (threadIdx.x < 2) outside[threadIdx.x] = 0;
     if (threadIdx.x < Cfg::kVB * 32) tiny_values[threadIdx.x] = 0;
 
     // Q^T's planes, pre-scaled: step t, k = 16 t + 8 half + i of the query.
@@ -570,15 +584,15 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_prefill_kernel(AttnArgs a,
         if constexpr (Cfg::kQLds) *reinterpret_cast<u32x4*>(lq + t * 1024) = third;
         else qp[t][kQRegs - 1] = third;
     }
-    // Whether the lane's query met operands outside the split (decided here for
-    // Q, or its values would be kept until the end). Two lanes hold a query.
+    // The wave's queries outside the split (decided here, or their values would
+    // be kept until the end), and what it met in its tiles.
     const uint64_t far_q = __builtin_amdgcn_ballot_w64(query.big > kScoreTop);
-    bool again = (far_q | far_q >> 32) >> l32 & 1;
+    uint32_t met = 0;
 
     auto store_k = [&](int i) {
+        SplitRange score;
 #pragma unroll
         for (int u = 0; u < Cfg::kKUnits; ++u) {
-            SplitRange score;
             const int f = threadIdx.x + u * Cfg::kThreads;
             if (Cfg::kKUnits * Cfg::kThreads != Cfg::kBKV * D / 4 && f >= Cfg::kBKV * D / 4) continue;
             const int row = f / (D / 4), c = f % (D / 4);
@@ -593,8 +607,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_prefill_kernel(AttnArgs a,
             char* at = lk + c / 2 * Cfg::kKChunk + row * 16 + c % 2 * 8;
 #pragma unroll
             for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x2*>(at + p * Cfg::kKPlane) = u32x2{p0[p], p1[p]};
-            if (score.big > kScoreTop) atomicOr(&far_keys[i & 1], 1u << row);
         }
+        if (score.big > kScoreTop) atomicOr(&outside[i & 1], kFarKey);
     };
     // V is scaled by a power of two that keeps any sum of 2^8 kv_seq weighted
     // rows finite, and the output by its inverse.
@@ -620,8 +634,10 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_prefill_kernel(AttnArgs a,
         char* at = lv + v_chunk * Cfg::kVChunk + v_col * 16;
 #pragma unroll
         for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4*>(at + q * Cfg::kVPlane) = p[q];
-        if (value.big > kValueTop) bad_values[i & 1] = 1;
-        if (value.least < v_tiny) tiny_values[v_col] = any_tiny = 1;
+        if (value.big > kValueTop || value.least < v_tiny) {
+            atomicOr(&outside[i & 1], (value.big > kValueTop ? kBadValue : 0) | (value.least < v_tiny ? kTinyValue : 0));
+            if (value.least < v_tiny) tiny_values[v_col] = 1;
+        }
     };
     auto mfma = [](bf16x8 x, bf16x8 y, v16f c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, c, 0, 0, 0); };
     auto as_bf16 = [](u32x4 v) { return __builtin_bit_cast(bf16x8, v); };
@@ -643,7 +659,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_prefill_kernel(AttnArgs a,
                 if (i + 2 < i_end) load_k(i + 2);
             };
             // (Read last in the tile before, set next after this tile's barrier.)
-            if (threadIdx.x == 0) far_keys[(i + 1) & 1] = bad_values[(i + 1) & 1] = 0;
+            if (threadIdx.x == 0) outside[(i + 1) & 1] = 0;
             v16f s;
             u32x4 pp[2][3];  // the probabilities' planes: step, plane
             float alpha = 1.0f;
@@ -685,10 +701,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_prefill_kernel(AttnArgs a,
             }
             mhip::lds_barrier<0>();
             if (mine) {
-                // (A value that is not finite reaches every query of the wave.)
-                const uint32_t far = far_keys[i & 1];
-                const int bad = bad_values[i & 1];
-                if (far | bad) again |= bad || (far & tile_keys(w.lo - rel, w.hi - rel));
+                met |= outside[i & 1];
                 if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
 #pragma unroll
                     for (int vb = 0; vb < Cfg::kVB; ++vb)
@@ -748,22 +761,30 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_prefill_kernel(AttnArgs a,
             }
     };
     // What is to be summed again: a query whose own row or keys lie outside the
-    // split, and an output so small that its column's tiny values (planes off
-    // by less than 2^-124 of the scaled mean) can have cost it a rounding.
+    // split or whose wave met a value that is not finite, and an output so small
+    // that its column's tiny values (planes off by less than 2^-124 of the
+    // scaled mean) can have cost it a rounding.
     uint32_t redo[2] = {0, 0};
-    if (any_tiny) {
-        const float least = __uint_as_float(static_cast<uint32_t>(127 + v_shift - 98) << 23);
+    bool again = false;
+    met = __builtin_amdgcn_readfirstlane(met);
+    bool some = met != 0 || far_q != 0;
+    if (some) {
+        again = (far_q | far_q >> 32) >> l32 & 1 || (met & kBadValue);
+        if (met & kFarKey) again |= admits_far_key<D>(end, kv_ld, half);
+        if (met & kTinyValue) {
+            const float least = __uint_as_float(static_cast<uint32_t>(127 + v_shift - 98) << 23);
 #pragma unroll
-        for (int vb = 0; vb < Cfg::kVB; ++vb)
+            for (int vb = 0; vb < Cfg::kVB; ++vb)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int c = vb * 32 + 8 * (r / 4) + first + r % 4;
-                if (tiny_values[c] && fabsf(o[vb][r]) < least) redo[vb / 2] |= 1u << (vb % 2 * 16 + r);
-            }
+                for (int r = 0; r < 16; ++r) {
+                    const int c = vb * 32 + 8 * (r / 4) + first + r % 4;
+                    if (tiny_values[c] && fabsf(o[vb][r]) < least) redo[vb / 2] |= 1u << (vb % 2 * 16 + r);
+                }
+        }
+        if (again) redo[0] = redo[1] = 0xFFFFFFFFu;
+        if (!end.q_live) redo[0] = redo[1] = 0;
+        some = __builtin_amdgcn_ballot_w64((redo[0] | redo[1]) != 0) != 0;
     }
-    if (again) redo[0] = redo[1] = 0xFFFFFFFFu;
-    if (!end.q_live) redo[0] = redo[1] = 0;
-    const bool some = __builtin_amdgcn_ballot_w64((redo[0] | redo[1]) != 0) != 0;
     auto store_some = [&](uint32_t flip) {
         if (!end.q_live) return;
         if (end.ml && first == 0 && again == (flip == 0)) *reinterpret_cast<float2*>(end.ml) = make_float2(m, l);
